@@ -457,8 +457,9 @@ __device__ __forceinline__ void flux_roe(const FaceState<C> &L, const FaceState<
 
 __device__ __forceinline__ double mu_of_T(const Phys &ph, double T) {
     if (ph.mu_model == FVMR_MU_CONSTANT) return ph.mu0;
-    // get_mu_using_Sutherland_air_host_device (ViscousFluxGPU.h:30-32)
-    return ph.sutherland_C1 * pow(T, 1.5) / (T + 110.4);
+    // get_mu_using_Sutherland_air_host_device (ViscousFluxGPU.h:30-32); T^1.5 as T sqrt(T): the
+    // library's pow is some 200 instructions and 60 registers in each kernel that inlines it
+    return fdiv(ph.sutherland_C1 * (T * sqrt(T)), T + 110.4);
 }
 
 // viscous_flux_device_kernel body (ViscousFluxGPU.cu:139-229); returns F_v (to be subtracted)
@@ -671,8 +672,8 @@ __device__ __forceinline__ void edge_alpha(const Phys &ph, const T ra[4], const 
     *vis = T(0);
     if (ph.equation == FVMR_EQ_NS) {
         const double value_1 = fmax(4.0 / 3.0, ph.gamma / ph.Pr);
-        const double Tt = (double)p / ph.R / (double)rho;
-        *vis = (T)(2.0 * (double)len * value_1 * mu_of_T(ph, Tt) / (double)rho / (double)vol_c);
+        const double Tt = fdiv(fdiv((double)p, ph.R), (double)rho);
+        *vis = (T)fdiv(fdiv(2.0 * (double)len * value_1 * mu_of_T(ph, Tt), (double)rho), (double)vol_c);
     }
 }
 
@@ -1612,7 +1613,7 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
             double av, vv;
             if (!(ent >> 2)) {
                 av = sAi[f];
-                vv = sAv[f] / vol_c;
+                vv = fdiv(sAv[f], vol_c);
             } else {
                 // the periodic pair of face f, seen from this cell (the face's L) and its R
                 const int4 ff = sFace[f];
