@@ -1270,6 +1270,12 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
         const int a = h->cur, b = (a + 1) % 3, c = (a + 2) % 3;
         S4 *Ua = h->Ubuf[a], *Ub = h->Ubuf[b], *Uc = h->Ubuf[c];
         const bool check = (it % kAdjCheck == 0);
+        if (h->run_steady_kernel && !check) {   // the iterations up to the next check in one launch
+            const int n = std::min(kAdjCheck - it % kAdjCheck, max_iters - it);
+            if ((rc = launch_run<double, double>(h, n, -1, true))) return rc;
+            it += n;
+            continue;
+        }
         if ((rc = local_dt(h, Ua))) return rc;
         if ((rc = steady_stage(h, Ua, Ua, Ub, 0.0, 1.0, 1, check ? h->rhs : nullptr))) return rc;
         if (h->p.time_advance == FVMR_EVO_RK3) {
@@ -1289,6 +1295,11 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
     }
     h->rhs_valid = false;
     free_graphs(h);
+    if (h->run_steady_kernel) {
+        Scalars s{};
+        if ((rc = read_scalars(h, s))) return rc;
+        if (s.run_failed) return set_error(FVMR_ERR_HIP, "resident step kernel: a work-group waited too long for its neighbours");
+    }
     if (iters) *iters = it;
     if (res) { res[0] = r0; res[1] = r; }
     return FVMR_OK;

@@ -14,6 +14,9 @@
 //                   the signed sum in slot order, /(-V), RK update.
 //   k_restrict      one work-group: flagged cells repaired from their neighbours (Jacobi).
 //
+//   k_run           the above for many steps in one launch, on meshes whose tiles all fit on the
+//                   device at once (about 150,000 cells in FP64, 230,000 mixed).
+//
 // Cell family (any geometry; packed per-cell / per-edge records, a neighbour costs 1-2 lines):
 //   k_gradient<DT>  3 wave64 x 64 cells: wave j gathers face slot j; wave 0 forms the
 //                   gradient and limiter (and, in stage 1, the dt block minimum).
@@ -135,20 +138,22 @@ struct Phys {
 // Device scalars of a handle: t, dt, T, t at the start of the step.
 struct Scalars {
     double t, dt, T, t_rk;
-    unsigned int counter;
-    unsigned int spare;
+    unsigned int run_done;      // steps of the last launch of the resident kernel
+    unsigned int run_failed;    // one of its waits gave up
     int bad_count;              // sc[0]: length of the handle's list of flagged cells
     int n_restricted;           // cells of this case restricted in the current step
 };
 
 // Blocks are dispatched round-robin over the 8 XCDs; give each XCD a contiguous
 // range of logical blocks so that neighbouring cells share an L2.
-__device__ __forceinline__ int xcd_block() {
+__device__ __forceinline__ int xcd_block(int nb) {
     if (!FVMR_XCD_REMAP) return blockIdx.x;
-    const int nb = gridDim.x, b = blockIdx.x;
+    const int b = blockIdx.x;
     const int q = nb >> 3, r = nb & 7, x = b & 7;
     return x * q + min(x, r) + (b >> 3);
 }
+
+__device__ __forceinline__ int xcd_block() { return xcd_block(gridDim.x); }
 
 template <class T> __device__ __forceinline__ T tmin(T a, T b) { return (a < b) ? a : b; }
 template <class T> __device__ __forceinline__ T tmax(T a, T b) { return (a > b) ? a : b; }
@@ -1286,6 +1291,151 @@ inline bool tile_scheme_fixed(const Phys &ph) {
            ph.reconstruct == FVMR_REC_LINEAR;
 }
 
+// LDS of a work-group that computes a tile's stages: states (16-byte columns), node coordinates,
+// centroids, face records and normals; the gradients (16-byte columns of kMaxG), which the face
+// fluxes (columns of kMaxFF) replace once every flux is formed.
+template <class C, class G, class Cfg>
+struct TileLds {
+    using SU = TileState<C>;
+    static_assert(Cfg::kMaxL <= Cfg::kThreads && Cfg::kMaxFF <= Cfg::kThreads, "one local cell and one face per thread");
+    static_assert(Cfg::kMaxN <= Cfg::kThreads && Cfg::kMaxF <= 2 * Cfg::kThreads, "one node and two faces per thread");
+    static_assert(Cfg::kMaxFF * sizeof(V4<C>) <= Cfg::kMaxG * sizeof(Grad<G>), "flux buffer overlays the gradients");
+    char U[Cfg::kMaxL * sizeof(SU)];
+    V2<double> N[Cfg::kMaxN];
+    int4 face[Cfg::kMaxF];
+    char grfl[Cfg::kMaxG * sizeof(Grad<G>)];
+    V2<G> cen[Cfg::kMaxL];
+    V2<G> nrm[Cfg::kMaxF];
+};
+
+// Limited gradient of local cell i (tile or first ring) into LDS.  gs: its slot words, gco: its
+// Green-Gauss weights and volume, nw: its nodes.
+template <class C, class G, class Cfg>
+__device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg> &s, int i, const int4 gs,
+                                              const V4<G> gco, int nw) {
+    using SU = TileState<C>;
+    const int sw[3] = {gs.x, gs.y, gs.z};
+    const C vol = (C)gco.w;
+    C Uc[4];
+    {
+        const SU v = lds_get<SU>(s.U, Cfg::kMaxL, i);
+        Uc[0] = (C)v.x; Uc[1] = (C)v.y; Uc[2] = (C)v.z; Uc[3] = (C)v.w;
+    }
+    const C xc = (C)s.cen[i].x, yc = (C)s.cen[i].y;
+    struct {
+        C a[3][3], u[3][4], n[3][2];
+        __device__ __forceinline__ C A(int j, int q) const { return a[j][q]; }
+        __device__ __forceinline__ C Uo(int j, int k) const { return u[j][k]; }
+        __device__ __forceinline__ C N(int j, int q) const { return n[j][q]; }
+    } sl;
+    int fl[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int f = sw[j] & fvmr::kLocalMask;
+        const int out = (sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask;
+        const bool has_out = out != fvmr::kLocalNone;
+        const bool periodic = (sw[j] & fvmr::kGsPeriodic) != 0;
+        const C sgn = (sw[j] & fvmr::kGsIsR) ? C(-1) : C(1);
+        const int4 fr = s.face[f];
+        V4<G> eg;
+        V2<G> em;
+        tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
+        {
+            const SU v = lds_get<SU>(s.U, Cfg::kMaxL, has_out ? out : i);
+            sl.u[j][0] = (C)v.x; sl.u[j][1] = (C)v.y; sl.u[j][2] = (C)v.z; sl.u[j][3] = (C)v.w;
+        }
+        const V2<double> nd = s.N[lfield(nw, j)];
+        sl.n[j][0] = (C)(G)nd.x - xc;
+        sl.n[j][1] = (C)(G)nd.y - yc;
+        if (ph.gradient == FVMR_GRA_GREENGAUSS) {
+            // weight g_C of the slot precomputed by the host (the device formula in FP64)
+            const C len = (C)eg.z;
+            sl.a[j][0] = (C)(j == 0 ? gco.x : (j == 1 ? gco.y : gco.z));
+            sl.a[j][1] = (C)eg.x * len * sgn;
+            sl.a[j][2] = (C)eg.y * len * sgn;
+        } else {
+            C dxn = C(0), dyn = C(0);
+            if (has_out && !periodic) {   // element neighbours exclude periodic faces
+                dxn = (C)s.cen[out].x - xc;
+                dyn = (C)s.cen[out].y - yc;
+            }
+            sl.a[j][0] = dxn;
+            sl.a[j][1] = dyn;
+            sl.a[j][2] = C(0);
+        }
+        fl[j] = (has_out ? 1 : 0) | ((has_out && !periodic) ? 2 : 0);
+    }
+    C gx[4], gy[4];
+    grad_limit<C>(ph, Uc, sl, fl, vol, gx, gy);
+    Grad<G> g;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        g.x[k] = (G)gx[k];
+        g.y[k] = (G)gy[k];
+    }
+    lds_put(s.grfl, Cfg::kMaxG, i, g);
+}
+
+// The canonical L -> R flux of face f of the tile from the states and gradients in LDS.
+template <class C, class G, bool NS, class Cfg>
+__device__ __forceinline__ void tile_flux(const Phys &ph, const CaseBC &bc, double t_rk, const TileLds<C, G, Cfg> &s,
+                                          int f, C F[4]) {
+    const TileCells<G, TileState<C>> cells{s.U, Cfg::kMaxL, s.cen, s.grfl, Cfg::kMaxG};
+    const int4 fr = s.face[f];
+    V4<G> eg;
+    V2<G> em;
+    tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
+    const int L = lfield(fr.y, 0), R = lfield(fr.y, 1), pl = lfield(fr.y, 2);
+    const int bType = tile_btype(fr);
+    const bool has_pair = pl != fvmr::kLocalNone;
+    const V2<G> pm = (bType != -1 && has_pair) ? tile_face_mid<G>(s.N, s.face[pl]) : em;
+    face_flux<C, G, NS>(cells, ph, bc, t_rk, L, R == fvmr::kLocalNone ? -1 : R, bType, has_pair, eg, em, pm, F);
+}
+
+// r = -(1/V) sum_j s_j F_j of a tile cell, the fluxes of its faces taken from LDS in slot order.
+template <class C, class G, class Cfg>
+__device__ __forceinline__ void tile_rhs(const TileLds<C, G, Cfg> &s, const int4 gs, const V4<G> gco, double r[4]) {
+    const int sw[3] = {gs.x, gs.y, gs.z};
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const V4<C> fv = lds_get<V4<C>>(s.grfl, Cfg::kMaxFF, sw[j] & fvmr::kLocalMask);
+        const double sg = (sw[j] & fvmr::kGsIsR) ? -1.0 : 1.0;
+        acc[0] += sg * (double)fv.x;
+        acc[1] += sg * (double)fv.y;
+        acc[2] += sg * (double)fv.z;
+        acc[3] += sg * (double)fv.w;
+    }
+    const double w = -1.0 * (double)gco.w;
+#pragma unroll
+    for (int k = 0; k < 4; k++) r[k] = fdiv(acc[k], w);
+}
+
+// The new state of one variable: s = Ui + dt r in the first stage, a Ub + b s in the others, with the
+// same roundings in every kernel.
+__device__ __forceinline__ double rk_update(double Ui, double Ub, double r, double dt, double a, double b, bool first) {
+    const double s = fma(dt, r, Ui);
+    return first ? s : fma(a, Ub, b * s);
+}
+
+// Whether a cell's new state is to be restricted: NaN, or rho or p out of range.
+__device__ __forceinline__ bool state_is_bad(const double U[4], double gamma) {
+    double rv[4];
+    prim(U, rv, gamma);
+    bool bad = out_of_range(rv[0], rv[3]);
+#pragma unroll
+    for (int k = 0; k < 4; k++) bad = bad || isnan(rv[k]);
+    return bad;
+}
+// Appends device cell c of case cs to the handle's list of cells to restrict (sc[0] holds its length).
+__device__ __forceinline__ void flag_bad(Scalars *sc, int *bad_list, int nc, int c, int cs) {
+    const int slot = atomicAdd(&sc->bad_count, 1);
+    if (slot < nc) {
+        bad_list[slot] = c;
+        bad_list[nc + slot] = cs;
+    }
+}
+
 // One RK stage over the tiles (the work of k_gradient + k_stage, see there).
 template <class C, class G, bool NS, bool LDT = false, int SCHEME = kTileAny, int SHAPE = 0>
 __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs<G> ta, Phys ph, const S4 *__restrict__ Uin,
@@ -1300,19 +1450,9 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
         ph.reconstruct = FVMR_REC_LINEAR;
     }
     using Cfg = TileCfg<C, SHAPE>;
-    constexpr int kTileThreads = Cfg::kThreads, kTileMaxG = Cfg::kMaxG, kTileMaxL = Cfg::kMaxL;
-    constexpr int kTileMaxN = Cfg::kMaxN, kTileMaxF = Cfg::kMaxF, kTileMaxFF = Cfg::kMaxFF;
-    static_assert(kTileMaxL <= kTileThreads && kTileMaxFF <= kTileThreads, "one local cell and one face per thread");
+    constexpr int kTileThreads = Cfg::kThreads;
     using SU = TileState<C>;
-    __shared__ __align__(16) char sU[kTileMaxL * sizeof(SU)];   // states, 16-byte columns of kTileMaxL
-    __shared__ V2<double> sN[kTileMaxN];
-    __shared__ V2<G> sC[kTileMaxL];
-    __shared__ int4 sFace[kTileMaxF];
-    __shared__ V2<G> sNrm[kTileMaxF];   // face normals
-    // the face fluxes (16-byte columns of kTileMaxFF) replace the gradients (columns of
-    // kTileMaxG) once every flux is formed
-    static_assert(kTileMaxFF * sizeof(V4<C>) <= kTileMaxG * sizeof(Grad<G>), "flux buffer overlays the gradients");
-    __shared__ __align__(16) char sGrFl[kTileMaxG * sizeof(Grad<G>)];
+    __shared__ __align__(16) TileLds<C, G, Cfg> lds;
     const int tid = threadIdx.x;
     const int *ti = ta.info + (size_t)xcd_block() * fvmr::kTileInfo;
     const int c0 = ti[fvmr::kTiC0], nT = ti[fvmr::kTiNT], nG = ti[fvmr::kTiNG], nL = ti[fvmr::kTiNL];
@@ -1326,10 +1466,8 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     const int nw = (i < nL) ? ta.lnodes[offL + i] : 0;
     const int4 gs = (i < nG) ? ta.gslot[offG + i] : make_int4(0, 0, 0, 0);
     const V4<G> gco = (i < nG) ? ta.gcoef[offG + i] : V4<G>{G(0.5), G(0.5), G(0.5), G(1)};
-    const G gvol = gco.w;
     // 1. stage nodes, states and face records: every global load is issued before the first
     // LDS store (a store between loads would make each wave wait for the loads before it)
-    static_assert(kTileMaxN <= kTileThreads && kTileMaxF <= 2 * kTileThreads, "one node and two faces per thread");
     const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : -1;
     const S4 uin = (src >= 0) ? Uin[src] : S4{0.0, 0.0, 0.0, 0.0};
     const V2<double> nd = (tid < nN) ? ta.nxy[offN + tid] : V2<double>{0.0, 0.0};
@@ -1341,165 +1479,141 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     const V2<G> nr0 = (tid < nF) ? ta.fnrm[offF + tid] : V2<G>{G(0), G(0)};
     const V2<G> nr1 = (tid + kTileThreads < nF) ? ta.fnrm[offF + tid + kTileThreads] : V2<G>{G(0), G(0)};
 #endif
-    if (tid < nN) sN[tid] = nd;
-    if (tid < nF) sFace[tid] = fr0;
-    if (tid + kTileThreads < nF) sFace[tid + kTileThreads] = fr1;
-    if (i < nL) lds_put(sU, kTileMaxL, i, SU{(C)uin.x, (C)uin.y, (C)uin.z, (C)uin.w});
+    if (tid < nN) lds.N[tid] = nd;
+    if (tid < nF) lds.face[tid] = fr0;
+    if (tid + kTileThreads < nF) lds.face[tid + kTileThreads] = fr1;
+    if (i < nL) lds_put(lds.U, Cfg::kMaxL, i, SU{(C)uin.x, (C)uin.y, (C)uin.z, (C)uin.w});
 #if FVMR_TILE_GEOM_LOADED
-    if (i < nL) sC[i] = cc;
-    if (tid < nF) sNrm[tid] = nr0;
-    if (tid + kTileThreads < nF) sNrm[tid + kTileThreads] = nr1;
+    if (i < nL) lds.cen[i] = cc;
+    if (tid < nF) lds.nrm[tid] = nr0;
+    if (tid + kTileThreads < nF) lds.nrm[tid + kTileThreads] = nr1;
     __syncthreads();
 #else
     __syncthreads();
     // 2. centroids and face normals
     if (i < nL) {
-        const V2<double> ct = tile_centroid(sN, nw);
-        sC[i] = V2<G>{(G)ct.x, (G)ct.y};
+        const V2<double> ct = tile_centroid(lds.N, nw);
+        lds.cen[i] = V2<G>{(G)ct.x, (G)ct.y};
     }
     for (int k = tid; k < nF; k += kTileThreads) {
         V4<G> eg;
         V2<G> em;
-        tile_face_geom<G>(sN, sFace[k], eg, em);
-        sNrm[k] = V2<G>{eg.x, eg.y};
+        tile_face_geom<G>(lds.N, lds.face[k], eg, em);
+        lds.nrm[k] = V2<G>{eg.x, eg.y};
     }
     __syncthreads();
 #endif
     // 3. limited gradients of the tile and the first ring
-    if (i < nG) {
-        const int sw[3] = {gs.x, gs.y, gs.z};
-        const C vol = (C)gvol;
-        C Uc[4];
-        {
-            const SU v = lds_get<SU>(sU, kTileMaxL, i);
-            Uc[0] = (C)v.x; Uc[1] = (C)v.y; Uc[2] = (C)v.z; Uc[3] = (C)v.w;
-        }
-        const C xc = (C)sC[i].x, yc = (C)sC[i].y;
-        struct {
-            C a[3][3], u[3][4], n[3][2];
-            __device__ __forceinline__ C A(int j, int q) const { return a[j][q]; }
-            __device__ __forceinline__ C Uo(int j, int k) const { return u[j][k]; }
-            __device__ __forceinline__ C N(int j, int q) const { return n[j][q]; }
-        } sl;
-        int fl[3];
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const int f = sw[j] & fvmr::kLocalMask;
-            const int out = (sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask;
-            const bool has_out = out != fvmr::kLocalNone;
-            const bool periodic = (sw[j] & fvmr::kGsPeriodic) != 0;
-            const C sgn = (sw[j] & fvmr::kGsIsR) ? C(-1) : C(1);
-            const int4 fr = sFace[f];
-            V4<G> eg;
-            V2<G> em;
-            tile_face_geom_n<G>(sN, sNrm, f, fr, eg, em);
-            {
-                const SU v = lds_get<SU>(sU, kTileMaxL, has_out ? out : i);
-                sl.u[j][0] = (C)v.x; sl.u[j][1] = (C)v.y; sl.u[j][2] = (C)v.z; sl.u[j][3] = (C)v.w;
-            }
-            const V2<double> nd = sN[lfield(nw, j)];
-            sl.n[j][0] = (C)(G)nd.x - xc;
-            sl.n[j][1] = (C)(G)nd.y - yc;
-            if (ph.gradient == FVMR_GRA_GREENGAUSS) {
-                // weight g_C of the slot precomputed by the host (the device formula in FP64)
-                const C len = (C)eg.z;
-                sl.a[j][0] = (C)(j == 0 ? gco.x : (j == 1 ? gco.y : gco.z));
-                sl.a[j][1] = (C)eg.x * len * sgn;
-                sl.a[j][2] = (C)eg.y * len * sgn;
-            } else {
-                C dxn = C(0), dyn = C(0);
-                if (has_out && !periodic) {   // element neighbours exclude periodic faces
-                    dxn = (C)sC[out].x - xc;
-                    dyn = (C)sC[out].y - yc;
-                }
-                sl.a[j][0] = dxn;
-                sl.a[j][1] = dyn;
-                sl.a[j][2] = C(0);
-            }
-            fl[j] = (has_out ? 1 : 0) | ((has_out && !periodic) ? 2 : 0);
-        }
-        C gx[4], gy[4];
-        grad_limit<C>(ph, Uc, sl, fl, vol, gx, gy);
-        Grad<G> g;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            g.x[k] = (G)gx[k];
-            g.y[k] = (G)gy[k];
-        }
-        lds_put(sGrFl, kTileMaxG, i, g);
-    }
+    if (i < nG) tile_gradient(ph, lds, i, gs, gco, nw);
     __syncthreads();
     // 4. one canonical flux per face of the tile (nFF <= threads), written over the gradients
     const double t_rk = sc[cs].t_rk;
     const CaseBC &bc = ta.cbc[cs];
-    const TileCells<G, SU> cells{sU, kTileMaxL, sC, sGrFl, kTileMaxG};
     C F[4] = {C(0), C(0), C(0), C(0)};
     const int f = tid;
-    if (f < nFF) {
-        const int4 fr = sFace[f];
-        V4<G> eg;
-        V2<G> em;
-        tile_face_geom_n<G>(sN, sNrm, f, fr, eg, em);
-        const int L = lfield(fr.y, 0), R = lfield(fr.y, 1), pl = lfield(fr.y, 2);
-        const int bType = tile_btype(fr);
-        const bool has_pair = pl != fvmr::kLocalNone;
-        const V2<G> pm = (bType != -1 && has_pair) ? tile_face_mid<G>(sN, sFace[pl]) : em;
-        face_flux<C, G, NS>(cells, ph, bc, t_rk, L, R == fvmr::kLocalNone ? -1 : R, bType, has_pair, eg, em, pm, F);
-    }
+    if (f < nFF) tile_flux<C, G, NS>(ph, bc, t_rk, lds, f, F);
     __syncthreads();
-    if (f < nFF) lds_put(sGrFl, kTileMaxFF, f, V4<C>{F[0], F[1], F[2], F[3]});
+    if (f < nFF) lds_put(lds.grfl, Cfg::kMaxFF, f, V4<C>{F[0], F[1], F[2], F[3]});
     __syncthreads();
     // 5. cell-owned sum in slot order, /(-V), RK update (as k_stage); LDT: the cell's own dt
     double dt = sc[cs].dt;
     if (i < nT) {
         const int c = c0 + i;
         if (LDT) dt = ta.dtl[c];
-        const int sw[3] = {gs.x, gs.y, gs.z};
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const V4<C> fv = lds_get<V4<C>>(sGrFl, kTileMaxFF, sw[j] & fvmr::kLocalMask);
-            const double s = (sw[j] & fvmr::kGsIsR) ? -1.0 : 1.0;
-            acc[0] += s * (double)fv.x;
-            acc[1] += s * (double)fv.y;
-            acc[2] += s * (double)fv.z;
-            acc[3] += s * (double)fv.w;
-        }
-        const double w = -1.0 * (double)gvol;
         // the cell's own FP64 state: from LDS in the plain path, from this thread's staging
         // registers in mixed precision (its LDS copy is FP32)
         double Ui[4];
         if (std::is_same<SU, S4>::value) {
-            const SU v = lds_get<SU>(sU, kTileMaxL, i);
+            const SU v = lds_get<SU>(lds.U, Cfg::kMaxL, i);
             Ui[0] = v.x; Ui[1] = v.y; Ui[2] = v.z; Ui[3] = v.w;
         } else {
             Ui[0] = uin.x; Ui[1] = uin.y; Ui[2] = uin.z; Ui[3] = uin.w;
         }
         double Ub[4] = {0, 0, 0, 0}, r[4], Unew[4];
         if (!first) { Ub[0] = un.x; Ub[1] = un.y; Ub[2] = un.z; Ub[3] = un.w; }
+        tile_rhs(lds, gs, gco, r);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            r[k] = fdiv(acc[k], w);
-            const double s = Ui[k] + dt * r[k];
-            Unew[k] = first ? s : a * Ub[k] + b * s;
-        }
+        for (int k = 0; k < 4; k++) Unew[k] = rk_update(Ui[k], Ub[k], r[k], dt, a, b, first != 0);
         if (rhs_out) st(rhs_out, c, r);
         if (std::is_same<C, double>::value) st_stream(Uout, c, Unew);
         else st(Uout, c, Unew);
         if (!last) return;
-        double rv[4];
-        prim(Unew, rv, ph.gamma);
-        bool bad = out_of_range(rv[0], rv[3]);
-#pragma unroll
-        for (int k = 0; k < 4; k++) bad = bad || isnan(rv[k]);
-        if (bad) {
-            const int slot = atomicAdd(&sc->bad_count, 1);   // the handle's list: sc[0]
-            if (slot < nc) {
-                bad_list[slot] = c;
-                bad_list[nc + slot] = cs;
-            }
-        }
+        if (state_is_bad(Unew, ph.gamma)) flag_bad(sc, bad_list, nc, c, cs);
     }
+}
+
+// Spectral radius of one face of a tile from the states of its two cells (uR = uL without an R):
+// the inviscid part, and the viscous part up to the division by the cell volume.  LDT: the
+// consistent radius (|u.n| + a) L of the pseudo-time steps.
+template <class G, bool LDT>
+__device__ __forceinline__ void face_alpha(const Phys &ph, const double uL[4], const double uR[4], bool has_R,
+                                           const V4<G> eg, double *av, double *vv) {
+    if (!LDT && !std::is_same<G, double>::value) {
+        // mixed precision: the face's primitives and spectral radius in FP32 (the per-cell
+        // sums and the minimum in FP64)
+        G ua[4], ub[4], ra[4], rb[4], a32, v32;
+#pragma unroll
+        for (int k = 0; k < 4; k++) { ua[k] = (G)uL[k]; ub[k] = (G)uR[k]; }
+        prim(ua, ra, (G)ph.gamma);
+        prim(ub, rb, (G)ph.gamma);
+        edge_alpha<G>(ph, ra, rb, has_R, eg.x, eg.y, eg.z, G(1), &a32, &v32);
+        *av = (double)a32;
+        *vv = (double)v32;
+        return;
+    }
+    double rL[4], rR[4];
+    prim(uL, rL, ph.gamma);
+    prim(uR, rR, ph.gamma);
+    if (LDT) {
+        double r[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) r[k] = has_R ? 0.5 * (rL[k] + rR[k]) : rL[k];
+        const double Lf = (double)eg.z;
+        *av = (fabs(r[1] * (double)eg.x + r[2] * (double)eg.y) + sqrt(ph.gamma * r[3] / r[0])) * Lf;
+        *vv = 0.0;
+        if (ph.equation == FVMR_EQ_NS) {
+            const double T = r[3] / ph.R / r[0];
+            *vv = fmax(4.0 / 3.0, ph.gamma / ph.Pr) * mu_of_T(ph, T) / r[0] * Lf * Lf;
+        }
+    } else {
+        edge_alpha<double>(ph, rL, rR, has_R, (double)eg.x, (double)eg.y, (double)eg.z, 1.0, av, vv);
+    }
+}
+
+// alphaC of a tile cell: its faces' radii (local faces f0, f1, f2 of its slots) in the reference
+// edge order; code: count (3 bits) + 6 x (slot 2 bits, pair 1 bit); pair(f, av, vv): the radius of the
+// periodic pair of face f (inviscid, and viscous divided by the volume).
+template <class Pair>
+__device__ __forceinline__ double cell_alpha(const Phys &ph, int code, int f0, int f1, int f2, const double *sAi,
+                                             const double *sAv, double vol_c, Pair &&pair) {
+    const int cnt = code & 7;
+    double alpha_c = 0.0;
+    for (int q = 0; q < cnt; q++) {
+        const int ent = (code >> (3 + 3 * q)) & 7;
+        const int f = (ent & 3) == 0 ? f0 : ((ent & 3) == 1 ? f1 : f2);
+        double av, vv;
+        if (!(ent >> 2)) {
+            av = sAi[f];
+            vv = fdiv(sAv[f], vol_c);
+        } else {
+            pair(f, &av, &vv);
+        }
+        alpha_c += av;
+        if (ph.equation == FVMR_EQ_NS) alpha_c += vv;
+    }
+    return alpha_c;
+}
+// The same for a pseudo-time step: the three slots in order (k_local_dt's).
+__device__ __forceinline__ double local_alpha(const Phys &ph, int f0, int f1, int f2, const double *sAi,
+                                              const double *sAv, double vol_c) {
+    const int f[3] = {f0, f1, f2};
+    double alpha_c = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        alpha_c += sAi[f[j]];
+        if (ph.equation == FVMR_EQ_NS) alpha_c += sAv[f[j]] / vol_c;
+    }
+    return alpha_c;
 }
 
 // Block minima of CFL V / alphaC over the tiles (the dt part of k_gradient<DT>): the
@@ -1542,98 +1656,42 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
     // faces of the tile cells (one per thread): L and R (when present) are tile or first-ring cells
     static_assert(kTileMaxFF <= kTileThreads, "one face per thread");
     if (tid < nFF) {
-        const int f = tid;
         const int L = lfield(fr.y, 0), R = lfield(fr.y, 1);
         V4<G> eg;
         V2<G> em;
         tile_face_geom<G>(sN, fr, eg, em);
-        double uL[4], rL[4], uR[4], rR[4];
+        double uL[4], uR[4];
         lds_state(sU, kTileMaxG, L, uL);
         const bool has_R = R != fvmr::kLocalNone;
         lds_state(sU, kTileMaxG, has_R ? R : L, uR);
-        double av, vv;
-        if (!LDT && !std::is_same<G, double>::value) {
-            // mixed precision: the face's primitives and spectral radius in FP32 (the per-cell
-            // sums and the minimum in FP64)
-            G ua[4], ub[4], ra[4], rb[4], a32, v32;
-#pragma unroll
-            for (int k = 0; k < 4; k++) { ua[k] = (G)uL[k]; ub[k] = (G)uR[k]; }
-            prim(ua, ra, (G)ph.gamma);
-            prim(ub, rb, (G)ph.gamma);
-            edge_alpha<G>(ph, ra, rb, has_R, eg.x, eg.y, eg.z, G(1), &a32, &v32);
-            av = (double)a32;
-            vv = (double)v32;
-        } else if (LDT) {
-            prim(uL, rL, ph.gamma);
-            prim(uR, rR, ph.gamma);
-            double r[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) r[k] = has_R ? 0.5 * (rL[k] + rR[k]) : rL[k];
-            const double Lf = (double)eg.z;
-            av = (fabs(r[1] * (double)eg.x + r[2] * (double)eg.y) + sqrt(ph.gamma * r[3] / r[0])) * Lf;
-            vv = 0.0;
-            if (ph.equation == FVMR_EQ_NS) {
-                const double T = r[3] / ph.R / r[0];
-                vv = fmax(4.0 / 3.0, ph.gamma / ph.Pr) * mu_of_T(ph, T) / r[0] * Lf * Lf;
-            }
-        } else {
-            prim(uL, rL, ph.gamma);
-            prim(uR, rR, ph.gamma);
-            edge_alpha<double>(ph, rL, rR, has_R, (double)eg.x, (double)eg.y, (double)eg.z, 1.0, &av, &vv);
-        }
-        sAi[f] = av;
-        sAv[f] = vv;
+        face_alpha<G, LDT>(ph, uL, uR, has_R, eg, &sAi[tid], &sAv[tid]);
     }
     __syncthreads();
     if (LDT) {
-        if (tid < nT) {
-            const double vol_c = dr.vol;
-            double alpha_c = 0.0;
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const int f = lfield(dr.faces, j);
-                alpha_c += sAi[f];
-                if (ph.equation == FVMR_EQ_NS) alpha_c += sAv[f] / vol_c;
-            }
-            ta.dtl[c0 + tid] = ta.cbc[ti[fvmr::kTiCase]].CFL * vol_c / alpha_c;
-        }
+        if (tid < nT)
+            ta.dtl[c0 + tid] = ta.cbc[ti[fvmr::kTiCase]].CFL * dr.vol /
+                               local_alpha(ph, lfield(dr.faces, 0), lfield(dr.faces, 1), lfield(dr.faces, 2), sAi, sAv, dr.vol);
         return;
     }
     double dtc = 1e10;
     if (tid < nT) {
-        const int i = tid;
-        const int code = dr.code;
-        const double vol_c = dr.vol;
-        // alphaC in the reference edge order: count (3 bits) + 6 x (slot 2 bits, pair 1 bit)
-        const int cnt = code & 7;
-        double alpha_c = 0.0;
-        for (int q = 0; q < cnt; q++) {
-            const int ent = (code >> (3 + 3 * q)) & 7;
-            const int f = lfield(dr.faces, ent & 3);
-            double av, vv;
-            if (!(ent >> 2)) {
-                av = sAi[f];
-                vv = fdiv(sAv[f], vol_c);
-            } else {
+        const double alpha_c = cell_alpha(ph, dr.code, lfield(dr.faces, 0), lfield(dr.faces, 1), lfield(dr.faces, 2), sAi, sAv, dr.vol,
+            [&](int f, double *av, double *vv) {
                 // the periodic pair of face f, seen from this cell (the face's L) and its R
                 const int4 ff = sFace[f];
                 const int out = lfield(ff.y, 1);
-                const int pf = lfield(ff.y, 2);
-                const int4 fr = ta.face[offF + pf];
+                const int4 pr = ta.face[offF + lfield(ff.y, 2)];
                 V4<G> eg;
                 V2<G> em;
-                tile_face_geom<G>(sN, fr, eg, em);
+                tile_face_geom<G>(sN, pr, eg, em);
                 double Uc[4], rc[4], Uo[4], ro[4];
-                lds_state(sU, kTileMaxG, i, Uc);
+                lds_state(sU, kTileMaxG, tid, Uc);
                 prim(Uc, rc, ph.gamma);
                 lds_state(sU, kTileMaxG, out, Uo);
                 prim(Uo, ro, ph.gamma);
-                edge_alpha(ph, rc, ro, true, (double)eg.x, (double)eg.y, (double)eg.z, vol_c, &av, &vv);
-            }
-            alpha_c += av;
-            if (ph.equation == FVMR_EQ_NS) alpha_c += vv;
-        }
-        dtc = fmin(dtc, fdiv(ta.cbc[ti[fvmr::kTiCase]].CFL * vol_c, alpha_c));
+                edge_alpha(ph, rc, ro, true, (double)eg.x, (double)eg.y, (double)eg.z, dr.vol, av, vv);
+            });
+        dtc = fmin(dtc, fdiv(ta.cbc[ti[fvmr::kTiCase]].CFL * dr.vol, alpha_c));
     }
     const double wm = wave_min(dtc);
     if ((tid & 63) == 0) sMin[tid >> 6] = wm;
@@ -1642,6 +1700,367 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
         double m = sMin[0];
         for (int w = 1; w < kTileThreads / 64; w++) m = fmin(m, sMin[w]);
         partial[blk] = m;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Resident kernel: many steps in one launch, for meshes whose tiles all fit on the chip at once.
+//
+// A step of a small mesh is bound by the latency of its dependent launches (4 to 6 of them, 4-6 us
+// each, whatever they do).  Measured per step, launched and resident, on one box: 8,192 cells SSP-RK3 27 and
+// 11.6 us, 34,182 cells viscous forward Euler 17.6 and 9.5 us, 131,070 cells viscous mixed SSP-RK3 43 and 28 us;
+// 50 pseudo-time iterations of 40,000 cells 1.72 and 1.38 ms.  What bounds a resident stage of the 8,192
+// cells (3.9 us): the latency chains of the gradients (1.5 us) and fluxes (0.9 us) at one wave per SIMD,
+// and the exchange, a store to and a load from memory (1.6 us).  Here every tile's work-group stays on its CU for all steps: geometry,
+// slots and states stay in LDS and registers, the new states of the cells that other tiles need
+// are exchanged through global memory after each stage, and the time step's minimum goes through
+// one more work-group, which only reduces.  The launch is cooperative, so all work-groups run at
+// once or the launch fails; every wait ends after kRunSpin polls at the latest.
+//
+// Exchange.  A double travels as two 64-bit words, each half of its bits with the number of the
+// exchange in the upper 32 bits.  Words are written and read by relaxed device-scope atomics, so
+// each is valid by itself and no ordering between words (fence, flag, cache write-back) is needed:
+// a reader polls the words that it needs until they carry the number that it waits for.  Two
+// buffers in turn are enough: a tile writes exchange e + 1 only after it has read exchange e of
+// every tile around it, and those wrote e after they had read e - 1 (tiles need each other's cells
+// mutually; the host checks that).  The partial minima and the published minimum have one buffer
+// each: a tile posts the next minimum only after it has read the last published one.
+// ---------------------------------------------------------------------------
+constexpr int kRunSpin = 1 << 21;     // polls before a wait gives up (about 1 us each)
+constexpr int kRunCopies = 32;        // copies of the published time step, kRunStride words apart
+constexpr int kRunStride = 16;
+struct RunArgs {
+    unsigned long long *ll;     // exchanged states: [2][8][nc] words
+    unsigned long long *part;   // per tile: minimum (2 words), restriction flag (1 word), [3][ntiles]
+    unsigned long long *pub;    // kRunCopies x {minimum (2 words), stop flag}
+    const unsigned char *need;  // per device cell: another tile reads it
+    unsigned ex0, dt0;          // numbers of the last exchange and time step before this launch
+    int nsteps, stages, ntiles;
+    int rhs_step;               // the step whose first-stage rhs is kept (-1: none)
+    double a[3], b[3];          // stage s > 0: Uout = a Un + b (Uin + dt rhs)
+};
+
+// The kernel's one argument.  It is read again from the kernel-argument segment (scalar loads) in
+// every stage, through a pointer that the compiler cannot see through: otherwise it keeps all that
+// depends on the parameters alone in vector registers for the whole loop (188 of them, against 106
+// in k_tile).
+template <class G>
+struct RunKernArg {
+    TileArgs<G> ta;
+    Phys ph;
+    const S4 *Uin;
+    S4 *Uout, *rhs_out;
+    Scalars *sc;
+    int *bad_list;
+    int nc;
+    RunArgs ra;
+};
+#define FVMR_AS4 __attribute__((address_space(4)))
+template <class G>
+__device__ __forceinline__ const RunKernArg<G> &run_args() {
+    FVMR_AS4 void *q = (FVMR_AS4 void *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(q));
+    return *(const RunKernArg<G> *)q;
+}
+// Makes a register value opaque: nothing derived from it is kept from one stage to the next.
+__device__ __forceinline__ void opaque(int &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void opaque(float &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void opaque(double &x) { asm volatile("" : "+v"(x)); }
+
+template <int SCHEME, bool NS>
+__device__ __forceinline__ void fix_scheme(Phys &ph) {
+    if (!NS) ph.equation = FVMR_EQ_EULER;
+    if (SCHEME == kTileGgBarthRoe) {
+        ph.gradient = FVMR_GRA_GREENGAUSS;
+        ph.limiter = FVMR_LIM_BARTH;
+        ph.scheme = FVMR_SOL_ROE;
+        ph.reconstruct = FVMR_REC_LINEAR;
+    }
+}
+
+__device__ __forceinline__ unsigned long long ll_load(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void ll_store(unsigned long long *p, unsigned tag, unsigned bits) {
+    __hip_atomic_store(p, ((unsigned long long)tag << 32) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool ll_is(unsigned long long w, unsigned tag) { return (unsigned)(w >> 32) == tag; }
+__device__ __forceinline__ double ll_double(unsigned long long lo, unsigned long long hi) {
+    return __hiloint2double((int)(unsigned)hi, (int)(unsigned)lo);
+}
+__device__ __forceinline__ void ll_put_double(unsigned long long *lo, unsigned long long *hi, unsigned tag, double v) {
+    ll_store(lo, tag, (unsigned)__double2loint(v));
+    ll_store(hi, tag, (unsigned)__double2hiint(v));
+}
+
+// The reducing work-group: per step the minimum of the tiles' partial minima, published with
+// whether any tile has a cell to restrict (then the tiles stop before they change their states).
+template <int THREADS>
+__device__ __forceinline__ void run_reduce(const RunArgs &ra) {
+    __shared__ double sMin[THREADS / 64];
+    __shared__ int sFlag[THREADS / 64];
+    const int tid = threadIdx.x, n = ra.ntiles;
+    for (int s = 0; s < ra.nsteps; s++) {
+        const unsigned tag = ra.dt0 + 1 + (unsigned)s;
+        double d = 1e10;
+        int stop = 0;
+        for (int k = tid; k < n; k += THREADS) {
+            unsigned long long lo, hi, fl;
+            int spin = 0;
+            do {
+                lo = ll_load(ra.part + k);
+                hi = ll_load(ra.part + n + k);
+                fl = ll_load(ra.part + 2 * n + k);
+            } while (!(ll_is(lo, tag) && ll_is(hi, tag) && ll_is(fl, tag)) && ++spin < kRunSpin);
+            if (spin >= kRunSpin) stop = 2;
+            else {
+                d = fmin(d, ll_double(lo, hi));
+                stop |= (int)(fl & 3u);
+            }
+        }
+        d = wave_min(d);
+        stop = __any(stop & 2) ? 2 : (__any(stop & 1) ? 1 : 0);
+        if ((tid & 63) == 0) {
+            sMin[tid >> 6] = d;
+            sFlag[tid >> 6] = stop;
+        }
+        __syncthreads();
+        stop = 0;
+        d = sMin[0];
+        for (int w = 0; w < THREADS / 64; w++) {
+            d = fmin(d, sMin[w]);
+            stop = max(stop, sFlag[w]);
+        }
+        if (tid < kRunCopies) {
+            unsigned long long *q = ra.pub + tid * kRunStride;
+            ll_put_double(q, q + 1, tag, d);
+            ll_store(q + 2, tag, (unsigned)stop);
+        }
+        if (stop) return;
+        __syncthreads();   // sMin and sFlag are read before the next step writes them
+    }
+}
+
+// ra.nsteps steps (k_tile_dt, k_dt_finish, k_tile per stage) of every tile; stops before a step when
+// the last one left cells to restrict (bad_list, as k_tile).  LDT: pseudo-time iterations with
+// per-cell steps and no restriction (no reducing work-group).  The arithmetic is that of k_tile_dt
+// and k_tile.
+template <class C, class G, bool NS, bool LDT, int SCHEME, int WAVES>
+__global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKernArg<G> arg) {
+    using Cfg = TileCfg<C, 0>;
+    using SU = TileState<C>;
+    constexpr bool kF64 = std::is_same<SU, S4>::value;
+    if (!LDT && (int)blockIdx.x == arg.ra.ntiles) {
+        run_reduce<Cfg::kThreads>(arg.ra);
+        return;
+    }
+    const TileArgs<G> &ta = arg.ta;
+    const RunArgs &ra = arg.ra;
+    Scalars *const sc = arg.sc;
+    const int nc = arg.nc;
+    __shared__ __align__(16) TileLds<C, G, Cfg> lds;
+    __shared__ double sMin[Cfg::kThreads / 64];
+    __shared__ double sT, sTrk, sDt;   // t, t at the start of the step, dt
+    __shared__ int sStop, sFail, sBad;   // the published flag; a wait of this work-group gave up; a cell to restrict
+    // the faces' spectral radii, before the gradients take their place
+    static_assert(2 * Cfg::kMaxFF * sizeof(double) <= sizeof(lds.grfl), "radii overlay the gradients");
+    double *const sAi = reinterpret_cast<double *>(lds.grfl), *const sAv = sAi + Cfg::kMaxFF;
+    const int tid = threadIdx.x, i = tid;
+    const int tile = xcd_block(ra.ntiles);
+    const int *ti = ta.info + (size_t)tile * fvmr::kTileInfo;
+    const int c0 = ti[fvmr::kTiC0], nT = ti[fvmr::kTiNT], nG = ti[fvmr::kTiNG], nL = ti[fvmr::kTiNL];
+    const int nN = ti[fvmr::kTiNN], nF = ti[fvmr::kTiNF], nFF = ti[fvmr::kTiNFF];
+    const int offH = ti[fvmr::kTiOffH], offN = ti[fvmr::kTiOffN], offF = ti[fvmr::kTiOffF];
+    const int offL = ti[fvmr::kTiOffL], offG = ti[fvmr::kTiOffG];
+    int nw = (i < nL) ? ta.lnodes[offL + i] : 0;
+    int4 gs = (i < nG) ? ta.gslot[offG + i] : make_int4(0, 0, 0, 0);
+    V4<G> gco = (i < nG) ? ta.gcoef[offG + i] : V4<G>{G(0.5), G(0.5), G(0.5), G(1)};
+    const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : -1;
+    S4 uc = (src >= 0) ? arg.Uin[src] : S4{0.0, 0.0, 0.0, 0.0};   // the cell's state (mixed: its FP64 state)
+    const bool needed = i < nT && ra.need[src] != 0;
+    if (i < nN) lds.N[i] = ta.nxy[offN + i];
+    for (int k = i; k < nF; k += Cfg::kThreads) {
+        lds.face[k] = ta.face[offF + k];
+        lds.nrm[k] = ta.fnrm[offF + k];
+    }
+    if (i < nL) {
+        lds.cen[i] = ta.lcxy[offL + i];
+        lds_put(lds.U, Cfg::kMaxL, i, SU{(C)uc.x, (C)uc.y, (C)uc.z, (C)uc.w});
+    }
+    if (i == 0) {
+        sStop = sFail = sBad = 0;
+        sT = sc->t;
+        sTrk = sc->t_rk;
+        sDt = sc->dt;
+    }
+    double dtl = 0.0;   // LDT: the cell's own step
+    unsigned ex = ra.ex0;
+    int done = 0;
+    __syncthreads();
+    for (; done < ra.nsteps; done++) {
+        const unsigned dtag = ra.dt0 + 1 + (unsigned)done;
+        // time step: the faces' radii, their sums per cell, the tile's minimum
+        Phys ph = run_args<G>().ph;
+        fix_scheme<SCHEME, NS>(ph);
+        const CaseBC &bc = run_args<G>().ta.cbc[0];
+        if (i < nFF) {
+            const int4 fr = lds.face[i];
+            const int L = lfield(fr.y, 0), R = lfield(fr.y, 1);
+            const bool has_R = R != fvmr::kLocalNone;
+            const V2<G> n = lds.nrm[i];
+            const V4<G> eg{n.x, n.y, (G)(double)__int_as_float(fr.z), G(0)};
+            const SU a = lds_get<SU>(lds.U, Cfg::kMaxL, L), b = lds_get<SU>(lds.U, Cfg::kMaxL, has_R ? R : L);
+            const double uL[4] = {(double)a.x, (double)a.y, (double)a.z, (double)a.w};
+            const double uR[4] = {(double)b.x, (double)b.y, (double)b.z, (double)b.w};
+            face_alpha<G, LDT>(ph, uL, uR, has_R, eg, &sAi[i], &sAv[i]);
+        }
+        __syncthreads();
+        double dtc = 1e10;
+        if (i < nT) {
+            const double vol = (double)gco.w;
+            const int f0 = gs.x & fvmr::kLocalMask, f1 = gs.y & fvmr::kLocalMask, f2 = gs.z & fvmr::kLocalMask;
+            if (LDT) {
+                dtl = bc.CFL * vol / local_alpha(ph, f0, f1, f2, sAi, sAv, vol);
+            } else {
+                const double alpha_c = cell_alpha(ph, gs.w, f0, f1, f2, sAi, sAv, vol, [&](int f, double *av, double *vv) {
+                    // the periodic pair of face f, seen from this cell (the face's L) and its R (FP64 only:
+                    // the mixed LDS states are FP32)
+                    const int4 ff = lds.face[f];
+                    const int pf = lfield(ff.y, 2);
+                    const V2<G> n = lds.nrm[pf];
+                    const double len = (double)__int_as_float(lds.face[pf].z);
+                    const SU a = lds_get<SU>(lds.U, Cfg::kMaxL, i), b = lds_get<SU>(lds.U, Cfg::kMaxL, lfield(ff.y, 1));
+                    const double Uc[4] = {(double)a.x, (double)a.y, (double)a.z, (double)a.w};
+                    const double Uo[4] = {(double)b.x, (double)b.y, (double)b.z, (double)b.w};
+                    double rc[4], ro[4];
+                    prim(Uc, rc, ph.gamma);
+                    prim(Uo, ro, ph.gamma);
+                    edge_alpha(ph, rc, ro, true, (double)n.x, (double)n.y, len, vol, av, vv);
+                });
+                dtc = fmin(dtc, fdiv(bc.CFL * vol, alpha_c));
+            }
+        }
+        if (!LDT) {
+            const double wm = wave_min(dtc);
+            if ((i & 63) == 0) sMin[i >> 6] = wm;
+        }
+        __syncthreads();
+        if (!LDT && i == 0) {
+            double m = sMin[0];
+            for (int w = 1; w < Cfg::kThreads / 64; w++) m = fmin(m, sMin[w]);
+            ll_put_double(ra.part + tile, ra.part + ra.ntiles + tile, dtag, m);
+            ll_store(ra.part + 2 * ra.ntiles + tile, dtag, (unsigned)sBad);
+        }
+        if (!LDT && i == 0) sTrk = sT;
+        S4 un = uc;
+        if (kF64) {
+            if (i < nT) un = lds_get<S4>(lds.U, Cfg::kMaxL, i);
+        }
+#pragma unroll 1
+        for (int stage = 0; stage < ra.stages; stage++) {
+            Phys ph = run_args<G>().ph;
+            fix_scheme<SCHEME, NS>(ph);
+            const CaseBC &bc = run_args<G>().ta.cbc[0];
+            opaque(nw);
+            opaque(gs.x); opaque(gs.y); opaque(gs.z);
+            opaque(gco.x); opaque(gco.y); opaque(gco.z); opaque(gco.w);
+            if (i < nG) tile_gradient(ph, lds, i, gs, gco, nw);
+            __syncthreads();
+            C F[4] = {C(0), C(0), C(0), C(0)};
+            if (i < nFF) tile_flux<C, G, NS>(ph, bc, sTrk, lds, i, F);
+            __syncthreads();
+            if (i < nFF) lds_put(lds.grfl, Cfg::kMaxFF, i, V4<C>{F[0], F[1], F[2], F[3]});
+            if (!LDT && stage == 0 && i == 0) {
+                // the global minimum, long since reduced while the fluxes were formed
+                const unsigned long long *q = ra.pub + (tile & (kRunCopies - 1)) * kRunStride;
+                unsigned long long lo, hi, fl;
+                int spin = 0;
+                do {
+                    lo = ll_load(q);
+                    hi = ll_load(q + 1);
+                    fl = ll_load(q + 2);
+                } while (!(ll_is(lo, dtag) && ll_is(hi, dtag) && ll_is(fl, dtag)) && ++spin < kRunSpin);
+                const double t = sT, T = run_args<G>().sc->T;
+                double d = ll_double(lo, hi);
+                if (t + d > T) d = T - t;
+                const int stop = spin >= kRunSpin ? 2 : (int)(fl & 3u);
+                if (!stop) {
+                    sDt = d;
+                    sT = t + d;
+                }
+                sStop = stop;
+            }
+            __syncthreads();
+            if (!LDT && stage == 0 && sStop) break;
+            const double dt = LDT ? dtl : sDt;
+            const bool last = stage + 1 == ra.stages;
+            ex++;
+            if (i < nT) {
+                double Ui[4], r[4], Unew[4];
+                if (kF64) {
+                    const SU v = lds_get<SU>(lds.U, Cfg::kMaxL, i);
+                    Ui[0] = v.x; Ui[1] = v.y; Ui[2] = v.z; Ui[3] = v.w;
+                } else {
+                    Ui[0] = uc.x; Ui[1] = uc.y; Ui[2] = uc.z; Ui[3] = uc.w;
+                }
+                const double Ub[4] = {un.x, un.y, un.z, un.w};
+                tile_rhs(lds, gs, gco, r);
+                const double a = ra.a[stage], b = ra.b[stage];
+#pragma unroll
+                for (int k = 0; k < 4; k++) Unew[k] = rk_update(Ui[k], Ub[k], r[k], dt, a, b, stage == 0);
+                if (stage == 0 && done == ra.rhs_step) st(arg.rhs_out, src, r);
+                lds_put(lds.U, Cfg::kMaxL, i, SU{(C)Unew[0], (C)Unew[1], (C)Unew[2], (C)Unew[3]});
+                if (!kF64) uc = S4{Unew[0], Unew[1], Unew[2], Unew[3]};
+                if (needed) {
+                    unsigned long long *q = ra.ll + (size_t)(ex & 1u) * 8 * nc + src;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        ll_put_double(q + (size_t)(2 * k) * nc, q + (size_t)(2 * k + 1) * nc, ex, Unew[k]);
+                }
+                if (!LDT && last && state_is_bad(Unew, ph.gamma)) {
+                    flag_bad(sc, arg.bad_list, nc, src, 0);
+                    sBad = 1;
+                }
+            }
+            if (last && done + 1 == ra.nsteps) continue;   // nobody reads the last states here
+            if (i >= nT && i < nL) {
+                const unsigned long long *q = ra.ll + (size_t)(ex & 1u) * 8 * nc + src;
+                unsigned long long w[8];
+                int spin = 0;
+                bool ok;
+                // one word is polled until it is there, then all are read (and read again while any is
+                // not): polling all eight took 35.6 instead of 30.0 us per step at 131k cells
+                while (!ll_is(ll_load(q + 7 * (size_t)nc), ex) && ++spin < kRunSpin) {}
+                do {
+                    ok = true;
+#pragma unroll
+                    for (int k = 0; k < 8; k++) w[k] = ll_load(q + (size_t)k * nc);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) ok = ok && ll_is(w[k], ex);
+                } while (!ok && ++spin < kRunSpin);
+                if (!ok) sFail = 1;
+                lds_put(lds.U, Cfg::kMaxL, i, SU{(C)ll_double(w[0], w[1]), (C)ll_double(w[2], w[3]),
+                                                 (C)ll_double(w[4], w[5]), (C)ll_double(w[6], w[7])});
+            }
+            __syncthreads();
+            if (sFail) break;
+        }
+        if (sStop || sFail) break;
+    }
+    if (i < nT) {
+        double U[4] = {uc.x, uc.y, uc.z, uc.w};
+        if (kF64) lds_state(lds.U, Cfg::kMaxL, i, U);
+        st(arg.Uout, src, U);
+    }
+    if (i == 0 && (sStop == 2 || sFail)) sc->run_failed = 1;
+    if (i == 0 && tile == 0) {
+        sc->run_done = (unsigned)done;
+        if (!LDT) {
+            sc->t = sT;
+            sc->t_rk = sTrk;
+            sc->dt = sDt;
+            sc->n_restricted = 0;
+        }
     }
 }
 
@@ -2160,6 +2579,11 @@ struct fvmr_solver {
     void *t_gcoef = nullptr;
     void *t_lcxy = nullptr, *t_fnrm = nullptr;   // V2<G> per local cell / per face (FVMR_TILE_GEOM_LOADED)
     DtRec *t_dtrec = nullptr;
+    // resident kernel (k_run): exchange buffers, allocated by fvmr_create when the handle can use it
+    const void *run_step_kernel = nullptr, *run_steady_kernel = nullptr;   // NULL: not on this handle
+    unsigned long long *run_ll = nullptr, *run_part = nullptr, *run_pub = nullptr;
+    unsigned char *run_need = nullptr;
+    unsigned run_ex = 0, run_dt = 0;      // numbers of the last exchange and time step
     // output quantities: node -> cells (caller's element order), node buffers, boundary edges
     int *nc_off = nullptr, *nc_cells = nullptr;
     double *node_buf = nullptr;               // 6 x nv: ruvp, Cp, Ma
@@ -2389,10 +2813,87 @@ int run_step(fvmr_solver *h, bool store_rhs) {
     return device_step<double, double>(h, store_rhs);
 }
 
+// The resident kernel's instantiation for a handle (pseudo-time: FP64, any scheme).  W: waves per SIMD
+// it is compiled for: 2 in FP64 (4 mixed) while two work-groups per CU are enough, else 4 (6), which
+// spills a few registers.
+template <class C, class G, int W>
+const void *run_kernel_w(const fvmr_solver *h, bool steady) {
+    const bool ns = h->ph.equation == FVMR_EQ_NS, fixed = tile_scheme_fixed(h->ph);
+    if constexpr (std::is_same<C, double>::value) {
+        if (steady) return ns ? (const void *)k_run<C, G, true, true, kTileAny, W> : (const void *)k_run<C, G, false, true, kTileAny, W>;
+    }
+    if (ns) return fixed ? (const void *)k_run<C, G, true, false, kTileGgBarthRoe, W> : (const void *)k_run<C, G, true, false, kTileAny, W>;
+    return fixed ? (const void *)k_run<C, G, false, false, kTileGgBarthRoe, W> : (const void *)k_run<C, G, false, false, kTileAny, W>;
+}
+const void *run_kernel(const fvmr_solver *h, bool steady, bool wide) {
+    if (h->mixed) return wide ? run_kernel_w<float, float, 4>(h, steady) : run_kernel_w<float, float, 6>(h, steady);
+    return wide ? run_kernel_w<double, double, 2>(h, steady) : run_kernel_w<double, double, 4>(h, steady);
+}
+
+// Launches nsteps steps (steady: pseudo-time iterations) of the resident kernel from buffer cur to
+// the next one.
+template <class C, class G>
+int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
+    const int a = h->cur, b = (a + 1) % 3;
+    RunKernArg<G> k{};
+    k.ta = tile_args<G>(h);
+    k.ph = h->ph;
+    k.Uin = h->Ubuf[a];
+    k.Uout = h->Ubuf[b];
+    k.rhs_out = h->rhs;
+    k.sc = h->sc;
+    k.bad_list = h->bad_list;
+    k.nc = h->nc;
+    const int stages = h->p.time_advance == FVMR_EVO_RK3 ? 3 : 1;
+    k.ra = RunArgs{h->run_ll, h->run_part, h->run_pub, h->run_need, h->run_ex, h->run_dt, nsteps, stages, h->ntiles,
+                   rhs_step, {0.0, 0.75, 1.0 / 3.0}, {1.0, 0.25, 2.0 / 3.0}};
+    void *args[] = {&k};
+    HIP_OK(hipLaunchCooperativeKernel(steady ? h->run_steady_kernel : h->run_step_kernel, dim3(h->ntiles + (steady ? 0 : 1)),
+                                      dim3(TileCfg<C, 0>::kThreads), args, 0, h->stream));
+    h->run_ex += (unsigned)(nsteps * stages);
+    if (!steady) h->run_dt += (unsigned)nsteps;
+    h->cur = b;
+    return FVMR_OK;
+}
+
+int read_scalars(fvmr_solver *h, Scalars &s);
+
+// n steps by the resident kernel; *done: the steps done (fewer when a step left cells to restrict,
+// which are restricted here).
+int run_resident(fvmr_solver *h, int n, bool store_rhs_last, int *done) {
+    constexpr int kMost = 10000;   // steps per launch: a fraction of a second
+    int rc;
+    for (*done = 0; *done < n;) {
+        const int k = std::min(n - *done, kMost);
+        const int rhs_step = (store_rhs_last && *done + k == n) ? k - 1 : -1;
+        rc = h->mixed ? launch_run<float, float>(h, k, rhs_step, false) : launch_run<double, double>(h, k, rhs_step, false);
+        if (rc) return rc;
+        Scalars s{};
+        if ((rc = read_scalars(h, s))) return rc;
+        if (s.run_failed) return set_error(FVMR_ERR_HIP, "resident step kernel: a work-group waited too long for its neighbours");
+        *done += (int)s.run_done;
+        if (s.bad_count > 0) {
+            if ((rc = h->mixed ? launch_restrict<float>(h, h->Ubuf[h->cur]) : launch_restrict<double>(h, h->Ubuf[h->cur]))) return rc;
+        }
+        if ((int)s.run_done < k) return FVMR_OK;
+    }
+    if (store_rhs_last) h->rhs_valid = true;
+    return FVMR_OK;
+}
+
 // n steps; the last one keeps its stage-1 rhs when store_rhs_last.  Without profiling, runs of
 // three steps replay a captured graph (the same launches with the same arguments).
 int run_steps(fvmr_solver *h, int n, bool store_rhs_last) {
     int rc, done = 0;
+    // from 4 steps on: a cooperative launch costs about 40 us more than an ordinary one, a resident step
+    // 8-12 us less than a launched one (8,192 to 120,000 cells: 3 steps 143 / 201 against 143 / 208 us,
+    // 5 steps 182 / 274 against 199 / 301 us)
+    constexpr int kRunMin = 4;
+    if (h->run_step_kernel && !h->use_graphs && !h->profiling && n >= kRunMin) {
+        // (after a step with cells to restrict the rest runs by the kernels below, so that a flow
+        // which needs it in every step is not stopped at each)
+        if ((rc = run_resident(h, n, store_rhs_last, &done))) return rc;
+    }
     if (h->use_graphs && !h->profiling) {
         const int eager_tail = store_rhs_last ? 1 : 0;
         while (n - done - eager_tail >= 3) {
@@ -2421,6 +2922,58 @@ int run_steps(fvmr_solver *h, int n, bool store_rhs_last) {
     }
     for (; done < n; done++)
         if ((rc = run_step(h, store_rhs_last && done == n - 1))) return rc;
+    return FVMR_OK;
+}
+
+int read_scalars(fvmr_solver *h, Scalars &s) {
+    HIP_OK(hipMemcpyAsync(&s, h->sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
+    HIP_OK(hipStreamSynchronize(h->stream));
+    return FVMR_OK;
+}
+
+// Whether the resident kernel can serve the handle (one case, the default work-group shape, all
+// work-groups on the device at once, tiles that need each other's cells mutually; not mixed precision
+// with periodic faces, whose time step takes FP64 states across a face), and its buffers.
+int run_setup(fvmr_solver *h, const std::vector<int2> &cslot, const std::vector<int> &halo) {
+    if (!h->tiles || h->ncases != 1 || h->shape != 0 || (h->mixed && h->ph.has_periodic)) return FVMR_OK;
+    int coop = 0, cus = 0;
+    HIP_OK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, h->device));
+    HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
+    if (!coop) return FVMR_OK;
+    const int threads = shape_threads(h->mixed, 0);
+    auto pick = [&](bool steady, int groups) -> const void * {
+        for (bool wide : {true, false}) {
+            const void *kern = run_kernel(h, steady, wide);
+            int per = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, threads, 0) == hipSuccess && per * cus >= groups)
+                return kern;
+        }
+        return nullptr;
+    };
+    const void *run = pick(false, h->ntiles + 1), *steady = h->mixed ? nullptr : pick(true, h->ntiles);
+    if (!run && !steady) return FVMR_OK;
+    const int nc = h->nc;
+    for (int c = 0; c < nc; c++)
+        for (int j = 0; j < 3; j++) {
+            const int o = cslot[(size_t)j * nc + c].y;
+            if (o < 0) continue;
+            bool back = false;
+            for (int q = 0; q < 3; q++) back = back || cslot[(size_t)q * nc + o].y == c;
+            if (!back) return FVMR_OK;
+        }
+    std::vector<unsigned char> need(nc, 0);
+    for (int c : halo) need[c] = 1;
+    int rc;
+    if ((rc = upload(&h->run_need, need, h->stream))) return rc;
+    const size_t words[3] = {16 * (size_t)nc, 3 * (size_t)h->ntiles, (size_t)kRunCopies * kRunStride};
+    unsigned long long **dst[3] = {&h->run_ll, &h->run_part, &h->run_pub};
+    for (int k = 0; k < 3; k++) {
+        HIP_OK(hipMalloc((void **)dst[k], words[k] * sizeof(unsigned long long)));
+        HIP_OK(hipMemsetAsync(*dst[k], 0, words[k] * sizeof(unsigned long long), h->stream));
+    }
+    HIP_OK(hipStreamSynchronize(h->stream));   // need goes out of scope
+    h->run_step_kernel = run;
+    h->run_steady_kernel = steady;
     return FVMR_OK;
 }
 
@@ -2467,7 +3020,8 @@ void free_all(fvmr_solver *h) {
                     h->eint, h->partial, h->norm_out, h->bad_list, h->sc, h->t_info, h->t_halo, h->t_lnodes,
                     h->t_nxy, h->t_gslot, h->t_face, h->t_gcoef, h->t_dtrec, h->t_lcxy, h->t_fnrm,
                     h->nc_off, h->nc_cells, h->node_buf, h->cbc, h->tile_case_begin, h->perm_dev, h->io_soa,
-                    h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev};
+                    h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev, h->run_ll, h->run_part, h->run_pub,
+                    h->run_need};
     for (void *q : ptrs) if (q) (void)hipFree(q);
     for (int k = 0; k < kNumProf; k++)
         for (auto e : h->pending[k]) (void)hipEventDestroy(e);
@@ -2721,10 +3275,17 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             fvmr::TileInput ti{nc, nf, sx.data(), sy.data(), cnode.data(), eL.data(), eR.data(), et.data(), ep.data(),
                                en0.data(), en1.data(), elen.data(), m->node_xy[0], m->node_xy[1], vol.data(), dtcode.data(),
                                ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin};
+            // a mesh with fewer default tiles than the device has CUs is cut into smaller ones, one per
+            // CU and one CU left for the resident kernel's reducing work-group: its phases then share
+            // a CU's LDS among fewer waves (8,192 cells, 33 instead of 150 per tile: 16.6 instead of
+            // 18.4 us per SSP-RK3 step); fewer than 32 cells leave lanes of the only wave idle
+            int cus = 0;
+            if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
+            const int spread = (ncases == 1 && cus > 1) ? std::max(32, (nc + cus - 2) / (cus - 1)) : kTileMaxCells;
             auto caps_of = [&](auto cfg) {
                 using Cfg = decltype(cfg);
-                return fvmr::TileCaps{std::min(p->tile_cells ? p->tile_cells : Cfg::kCells, Cfg::kMaxG), Cfg::kMaxG,
-                                      Cfg::kMaxL, Cfg::kMaxN, Cfg::kMaxF, Cfg::kMaxFF};
+                return fvmr::TileCaps{std::min(p->tile_cells ? p->tile_cells : std::min(Cfg::kCells, spread), Cfg::kMaxG),
+                                      Cfg::kMaxG, Cfg::kMaxL, Cfg::kMaxN, Cfg::kMaxF, Cfg::kMaxFF};
             };
             h->shape = shape_of_threads(h->mixed, p->tile_threads);
             fvmr::TileCaps caps;
@@ -2830,6 +3391,7 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
         hipMemcpyAsync(h->sc, s0.data(), ncases * sizeof(Scalars), hipMemcpyHostToDevice, h->stream) != hipSuccess ||
         hipStreamSynchronize(h->stream) != hipSuccess)
         return bail(set_error(FVMR_ERR_HIP, "initial copy failed"));
+    if ((rc = run_setup(h, cslot, tm.halo))) return bail(rc);
     *out = h;
     return FVMR_OK;
 }
@@ -2996,12 +3558,6 @@ int fvmr_get_state(fvmr_handle *h, double *const U[4]) {
     return read_back(h, h->Ubuf[h->cur], U);
 }
 
-static int read_scalars(fvmr_handle *h, Scalars &s) {
-    HIP_OK(hipMemcpyAsync(&s, h->sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
-    HIP_OK(hipStreamSynchronize(h->stream));
-    return FVMR_OK;
-}
-
 int fvmr_advance(fvmr_handle *h, int nsteps, double *t, double T, fvmr_step_info *info) {
     if (!h || !t || nsteps < 0) return set_error(FVMR_ERR_INVALID_ARG, "invalid argument");
     Scalars s{};
@@ -3009,7 +3565,7 @@ int fvmr_advance(fvmr_handle *h, int nsteps, double *t, double T, fvmr_step_info
     if (rc) return rc;
     s.t = *t;
     s.T = T;
-    s.counter = 0; s.bad_count = 0; s.n_restricted = 0;
+    s.run_done = s.run_failed = 0; s.bad_count = 0; s.n_restricted = 0;
     HIP_OK(hipMemcpyAsync(h->sc, &s, sizeof(Scalars), hipMemcpyHostToDevice, h->stream));
     if ((rc = run_steps(h, nsteps, true))) return rc;
     if ((rc = read_scalars(h, s))) return rc;
@@ -3072,7 +3628,7 @@ int fvmr_batch_advance(fvmr_handle *h, int nsteps, double *t, const double *T) {
     HIP_OK(hipMemcpyAsync(s.data(), h->sc, s.size() * sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));
     for (int c = 0; c < h->ncases; c++) { s[c].t = t[c]; s[c].T = T[c]; }
-    s[0].counter = 0; s[0].bad_count = 0; s[0].n_restricted = 0;
+    s[0].bad_count = 0; s[0].n_restricted = 0;
     HIP_OK(hipMemcpyAsync(h->sc, s.data(), s.size() * sizeof(Scalars), hipMemcpyHostToDevice, h->stream));
     int rc;
     if ((rc = run_steps(h, nsteps, false))) return rc;
