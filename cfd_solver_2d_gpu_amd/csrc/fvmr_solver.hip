@@ -185,6 +185,46 @@ template <> __device__ __forceinline__ double fdiv<double>(double a, double b) {
 #endif
 template <class T> __device__ __forceinline__ T fsqrt(T a) { return sqrt(a); }
 template <> __device__ __forceinline__ float fsqrt<float>(float a) { return __builtin_amdgcn_sqrtf(a); }
+#if FVMR_FAST_DIV
+// FP64 square root without the library's scaling of tiny operands (half its instructions): the hardware's
+// 1/sqrt estimate, one Goldschmidt step (g -> sqrt(a), h -> 1 / (2 sqrt(a))) and two corrections with the
+// residual a - g g; 0 and infinity are their own roots.
+template <> __device__ __forceinline__ double fsqrt<double>(double a) {
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, a), h, g);
+    g = fma(fma(-g, g, a), h, g);
+    return __builtin_amdgcn_class(a, 0x260) ? a : g;   // -0, +0, +infinity
+}
+#endif
+// The smaller / larger of two values, the other one where one is a quiet NaN: the bare instructions.
+// fmin and fmax first quiet each operand that the compiler has not seen computed (signalling NaN, which
+// no arithmetic makes): 60 more instructions per cell in the limiter.
+template <class T> __device__ __forceinline__ T vmin(T a, T b) { return fmin(a, b); }
+template <class T> __device__ __forceinline__ T vmax(T a, T b) { return fmax(a, b); }
+template <> __device__ __forceinline__ double vmin<double>(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+template <> __device__ __forceinline__ double vmax<double>(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+template <> __device__ __forceinline__ float vmin<float>(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+template <> __device__ __forceinline__ float vmax<float>(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 
 __device__ __forceinline__ void ld(const S4 *p, int i, double u[4]) {
     const S4 v = p[i];
@@ -757,50 +797,112 @@ __device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[NV], const
             const V Kh = (V)ph.venkat_K * fsqrt(vol);
             eps2 = Kh * Kh * Kh;
         }
+        if constexpr (std::is_floating_point<C>::value) {
+            // Straight-line code over the variables, so that their dependent chains overlap: with one
+            // branch per quotient the gradient phase took 1.9 us at any occupancy, 10 cycles an instruction.
+            // Bounds over the cell and its non-periodic neighbours (a slot without one: the cell's own
+            // state, which leaves both bounds as they are); a NaN bound already makes the gradient NaN.
+            C hrel[NV], lrel[NV], phi[NV];
+            bool nan = false;
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
-            // bounds over the cell and its non-periodic neighbours (fmin/fmax: a NaN bound
-            // already makes the Green-Gauss or least-squares gradient NaN).  Without periodic
-            // faces a slot with no neighbour holds the cell's own state, which leaves both
-            // bounds as they are, so the plain types skip the per-slot test
-            C lo = Uc[k], hi = Uc[k];
-            if (std::is_floating_point<C>::value && !ph.has_periodic) {
+            for (int k = 0; k < NV; k++) {
+                C lo = Uc[k], hi = Uc[k];
 #pragma unroll
-                for (int i = 0; i < 3; i++) { lo = fmin(lo, S.Uo(i, k)); hi = fmax(hi, S.Uo(i, k)); }
+                for (int i = 0; i < 3; i++) {
+                    const C o = (!ph.has_periodic || (fl[i] & 2)) ? C(S.Uo(i, k)) : Uc[k];
+                    lo = vmin(lo, o);
+                    hi = vmax(hi, o);
+                }
+                hrel[k] = hi - Uc[k];
+                lrel[k] = lo - Uc[k];
+                nan = nan || isnan(hrel[k]) || isnan(lrel[k]);
+            }
+            if (ph.limiter == FVMR_LIM_BARTH) {
+                // min over vertices of min(1, hrel / (rel + eps)) (rel > 0) and of
+                // min(1, lrel / (rel - eps)) (rel < 0): division and addition round monotonically, so each
+                // minimum is one division by the extreme rel plus eps, which counts when it is below 1
+#pragma unroll
+                for (int k = 0; k < NV; k++) {
+                    C rel[3];
+#pragma unroll
+                    for (int jn = 0; jn < 3; jn++) {
+                        const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
+                        rel[jn] = Un - Uc[k];
+                    }
+                    const C mp = vmax(vmax(rel[0], rel[1]), rel[2]), mn = vmin(vmin(rel[0], rel[1]), rel[2]);
+                    const C dpos = mp + C(fvmr::kEPS), dneg = mn - C(fvmr::kEPS);
+                    const bool cpos = (mp > C(0)) & (hrel[k] < dpos), cneg = (mn < C(0)) & (lrel[k] > dneg);
+                    if constexpr (std::is_same<C, double>::value) {
+                        // one division, of the smaller of the two quotients (compared crosswise: dpos > 0 >
+                        // dneg); where they agree to a rounding either will do
+                        C num = cpos ? hrel[k] : C(1), den = cpos ? dpos : C(1);
+                        const bool neg = cneg & (lrel[k] * den > num * dneg);
+                        num = neg ? lrel[k] : num;
+                        den = neg ? dneg : den;
+                        phi[k] = fdiv(num, den);
+                    } else {
+                        const C qp = fdiv(hrel[k], dpos), qn = fdiv(lrel[k], dneg);
+                        phi[k] = cpos ? tmin(C(1), qp) : C(1);
+                        phi[k] = cneg ? tmin(phi[k], qn) : phi[k];
+                    }
+                }
+                if (nan) {
+                    // NaN bounds: the vertex loop as the reference writes it
+#pragma unroll
+                    for (int k = 0; k < NV; k++) {
+                        if (!isnan(hrel[k]) && !isnan(lrel[k])) continue;
+                        phi[k] = C(1);
+#pragma unroll
+                        for (int jn = 0; jn < 3; jn++) {
+                            const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
+                            C rel = Un - Uc[k];
+                            C pn = C(1.0);
+                            if (rel > C(0)) { rel += C(fvmr::kEPS); pn = tmin(C(1), fdiv(hrel[k], rel)); }
+                            else if (rel < C(0)) { rel -= C(fvmr::kEPS); pn = tmin(C(1), fdiv(lrel[k], rel)); }
+                            phi[k] = tmin(phi[k], pn);
+                        }
+                    }
+                }
             } else {
 #pragma unroll
-                for (int i = 0; i < 3; i++)
-                    if (fl[i] & 2) { lo = fmin(lo, S.Uo(i, k)); hi = fmax(hi, S.Uo(i, k)); }
+                for (int k = 0; k < NV; k++) {
+                    phi[k] = C(1);
+#pragma unroll
+                    for (int jn = 0; jn < 3; jn++) {
+                        const N_t ndx = S.N(jn, 0), ndy = S.N(jn, 1);
+                        const C d2 = gx[k] * ndx + gy[k] * ndy;
+                        const C d1 = (d2 > C(0)) ? hrel[k] : lrel[k];
+                        const C num = (d1 * d1 + eps2) * d2 + C(2.0) * d2 * d2 * d1;
+                        const C den = d1 * d1 + C(2.0) * d2 * d2 + d1 * d2 + eps2;
+                        const C q = fdiv(num, den * d2);
+                        phi[k] = tmin(phi[k], (d2 != C(0)) ? q : C(1));
+                    }
+                }
             }
+#pragma unroll
+            for (int k = 0; k < NV; k++) {
+                gx[k] *= phi[k];
+                gy[k] *= phi[k];
+            }
+            return;
+        }
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            // the dual types, whose derivatives follow the branch that the values take
+            C lo = Uc[k], hi = Uc[k];
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+                if (fl[i] & 2) { lo = fmin(lo, S.Uo(i, k)); hi = fmax(hi, S.Uo(i, k)); }
             C phi = C(1.0);
             const C hrel = hi - Uc[k], lrel = lo - Uc[k];
             if (ph.limiter == FVMR_LIM_BARTH && !isnan(hrel) && !isnan(lrel)) {
-                // min over vertices of min(1, hrel / (rel + eps)) (rel > 0) and of
-                // min(1, lrel / (rel - eps)) (rel < 0): division rounds monotonically, so each
-                // minimum is one division by the extreme denominator, needed only when the
-                // quotient can fall below 1
                 C dpos = C(0), dneg = C(0);
-                if (std::is_floating_point<C>::value) {
-                    // rounding is monotonic, so the largest rel + eps is the largest rel plus
-                    // eps: the extremes first, eps once (the same values, no per-vertex selects)
-                    C mp = C(0), mn = C(0);
 #pragma unroll
-                    for (int jn = 0; jn < 3; jn++) {
-                        const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                        const C rel = Un - Uc[k];
-                        mp = fmax(mp, rel);
-                        mn = fmin(mn, rel);
-                    }
-                    if (mp > C(0)) dpos = mp + C(fvmr::kEPS);
-                    if (mn < C(0)) dneg = mn - C(fvmr::kEPS);
-                } else {
-#pragma unroll
-                    for (int jn = 0; jn < 3; jn++) {
-                        const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                        const C rel = Un - Uc[k];
-                        if (rel > C(0)) dpos = fmax(dpos, rel + C(fvmr::kEPS));
-                        else if (rel < C(0)) dneg = fmin(dneg, rel - C(fvmr::kEPS));
-                    }
+                for (int jn = 0; jn < 3; jn++) {
+                    const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
+                    const C rel = Un - Uc[k];
+                    if (rel > C(0)) dpos = fmax(dpos, rel + C(fvmr::kEPS));
+                    else if (rel < C(0)) dneg = fmin(dneg, rel - C(fvmr::kEPS));
                 }
                 if (dpos > C(0) && hrel < dpos) phi = tmin(phi, fdiv(hrel, dpos));
                 if (dneg < C(0) && lrel > dneg) phi = tmin(phi, fdiv(lrel, dneg));
@@ -1140,15 +1242,21 @@ struct DtRec {
     double vol;
 };
 
+// Three ints: one 12-byte load; 16 bytes apart in LDS, where 12-byte records would straddle its 16-byte reads.
+struct I3 {
+    int x, y, z;
+};
+struct alignas(16) I3L : I3 {};
+
 template <class G>
 struct TileArgs {
     const int *info;          // fvmr::kTileInfo ints per tile
     const int *halo;          // device cell ids of halo cells
     const V2<double> *nxy;    // node coordinates per tile
     const int *lnodes;        // per local cell: 3 local node ids
-    const int4 *gslot;        // per gradient cell: 3 slot words + dtcode
+    const I3 *gslot;          // per gradient cell: 3 slot words
     const V4<G> *gcoef;       // per gradient cell: Green-Gauss weights of the 3 slots, volume
-    const int4 *face;         // per face: nodes | BC code, L | R | pair face, float length, edge
+    const I3 *face;           // per face: nodes | BC code, L | R | pair face, float length
     const DtRec *dtrec;       // per device cell
     const V2<G> *lcxy;        // per local cell: centroid (FVMR_TILE_GEOM_LOADED)
     const V2<G> *fnrm;        // per face: normal (FVMR_TILE_GEOM_LOADED)
@@ -1158,21 +1266,22 @@ struct TileArgs {
 
 __device__ __forceinline__ int lfield(int w, int k) { return (w >> (fvmr::kLocalBits * k)) & fvmr::kLocalMask; }
 
-// Centroid of a cell from its nodes as the host computes it ((0 + x0) + x1 + x2) / 3 (the
-// quotient by fdiv, which rounds as IEEE division does).
-__device__ __forceinline__ V2<double> tile_centroid(const V2<double> *sN, int w) {
+// s / 3 rounded as IEEE division rounds it: the product with 1/3, corrected once with its residual
+// (Markstein: the constant is the correctly rounded reciprocal).
+__device__ __forceinline__ double third(double s) {
+    const double q = s * (1.0 / 3.0);
+    return fma(fma(-3.0, q, s), 1.0 / 3.0, q);
+}
+// Centroid of a cell from its nodes as the host computes it, ((0 + x0) + x1 + x2) / 3.
+__device__ __forceinline__ V2<double> tile_centroid(const V2<double> &a, const V2<double> &b, const V2<double> &c) {
 #pragma clang fp contract(off)
-    const V2<double> a = sN[lfield(w, 0)], b = sN[lfield(w, 1)], c = sN[lfield(w, 2)];
-    double sx = 0.0, sy = 0.0;
-    sx += a.x; sx += b.x; sx += c.x;
-    sy += a.y; sy += b.y; sy += c.y;
-    return V2<double>{fdiv(sx, 3.0), fdiv(sy, 3.0)};
+    return V2<double>{third(0.0 + a.x + b.x + c.x), third(0.0 + a.y + b.y + c.y)};
 }
 
 // Face geometry from a face record as the host computes it: normal (dy, -dx) / L with the
 // stored (float) length L, midpoint (xa + xb) / 2; rounded to G like the global records.
 template <class G>
-__device__ __forceinline__ void tile_face_geom(const V2<double> *sN, int4 fr, V4<G> &eg, V2<G> &em) {
+__device__ __forceinline__ void tile_face_geom(const V2<double> *sN, const I3 fr, V4<G> &eg, V2<G> &em) {
 #pragma clang fp contract(off)
     const V2<double> a = sN[lfield(fr.x, 0)], b = sN[lfield(fr.x, 1)];
     const double len = (double)__int_as_float(fr.z);
@@ -1182,7 +1291,7 @@ __device__ __forceinline__ void tile_face_geom(const V2<double> *sN, int4 fr, V4
 }
 // Face geometry with the normal of face f already formed in sNrm.
 template <class G>
-__device__ __forceinline__ void tile_face_geom_n(const V2<double> *sN, const V2<G> *sNrm, int f, int4 fr, V4<G> &eg,
+__device__ __forceinline__ void tile_face_geom_n(const V2<double> *sN, const V2<G> *sNrm, int f, const I3 fr, V4<G> &eg,
                                                  V2<G> &em) {
 #pragma clang fp contract(off)
     const V2<double> a = sN[lfield(fr.x, 0)], b = sN[lfield(fr.x, 1)];
@@ -1191,12 +1300,12 @@ __device__ __forceinline__ void tile_face_geom_n(const V2<double> *sN, const V2<
     em = V2<G>{(G)((a.x + b.x) / 2.0), (G)((a.y + b.y) / 2.0)};
 }
 template <class G>
-__device__ __forceinline__ V2<G> tile_face_mid(const V2<double> *sN, int4 fr) {
+__device__ __forceinline__ V2<G> tile_face_mid(const V2<double> *sN, const I3 fr) {
 #pragma clang fp contract(off)
     const V2<double> a = sN[lfield(fr.x, 0)], b = sN[lfield(fr.x, 1)];
     return V2<G>{(G)((a.x + b.x) / 2.0), (G)((a.y + b.y) / 2.0)};
 }
-__device__ __forceinline__ int tile_btype(int4 fr) {
+__device__ __forceinline__ int tile_btype(const I3 fr) {
     const int bc = (fr.x >> fvmr::kBcShift) & 127;
     return bc ? bc + fvmr::kBcBase : -1;
 }
@@ -1302,16 +1411,25 @@ struct TileLds {
     static_assert(Cfg::kMaxFF * sizeof(V4<C>) <= Cfg::kMaxG * sizeof(Grad<G>), "flux buffer overlays the gradients");
     char U[Cfg::kMaxL * sizeof(SU)];
     V2<double> N[Cfg::kMaxN];
-    int4 face[Cfg::kMaxF];
+    I3L face[Cfg::kMaxF];
     char grfl[Cfg::kMaxG * sizeof(Grad<G>)];
     V2<G> cen[Cfg::kMaxL];
     V2<G> nrm[Cfg::kMaxF];
 };
 
+// -x where the slot word says that the cell is the face's R: the word's bit 20 into the sign bit.
+static_assert(fvmr::kGsIsR == 1 << 20, "the R flag moves to bit 31");
+__device__ __forceinline__ int sign_of_slot(int sw) { return (sw << 11) & (int)0x80000000; }
+__device__ __forceinline__ float negate_if_R(float x, int sw) { return __int_as_float(__float_as_int(x) ^ sign_of_slot(sw)); }
+__device__ __forceinline__ double negate_if_R(double x, int sw) {
+    return __hiloint2double(__double2hiint(x) ^ sign_of_slot(sw), __double2loint(x));
+}
+
 // Limited gradient of local cell i (tile or first ring) into LDS.  gs: its slot words, gco: its
-// Green-Gauss weights and volume, nw: its nodes.
-template <class C, class G, class Cfg>
-__device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg> &s, int i, const int4 gs,
+// Green-Gauss weights and volume, nw: its nodes.  CEN: its centroid is formed here, from the nodes that the
+// limiter reads in any case, and put into LDS for the fluxes (only least squares reads a neighbour's here).
+template <bool CEN, class C, class G, class Cfg>
+__device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg> &s, int i, const I3 gs,
                                               const V4<G> gco, int nw) {
     using SU = TileState<C>;
     const int sw[3] = {gs.x, gs.y, gs.z};
@@ -1321,7 +1439,16 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
         const SU v = lds_get<SU>(s.U, Cfg::kMaxL, i);
         Uc[0] = (C)v.x; Uc[1] = (C)v.y; Uc[2] = (C)v.z; Uc[3] = (C)v.w;
     }
-    const C xc = (C)s.cen[i].x, yc = (C)s.cen[i].y;
+    const V2<double> nd[3] = {s.N[lfield(nw, 0)], s.N[lfield(nw, 1)], s.N[lfield(nw, 2)]};
+    V2<G> cen;
+    if (CEN) {
+        const V2<double> ct = tile_centroid(nd[0], nd[1], nd[2]);
+        cen = V2<G>{(G)ct.x, (G)ct.y};
+        s.cen[i] = cen;
+    } else {
+        cen = s.cen[i];
+    }
+    const C xc = (C)cen.x, yc = (C)cen.y;
     struct {
         C a[3][3], u[3][4], n[3][2];
         __device__ __forceinline__ C A(int j, int q) const { return a[j][q]; }
@@ -1335,8 +1462,7 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
         const int out = (sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask;
         const bool has_out = out != fvmr::kLocalNone;
         const bool periodic = (sw[j] & fvmr::kGsPeriodic) != 0;
-        const C sgn = (sw[j] & fvmr::kGsIsR) ? C(-1) : C(1);
-        const int4 fr = s.face[f];
+        const I3 fr = s.face[f];
         V4<G> eg;
         V2<G> em;
         tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
@@ -1344,15 +1470,14 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
             const SU v = lds_get<SU>(s.U, Cfg::kMaxL, has_out ? out : i);
             sl.u[j][0] = (C)v.x; sl.u[j][1] = (C)v.y; sl.u[j][2] = (C)v.z; sl.u[j][3] = (C)v.w;
         }
-        const V2<double> nd = s.N[lfield(nw, j)];
-        sl.n[j][0] = (C)(G)nd.x - xc;
-        sl.n[j][1] = (C)(G)nd.y - yc;
+        sl.n[j][0] = (C)(G)nd[j].x - xc;
+        sl.n[j][1] = (C)(G)nd[j].y - yc;
         if (ph.gradient == FVMR_GRA_GREENGAUSS) {
             // weight g_C of the slot precomputed by the host (the device formula in FP64)
             const C len = (C)eg.z;
             sl.a[j][0] = (C)(j == 0 ? gco.x : (j == 1 ? gco.y : gco.z));
-            sl.a[j][1] = (C)eg.x * len * sgn;
-            sl.a[j][2] = (C)eg.y * len * sgn;
+            sl.a[j][1] = negate_if_R((C)eg.x * len, sw[j]);
+            sl.a[j][2] = negate_if_R((C)eg.y * len, sw[j]);
         } else {
             C dxn = C(0), dyn = C(0);
             if (has_out && !periodic) {   // element neighbours exclude periodic faces
@@ -1381,7 +1506,7 @@ template <class C, class G, bool NS, class Cfg>
 __device__ __forceinline__ void tile_flux(const Phys &ph, const CaseBC &bc, double t_rk, const TileLds<C, G, Cfg> &s,
                                           int f, C F[4]) {
     const TileCells<G, TileState<C>> cells{s.U, Cfg::kMaxL, s.cen, s.grfl, Cfg::kMaxG};
-    const int4 fr = s.face[f];
+    const I3 fr = s.face[f];
     V4<G> eg;
     V2<G> em;
     tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
@@ -1394,7 +1519,7 @@ __device__ __forceinline__ void tile_flux(const Phys &ph, const CaseBC &bc, doub
 
 // r = -(1/V) sum_j s_j F_j of a tile cell, the fluxes of its faces taken from LDS in slot order.
 template <class C, class G, class Cfg>
-__device__ __forceinline__ void tile_rhs(const TileLds<C, G, Cfg> &s, const int4 gs, const V4<G> gco, double r[4]) {
+__device__ __forceinline__ void tile_rhs(const TileLds<C, G, Cfg> &s, const I3 gs, const V4<G> gco, double r[4]) {
     const int sw[3] = {gs.x, gs.y, gs.z};
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -1463,28 +1588,29 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     // thread i owns local cell i (phases 2, 3, 5) and face i (phase 4); its records are
     // fetched with the staging loads
     const int i = tid;
-    const int nw = (i < nL) ? ta.lnodes[offL + i] : 0;
-    const int4 gs = (i < nG) ? ta.gslot[offG + i] : make_int4(0, 0, 0, 0);
+    constexpr bool kOwnCen = SCHEME == kTileGgBarthRoe && FVMR_TILE_GEOM_LOADED;
+    const int nw = (i < (kOwnCen ? nG : nL)) ? ta.lnodes[offL + i] : 0;
+    const I3 gs = (i < nG) ? ta.gslot[offG + i] : I3{0, 0, 0};
     const V4<G> gco = (i < nG) ? ta.gcoef[offG + i] : V4<G>{G(0.5), G(0.5), G(0.5), G(1)};
     // 1. stage nodes, states and face records: every global load is issued before the first
     // LDS store (a store between loads would make each wave wait for the loads before it)
     const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : -1;
     const S4 uin = (src >= 0) ? Uin[src] : S4{0.0, 0.0, 0.0, 0.0};
     const V2<double> nd = (tid < nN) ? ta.nxy[offN + tid] : V2<double>{0.0, 0.0};
-    const int4 fr0 = (tid < nF) ? ta.face[offF + tid] : make_int4(0, 0, 0, 0);
-    const int4 fr1 = (tid + kTileThreads < nF) ? ta.face[offF + tid + kTileThreads] : make_int4(0, 0, 0, 0);
+    const I3 fr0 = (tid < nF) ? ta.face[offF + tid] : I3{0, 0, 0};
+    const I3 fr1 = (tid + kTileThreads < nF) ? ta.face[offF + tid + kTileThreads] : I3{0, 0, 0};
     const S4 un = (!first && i < nT) ? Un[c0 + i] : S4{0.0, 0.0, 0.0, 0.0};
 #if FVMR_TILE_GEOM_LOADED
-    const V2<G> cc = (i < nL) ? ta.lcxy[offL + i] : V2<G>{G(0), G(0)};
+    const V2<G> cc = (!kOwnCen && i < nL) ? ta.lcxy[offL + i] : V2<G>{G(0), G(0)};
     const V2<G> nr0 = (tid < nF) ? ta.fnrm[offF + tid] : V2<G>{G(0), G(0)};
     const V2<G> nr1 = (tid + kTileThreads < nF) ? ta.fnrm[offF + tid + kTileThreads] : V2<G>{G(0), G(0)};
 #endif
     if (tid < nN) lds.N[tid] = nd;
-    if (tid < nF) lds.face[tid] = fr0;
-    if (tid + kTileThreads < nF) lds.face[tid + kTileThreads] = fr1;
+    if (tid < nF) static_cast<I3 &>(lds.face[tid]) = fr0;
+    if (tid + kTileThreads < nF) static_cast<I3 &>(lds.face[tid + kTileThreads]) = fr1;
     if (i < nL) lds_put(lds.U, Cfg::kMaxL, i, SU{(C)uin.x, (C)uin.y, (C)uin.z, (C)uin.w});
 #if FVMR_TILE_GEOM_LOADED
-    if (i < nL) lds.cen[i] = cc;
+    if (!kOwnCen && i < nL) lds.cen[i] = cc;
     if (tid < nF) lds.nrm[tid] = nr0;
     if (tid + kTileThreads < nF) lds.nrm[tid + kTileThreads] = nr1;
     __syncthreads();
@@ -1492,7 +1618,7 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     __syncthreads();
     // 2. centroids and face normals
     if (i < nL) {
-        const V2<double> ct = tile_centroid(lds.N, nw);
+        const V2<double> ct = tile_centroid(lds.N[lfield(nw, 0)], lds.N[lfield(nw, 1)], lds.N[lfield(nw, 2)]);
         lds.cen[i] = V2<G>{(G)ct.x, (G)ct.y};
     }
     for (int k = tid; k < nF; k += kTileThreads) {
@@ -1504,7 +1630,7 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     __syncthreads();
 #endif
     // 3. limited gradients of the tile and the first ring
-    if (i < nG) tile_gradient(ph, lds, i, gs, gco, nw);
+    if (i < nG) tile_gradient<kOwnCen>(ph, lds, i, gs, gco, nw);
     __syncthreads();
     // 4. one canonical flux per face of the tile (nFF <= threads), written over the gradients
     const double t_rk = sc[cs].t_rk;
@@ -1632,7 +1758,7 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
     constexpr int kTileMaxFF = Cfg::kMaxFF;
     __shared__ __align__(16) char sU[kTileMaxG * sizeof(S4)];   // states, 16-byte columns (lds_put)
     __shared__ V2<double> sN[kTileMaxN];
-    __shared__ int4 sFace[kTileMaxFF];   // faces of the tile cells
+    __shared__ I3L sFace[kTileMaxFF];   // faces of the tile cells
     __shared__ double sAi[kTileMaxFF], sAv[kTileMaxFF];
     __shared__ double sMin[kTileThreads / 64];
     static_assert(kTileMaxG <= kTileThreads, "one cell per thread");
@@ -1646,11 +1772,11 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
     static_assert(kTileMaxN <= kTileThreads, "one node per thread");
     const DtRec dr = (tid < nT) ? ta.dtrec[c0 + tid] : DtRec{0, 0, 1.0};
     const V2<double> nd = (tid < nN) ? ta.nxy[offN + tid] : V2<double>{0.0, 0.0};
-    const int4 fr = (tid < nFF) ? ta.face[offF + tid] : make_int4(0, 0, 0, 0);
+    const I3 fr = (tid < nFF) ? ta.face[offF + tid] : I3{0, 0, 0};
     const int src = (tid < nG) ? (tid < nT ? c0 + tid : ta.halo[offH + tid - nT]) : -1;
     const S4 u = (src >= 0) ? U[src] : S4{0.0, 0.0, 0.0, 0.0};
     if (tid < nN) sN[tid] = nd;
-    if (tid < nFF) sFace[tid] = fr;
+    if (tid < nFF) static_cast<I3 &>(sFace[tid]) = fr;
     if (tid < nG) lds_put(sU, kTileMaxG, tid, u);
     __syncthreads();
     // faces of the tile cells (one per thread): L and R (when present) are tile or first-ring cells
@@ -1678,9 +1804,9 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
         const double alpha_c = cell_alpha(ph, dr.code, lfield(dr.faces, 0), lfield(dr.faces, 1), lfield(dr.faces, 2), sAi, sAv, dr.vol,
             [&](int f, double *av, double *vv) {
                 // the periodic pair of face f, seen from this cell (the face's L) and its R
-                const int4 ff = sFace[f];
+                const I3 ff = sFace[f];
                 const int out = lfield(ff.y, 1);
-                const int4 pr = ta.face[offF + lfield(ff.y, 2)];
+                const I3 pr = ta.face[offF + lfield(ff.y, 2)];
                 V4<G> eg;
                 V2<G> em;
                 tile_face_geom<G>(sN, pr, eg, em);
@@ -1873,14 +1999,15 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
     const int offH = ti[fvmr::kTiOffH], offN = ti[fvmr::kTiOffN], offF = ti[fvmr::kTiOffF];
     const int offL = ti[fvmr::kTiOffL], offG = ti[fvmr::kTiOffG];
     int nw = (i < nL) ? ta.lnodes[offL + i] : 0;
-    int4 gs = (i < nG) ? ta.gslot[offG + i] : make_int4(0, 0, 0, 0);
+    I3 gs = (i < nG) ? ta.gslot[offG + i] : I3{0, 0, 0};
     V4<G> gco = (i < nG) ? ta.gcoef[offG + i] : V4<G>{G(0.5), G(0.5), G(0.5), G(1)};
     const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : -1;
     S4 uc = (src >= 0) ? arg.Uin[src] : S4{0.0, 0.0, 0.0, 0.0};   // the cell's state (mixed: its FP64 state)
     const bool needed = i < nT && ra.need[src] != 0;
+    const int code = (!LDT && i < nT) ? ta.dtrec[src].code : 0;
     if (i < nN) lds.N[i] = ta.nxy[offN + i];
     for (int k = i; k < nF; k += Cfg::kThreads) {
-        lds.face[k] = ta.face[offF + k];
+        static_cast<I3 &>(lds.face[k]) = ta.face[offF + k];
         lds.nrm[k] = ta.fnrm[offF + k];
     }
     if (i < nL) {
@@ -1904,7 +2031,7 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
         fix_scheme<SCHEME, NS>(ph);
         const CaseBC &bc = run_args<G>().ta.cbc[0];
         if (i < nFF) {
-            const int4 fr = lds.face[i];
+            const I3 fr = lds.face[i];
             const int L = lfield(fr.y, 0), R = lfield(fr.y, 1);
             const bool has_R = R != fvmr::kLocalNone;
             const V2<G> n = lds.nrm[i];
@@ -1922,10 +2049,10 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
             if (LDT) {
                 dtl = bc.CFL * vol / local_alpha(ph, f0, f1, f2, sAi, sAv, vol);
             } else {
-                const double alpha_c = cell_alpha(ph, gs.w, f0, f1, f2, sAi, sAv, vol, [&](int f, double *av, double *vv) {
+                const double alpha_c = cell_alpha(ph, code, f0, f1, f2, sAi, sAv, vol, [&](int f, double *av, double *vv) {
                     // the periodic pair of face f, seen from this cell (the face's L) and its R (FP64 only:
                     // the mixed LDS states are FP32)
-                    const int4 ff = lds.face[f];
+                    const I3 ff = lds.face[f];
                     const int pf = lfield(ff.y, 2);
                     const V2<G> n = lds.nrm[pf];
                     const double len = (double)__int_as_float(lds.face[pf].z);
@@ -1964,7 +2091,7 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
             opaque(nw);
             opaque(gs.x); opaque(gs.y); opaque(gs.z);
             opaque(gco.x); opaque(gco.y); opaque(gco.z); opaque(gco.w);
-            if (i < nG) tile_gradient(ph, lds, i, gs, gco, nw);
+            if (i < nG) tile_gradient<false>(ph, lds, i, gs, gco, nw);
             __syncthreads();
             C F[4] = {C(0), C(0), C(0), C(0)};
             if (i < nFF) tile_flux<C, G, NS>(ph, bc, sTrk, lds, i, F);
@@ -2575,7 +2702,7 @@ struct fvmr_solver {
     int shape = 0;                        // work-group shape of the tile kernels (TileCfg<., shape>)
     int *t_info = nullptr, *t_halo = nullptr, *t_lnodes = nullptr;
     V2<double> *t_nxy = nullptr;
-    int4 *t_gslot = nullptr, *t_face = nullptr;
+    I3 *t_gslot = nullptr, *t_face = nullptr;
     void *t_gcoef = nullptr;
     void *t_lcxy = nullptr, *t_fnrm = nullptr;   // V2<G> per local cell / per face (FVMR_TILE_GEOM_LOADED)
     DtRec *t_dtrec = nullptr;
@@ -3297,11 +3424,9 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             h->ntiles = tm.ntiles;
             std::vector<V2<double>> txy(tm.nxy.size() / 2);
             for (size_t k = 0; k < txy.size(); k++) txy[k] = V2<double>{tm.nxy[2 * k], tm.nxy[2 * k + 1]};
-            std::vector<int4> tgs(tm.gslot.size() / 4), tfc(tm.face.size() / 4);
-            for (size_t k = 0; k < tgs.size(); k++)
-                tgs[k] = make_int4(tm.gslot[4 * k], tm.gslot[4 * k + 1], tm.gslot[4 * k + 2], tm.gslot[4 * k + 3]);
-            for (size_t k = 0; k < tfc.size(); k++)
-                tfc[k] = make_int4(tm.face[4 * k], tm.face[4 * k + 1], tm.face[4 * k + 2], tm.face[4 * k + 3]);
+            std::vector<I3> tgs(tm.gslot.size() / 3), tfc(tm.face.size() / 3);
+            for (size_t k = 0; k < tgs.size(); k++) tgs[k] = I3{tm.gslot[3 * k], tm.gslot[3 * k + 1], tm.gslot[3 * k + 2]};
+            for (size_t k = 0; k < tfc.size(); k++) tfc[k] = I3{tm.face[3 * k], tm.face[3 * k + 1], tm.face[3 * k + 2]};
             if ((rc = upload(&h->t_info, tm.info, h->stream)) || (rc = upload(&h->t_halo, tm.halo, h->stream)) ||
                 (rc = upload(&h->t_lnodes, tm.lnodes, h->stream)) || (rc = upload(&h->t_nxy, txy, h->stream)) ||
                 (rc = upload(&h->t_gslot, tgs, h->stream)) || (rc = upload(&h->t_face, tfc, h->stream)))

@@ -201,7 +201,7 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
         }
         const int nL = (int)cells.size(), nF = (int)faces.size(), nN = (int)nodes.size();
         const int info[kTileInfo] = {c0, s, nG, nL, nN, nF, nFF,
-                                     (int)out.halo.size(), (int)(out.nxy.size() / 2), (int)(out.face.size() / 4),
+                                     (int)out.halo.size(), (int)(out.nxy.size() / 2), (int)(out.face.size() / 3),
                                      (int)out.lnodes.size(), (int)(out.gcoef.size() / 4), cs};
         out.info.insert(out.info.end(), info, info + kTileInfo);
         for (int i = s; i < nL; i++) out.halo.push_back(cells[i]);
@@ -226,7 +226,6 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
                 out.gslot.push_back(w);
                 gw[j] = gg_weight(in, c, e, o, (x & (1 << 28)) != 0);
             }
-            out.gslot.push_back(i < s ? in.dtcode[c] : 0);
             if (i < s) {
                 int w = 0;
                 for (int j = 0; j < 3; j++) w |= fid[in.cslot_x[(size_t)j * nc + c] & ((1 << 28) - 1)] << (kLocalBits * j);
@@ -247,7 +246,6 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
             out.face.push_back(nid[in.en0[e]] | (nid[in.en1[e]] << kLocalBits) | (bc << kBcShift));
             out.face.push_back(loc(in.eL[e]) | (loc(in.eR[e]) << kLocalBits) | (pl << (2 * kLocalBits)));
             out.face.push_back(lbits);
-            out.face.push_back(e);
             out.fnrm.push_back(in.nx[e]);
             out.fnrm.push_back(in.ny[e]);
         }

@@ -26,8 +26,8 @@ constexpr int kGsOutShift = 10;
 constexpr int kGsIsR = 1 << 20;
 constexpr int kGsPeriodic = 1 << 21;
 
-// Face record (int4): x = node a | node b << 10 | boundary code << 20 (0 interior, else
-// type - 5999); y = L | R << 10 | pair face << 20; z = float bits of the length; w = edge.
+// Face record (3 ints): x = node a | node b << 10 | boundary code << 20 (0 interior, else
+// type - 5999); y = L | R << 10 | pair face << 20; z = float bits of the length.
 constexpr int kBcShift = 20;
 constexpr int kBcBase = 5999;
 
@@ -46,11 +46,11 @@ struct TileMesh {
     std::vector<int> halo;        // device cell id of local cells nT .. nL-1
     std::vector<double> nxy;      // node coordinates, 2 per local node
     std::vector<int> lnodes;      // per local cell: 3 local node ids (10 bits each)
-    std::vector<int> gslot;       // per gradient cell: 3 slot words + dtcode (tile cells)
+    std::vector<int> gslot;       // per gradient cell: 3 slot words
     std::vector<double> gcoef;    // per gradient cell: Green-Gauss weight of slots 0-2, volume
     std::vector<double> lcxy;     // per local cell: centroid x, y (the caller's, as lnodes)
     std::vector<double> fnrm;     // per face: normal x, y (the caller's, as face)
-    std::vector<int> face;        // 4 ints per face
+    std::vector<int> face;        // 3 ints per face
     std::vector<int> dtface;      // per device cell: its 3 slot faces, local ids in its tile
     std::vector<int> case_tile_begin;  // tiles of case c: [c] .. [c+1]-1
     int max_nL = 0, max_nG = 0, max_nF = 0, max_nFF = 0, max_nN = 0;
