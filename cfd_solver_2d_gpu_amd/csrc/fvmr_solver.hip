@@ -3244,6 +3244,35 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
     ph.equation = p->equation; ph.scheme = p->flux_scheme;
     ph.reconstruct = (p->reconstruct == FVMR_REC_LINEAR) ? FVMR_REC_LINEAR : FVMR_REC_CONSTANT;
     ph.gradient = p->gradient; ph.limiter = p->limiter; ph.mu_model = p->viscosity_model; ph.compat_inv = p->compat_inv2x2;
+    // the tile kernels, their work-group shape and the tiles' capacities
+    bool use_tiles = false;
+    fvmr::TileCaps caps{};
+    if (p->kernels != FVMR_KERNELS_CELL) {
+        const char *why = nullptr;
+        use_tiles = fvmr::standard_geometry(m, &why);
+        if (!use_tiles && p->kernels == FVMR_KERNELS_TILE)
+            return bail(set_error(FVMR_ERR_UNSUPPORTED, std::string("tile kernels: ") + why));
+        // a mesh with fewer default tiles than the device has CUs is cut into smaller ones, one per
+        // CU and one CU left for the resident kernel's reducing work-group: its phases then share
+        // a CU's LDS among fewer waves (8,192 cells, 33 instead of 150 per tile: 16.6 instead of
+        // 18.4 us per SSP-RK3 step); fewer than 32 cells leave lanes of the only wave idle
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
+        const int spread = (ncases == 1 && cus > 1) ? std::max(32, (int)(1.1 * nc / (cus - 1)) + 1) : kTileMaxCells;
+        // (grouped tiles are filled to about 0.95 of the most, and the waves they take count, not the cells)
+        const bool grouped = use_tiles && p->renumber == FVMR_RENUMBER_HILBERT;
+        auto caps_of = [&](auto cfg) {
+            using Cfg = decltype(cfg);
+            const int cells = grouped ? Cfg::kCells + Cfg::kCells / 15 : Cfg::kCells;
+            return fvmr::TileCaps{std::min(p->tile_cells ? p->tile_cells : std::min(cells, spread), Cfg::kMaxG),
+                                  Cfg::kMaxG, Cfg::kMaxL, Cfg::kMaxN, Cfg::kMaxF, Cfg::kMaxFF};
+        };
+        h->shape = shape_of_threads(h->mixed, p->tile_threads);
+        if (h->mixed) caps = (h->shape == 1) ? caps_of(TileCfg<float, 1>{}) : caps_of(TileCfg<float, 0>{});
+        else caps = (h->shape == 1) ? caps_of(TileCfg<double, 1>{})
+                                    : ((h->shape == 2) ? caps_of(TileCfg<double, 2>{}) : caps_of(TileCfg<double, 0>{}));
+    }
+    std::vector<int> tile_sizes;   // of the tiles that the Hilbert order is grouped into
     // cell permutation, within each case (case c keeps cells case_begin[c] .. [c+1]-1)
     h->perm.resize(nc);
     for (int cs = 0; cs < ncases; cs++) {
@@ -3251,6 +3280,24 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
         std::vector<int> local;
         if (p->renumber == FVMR_RENUMBER_HILBERT) {
             local = fvmr::hilbert_order(n, m->element_xy[0] + b, m->element_xy[1] + b);
+            if (use_tiles) {
+                std::vector<int> at(n), nbr(3 * (size_t)n), order, sizes;
+                for (int i = 0; i < n; i++) at[local[i]] = i;
+                for (int i = 0; i < n; i++)
+                    for (int j = 0; j < 3; j++) {
+                        const int e = m->element_edges[j][b + local[i]];
+                        const int L = m->edge_elementL[e], R = m->edge_elementR[e];
+                        const int o = (b + local[i] != R) ? R : L;
+                        nbr[3 * (size_t)i + j] = (o >= b && o < b + n) ? at[o - b] : -1;
+                    }
+                // gradients are formed in whole waves: tiles grow until theirs are full
+                fvmr::group_tiles(n, nbr.data(), caps.cells, std::max(8, caps.gcells / 64 * 64), caps.gcells, caps.ffaces,
+                                  order, sizes);
+                std::vector<int> grouped(n);
+                for (int i = 0; i < n; i++) grouped[i] = local[order[i]];
+                local.swap(grouped);
+                tile_sizes.insert(tile_sizes.end(), sizes.begin(), sizes.end());
+            }
         } else if (p->renumber == FVMR_RENUMBER_RCM) {
             std::vector<int> off(n + 1, 0), adj;
             adj.reserve(3 * (size_t)n);
@@ -3379,105 +3426,84 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
     }
     // tile records
     fvmr::TileMesh tm;
-    if (p->kernels != FVMR_KERNELS_CELL) {
-        const char *why = nullptr;
-        if (!fvmr::standard_geometry(m, &why)) {
-            if (p->kernels == FVMR_KERNELS_TILE) return bail(set_error(FVMR_ERR_UNSUPPORTED, std::string("tile kernels: ") + why));
-        } else {
-            std::vector<int> sx(3 * (size_t)nc), sy(3 * (size_t)nc), eL(nf), eR(nf), et(nf), ep(nf), en0(nf), en1(nf);
-            std::vector<double> elen(nf), vol(nc);
-            for (size_t k = 0; k < sx.size(); k++) { sx[k] = cslot[k].x; sy[k] = cslot[k].y; }
-            for (int e = 0; e < nf; e++) {
-                eL[e] = eint[e].x; eR[e] = eint[e].y; et[e] = eint[e].z; ep[e] = eint[e].w;
-                en0[e] = m->edge_nodes[0][eperm[e]]; en1[e] = m->edge_nodes[1][eperm[e]];
-                elen[e] = m->edge_length[eperm[e]];
-            }
-            for (int i = 0; i < nc; i++) vol[i] = m->element_volume[h->perm[i]];
-            std::vector<double> ccx(nc), ccy(nc), emx(nf), emy(nf), enx(nf), eny(nf);
-            for (int i = 0; i < nc; i++) { ccx[i] = m->element_xy[0][h->perm[i]]; ccy[i] = m->element_xy[1][h->perm[i]]; }
-            for (int e = 0; e < nf; e++) {
-                emx[e] = m->edge_xy[0][eperm[e]]; emy[e] = m->edge_xy[1][eperm[e]];
-                enx[e] = m->edge_normal[0][eperm[e]]; eny[e] = m->edge_normal[1][eperm[e]];
-            }
-            fvmr::TileInput ti{nc, nf, sx.data(), sy.data(), cnode.data(), eL.data(), eR.data(), et.data(), ep.data(),
-                               en0.data(), en1.data(), elen.data(), m->node_xy[0], m->node_xy[1], vol.data(), dtcode.data(),
-                               ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin};
-            // a mesh with fewer default tiles than the device has CUs is cut into smaller ones, one per
-            // CU and one CU left for the resident kernel's reducing work-group: its phases then share
-            // a CU's LDS among fewer waves (8,192 cells, 33 instead of 150 per tile: 16.6 instead of
-            // 18.4 us per SSP-RK3 step); fewer than 32 cells leave lanes of the only wave idle
-            int cus = 0;
-            if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
-            const int spread = (ncases == 1 && cus > 1) ? std::max(32, (nc + cus - 2) / (cus - 1)) : kTileMaxCells;
-            auto caps_of = [&](auto cfg) {
-                using Cfg = decltype(cfg);
-                return fvmr::TileCaps{std::min(p->tile_cells ? p->tile_cells : std::min(Cfg::kCells, spread), Cfg::kMaxG),
-                                      Cfg::kMaxG, Cfg::kMaxL, Cfg::kMaxN, Cfg::kMaxF, Cfg::kMaxFF};
-            };
-            h->shape = shape_of_threads(h->mixed, p->tile_threads);
-            fvmr::TileCaps caps;
-            if (h->mixed) caps = (h->shape == 1) ? caps_of(TileCfg<float, 1>{}) : caps_of(TileCfg<float, 0>{});
-            else caps = (h->shape == 1) ? caps_of(TileCfg<double, 1>{})
-                                        : ((h->shape == 2) ? caps_of(TileCfg<double, 2>{}) : caps_of(TileCfg<double, 0>{}));
-            if ((rc = fvmr::build_tiles(ti, caps, tm))) return bail(rc);
-            h->tiles = true;
-            h->ntiles = tm.ntiles;
-            std::vector<V2<double>> txy(tm.nxy.size() / 2);
-            for (size_t k = 0; k < txy.size(); k++) txy[k] = V2<double>{tm.nxy[2 * k], tm.nxy[2 * k + 1]};
-            std::vector<I3> tgs(tm.gslot.size() / 3), tfc(tm.face.size() / 3);
-            for (size_t k = 0; k < tgs.size(); k++) tgs[k] = I3{tm.gslot[3 * k], tm.gslot[3 * k + 1], tm.gslot[3 * k + 2]};
-            for (size_t k = 0; k < tfc.size(); k++) tfc[k] = I3{tm.face[3 * k], tm.face[3 * k + 1], tm.face[3 * k + 2]};
-            if ((rc = upload(&h->t_info, tm.info, h->stream)) || (rc = upload(&h->t_halo, tm.halo, h->stream)) ||
-                (rc = upload(&h->t_lnodes, tm.lnodes, h->stream)) || (rc = upload(&h->t_nxy, txy, h->stream)) ||
-                (rc = upload(&h->t_gslot, tgs, h->stream)) || (rc = upload(&h->t_face, tfc, h->stream)))
-                return bail(rc);
-            std::vector<V4<float>> gcf;
-            std::vector<V4<double>> gcd(tm.gcoef.size() / 4);
+    if (use_tiles) {
+        std::vector<int> sx(3 * (size_t)nc), sy(3 * (size_t)nc), eL(nf), eR(nf), et(nf), ep(nf), en0(nf), en1(nf);
+        std::vector<double> elen(nf), vol(nc);
+        for (size_t k = 0; k < sx.size(); k++) { sx[k] = cslot[k].x; sy[k] = cslot[k].y; }
+        for (int e = 0; e < nf; e++) {
+            eL[e] = eint[e].x; eR[e] = eint[e].y; et[e] = eint[e].z; ep[e] = eint[e].w;
+            en0[e] = m->edge_nodes[0][eperm[e]]; en1[e] = m->edge_nodes[1][eperm[e]];
+            elen[e] = m->edge_length[eperm[e]];
+        }
+        for (int i = 0; i < nc; i++) vol[i] = m->element_volume[h->perm[i]];
+        std::vector<double> ccx(nc), ccy(nc), emx(nf), emy(nf), enx(nf), eny(nf);
+        for (int i = 0; i < nc; i++) { ccx[i] = m->element_xy[0][h->perm[i]]; ccy[i] = m->element_xy[1][h->perm[i]]; }
+        for (int e = 0; e < nf; e++) {
+            emx[e] = m->edge_xy[0][eperm[e]]; emy[e] = m->edge_xy[1][eperm[e]];
+            enx[e] = m->edge_normal[0][eperm[e]]; eny[e] = m->edge_normal[1][eperm[e]];
+        }
+        fvmr::TileInput ti{nc, nf, sx.data(), sy.data(), cnode.data(), eL.data(), eR.data(), et.data(), ep.data(),
+                           en0.data(), en1.data(), elen.data(), m->node_xy[0], m->node_xy[1], vol.data(),
+                           ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin,
+                           tile_sizes.empty() ? nullptr : &tile_sizes};
+        if ((rc = fvmr::build_tiles(ti, caps, tm))) return bail(rc);
+        h->tiles = true;
+        h->ntiles = tm.ntiles;
+        std::vector<V2<double>> txy(tm.nxy.size() / 2);
+        for (size_t k = 0; k < txy.size(); k++) txy[k] = V2<double>{tm.nxy[2 * k], tm.nxy[2 * k + 1]};
+        std::vector<I3> tgs(tm.gslot.size() / 3), tfc(tm.face.size() / 3);
+        for (size_t k = 0; k < tgs.size(); k++) tgs[k] = I3{tm.gslot[3 * k], tm.gslot[3 * k + 1], tm.gslot[3 * k + 2]};
+        for (size_t k = 0; k < tfc.size(); k++) tfc[k] = I3{tm.face[3 * k], tm.face[3 * k + 1], tm.face[3 * k + 2]};
+        if ((rc = upload(&h->t_info, tm.info, h->stream)) || (rc = upload(&h->t_halo, tm.halo, h->stream)) ||
+            (rc = upload(&h->t_lnodes, tm.lnodes, h->stream)) || (rc = upload(&h->t_nxy, txy, h->stream)) ||
+            (rc = upload(&h->t_gslot, tgs, h->stream)) || (rc = upload(&h->t_face, tfc, h->stream)))
+            return bail(rc);
+        std::vector<V4<float>> gcf;
+        std::vector<V4<double>> gcd(tm.gcoef.size() / 4);
+        for (size_t k = 0; k < gcd.size(); k++)
+            gcd[k] = V4<double>{tm.gcoef[4 * k], tm.gcoef[4 * k + 1], tm.gcoef[4 * k + 2], tm.gcoef[4 * k + 3]};
+        if (h->mixed) {
+            gcf.resize(gcd.size());
             for (size_t k = 0; k < gcd.size(); k++)
-                gcd[k] = V4<double>{tm.gcoef[4 * k], tm.gcoef[4 * k + 1], tm.gcoef[4 * k + 2], tm.gcoef[4 * k + 3]};
-            if (h->mixed) {
-                gcf.resize(gcd.size());
-                for (size_t k = 0; k < gcd.size(); k++)
-                    gcf[k] = V4<float>{(float)gcd[k].x, (float)gcd[k].y, (float)gcd[k].z, (float)gcd[k].w};
-                V4<float> *d = nullptr;
-                if ((rc = upload(&d, gcf, h->stream))) return bail(rc);
-                h->t_gcoef = d;
-            } else {
-                V4<double> *d = nullptr;
-                if ((rc = upload(&d, gcd, h->stream))) return bail(rc);
-                h->t_gcoef = d;
-            }
-            if (FVMR_TILE_GEOM_LOADED) {
-                // centroids and normals as the kernels would recompute them (standard geometry:
-                // the caller's values), rounded to the kernels' geometry type
-                auto pack = [&](const std::vector<double> &xy, void **dst) -> int {
-                    if (h->mixed) {
-                        std::vector<V2<float>> v(xy.size() / 2);
-                        for (size_t k = 0; k < v.size(); k++) v[k] = V2<float>{(float)xy[2 * k], (float)xy[2 * k + 1]};
-                        V2<float> *d = nullptr;
-                        int r = upload(&d, v, h->stream);
-                        *dst = d;
-                        if (!r && hipStreamSynchronize(h->stream) != hipSuccess) r = set_error(FVMR_ERR_HIP, "tile upload failed");
-                        return r;
-                    }
-                    std::vector<V2<double>> v(xy.size() / 2);
-                    for (size_t k = 0; k < v.size(); k++) v[k] = V2<double>{xy[2 * k], xy[2 * k + 1]};
-                    V2<double> *d = nullptr;
+                gcf[k] = V4<float>{(float)gcd[k].x, (float)gcd[k].y, (float)gcd[k].z, (float)gcd[k].w};
+            V4<float> *d = nullptr;
+            if ((rc = upload(&d, gcf, h->stream))) return bail(rc);
+            h->t_gcoef = d;
+        } else {
+            V4<double> *d = nullptr;
+            if ((rc = upload(&d, gcd, h->stream))) return bail(rc);
+            h->t_gcoef = d;
+        }
+        if (FVMR_TILE_GEOM_LOADED) {
+            // centroids and normals as the kernels would recompute them (standard geometry:
+            // the caller's values), rounded to the kernels' geometry type
+            auto pack = [&](const std::vector<double> &xy, void **dst) -> int {
+                if (h->mixed) {
+                    std::vector<V2<float>> v(xy.size() / 2);
+                    for (size_t k = 0; k < v.size(); k++) v[k] = V2<float>{(float)xy[2 * k], (float)xy[2 * k + 1]};
+                    V2<float> *d = nullptr;
                     int r = upload(&d, v, h->stream);
                     *dst = d;
                     if (!r && hipStreamSynchronize(h->stream) != hipSuccess) r = set_error(FVMR_ERR_HIP, "tile upload failed");
                     return r;
-                };
-                if ((rc = pack(tm.lcxy, &h->t_lcxy)) || (rc = pack(tm.fnrm, &h->t_fnrm))) return bail(rc);
-            }
-            std::vector<DtRec> dtr(nc);
-            for (int i = 0; i < nc; i++)
-                dtr[i] = DtRec{dtcode[i], tm.dtface[i], h->mixed ? (double)(float)vol[i] : vol[i]};
-            if ((rc = upload(&h->t_dtrec, dtr, h->stream))) return bail(rc);
-            if ((rc = upload(&h->tile_case_begin, tm.case_tile_begin, h->stream))) return bail(rc);
-            // the host vectors of these uploads end with this block
-            if (hipStreamSynchronize(h->stream) != hipSuccess) return bail(set_error(FVMR_ERR_HIP, "tile upload failed"));
+                }
+                std::vector<V2<double>> v(xy.size() / 2);
+                for (size_t k = 0; k < v.size(); k++) v[k] = V2<double>{xy[2 * k], xy[2 * k + 1]};
+                V2<double> *d = nullptr;
+                int r = upload(&d, v, h->stream);
+                *dst = d;
+                if (!r && hipStreamSynchronize(h->stream) != hipSuccess) r = set_error(FVMR_ERR_HIP, "tile upload failed");
+                return r;
+            };
+            if ((rc = pack(tm.lcxy, &h->t_lcxy)) || (rc = pack(tm.fnrm, &h->t_fnrm))) return bail(rc);
         }
+        std::vector<DtRec> dtr(nc);
+        for (int i = 0; i < nc; i++)
+            dtr[i] = DtRec{dtcode[i], tm.dtface[i], h->mixed ? (double)(float)vol[i] : vol[i]};
+        if ((rc = upload(&h->t_dtrec, dtr, h->stream))) return bail(rc);
+        if ((rc = upload(&h->tile_case_begin, tm.case_tile_begin, h->stream))) return bail(rc);
+        // the host vectors of these uploads end with this block
+        if (hipStreamSynchronize(h->stream) != hipSuccess) return bail(set_error(FVMR_ERR_HIP, "tile upload failed"));
     }
     if (ncases > 1 && !h->tiles)
         return bail(set_error(FVMR_ERR_UNSUPPORTED, "a batch needs the tile kernels (standard geometry, kernels != CELL)"));

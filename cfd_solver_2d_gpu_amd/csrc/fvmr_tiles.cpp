@@ -84,6 +84,103 @@ std::vector<int> hilbert_order(int nc, const double *cx, const double *cy) {
     return order_out;
 }
 
+void group_tiles(int n, const int *nbr, int cells, int gcells, int gmost, int ffaces, std::vector<int> &order,
+                 std::vector<int> &sizes) {
+    std::vector<int> tile(n, -1);                    // tile of a cell
+    std::vector<int> seen(n, -1);                    // last tile that has met the cell, as cell or halo
+    std::vector<int> start{0}, member;               // tile t: member[start[t]] .. member[start[t + 1]]
+    member.reserve(n);
+    std::vector<int> seeds, notch, front;            // cells beside finished tiles; growth queues
+    size_t seed_head = 0;
+    int next = 0;
+    const int grow = std::max(1, cells - 1);         // the rest of the room is for cells left alone
+    while ((int)member.size() < n) {
+        const int t = (int)start.size() - 1;
+        // the oldest cell beside a finished tile, so that tiles fill the mesh as a front, else the next free one
+        int seed = -1;
+        while (seed < 0 && seed_head < seeds.size()) {
+            const int c = seeds[seed_head++];
+            if (tile[c] < 0) seed = c;
+        }
+        if (seed < 0) {
+            while (tile[next] >= 0) next++;
+            seed = next;
+        }
+        const size_t first = member.size();
+        int halo = 0, bfaces = 0;                    // first-ring cells, faces with one side in the tile
+        notch.clear();
+        front.clear();
+        size_t front_head = 0;
+        auto add = [&](int c) {
+            tile[c] = t;
+            member.push_back(c);
+            if (seen[c] == t) halo--;
+            seen[c] = t;
+            for (int j = 0; j < 3; j++) {
+                const int o = nbr[3 * (size_t)c + j];
+                if (o < 0 || tile[o] != t) bfaces++;
+                else if (o != c) bfaces--;
+                if (o < 0 || tile[o] == t) continue;
+                const bool again = seen[o] == t;
+                if (!again) {
+                    seen[o] = t;
+                    halo++;
+                }
+                if (tile[o] < 0) (again ? notch : front).push_back(o);   // a second face in the tile: fill it first
+            }
+        };
+        auto full = [&]() {
+            const int s = (int)(member.size() - first);
+            return s >= grow || s + halo + 2 > gcells || (3 * s + bfaces) / 2 + 3 > ffaces;
+        };
+        add(seed);
+        while (!full()) {
+            int c = -1;
+            while (c < 0 && !notch.empty()) {
+                if (tile[notch.back()] < 0) c = notch.back();
+                notch.pop_back();
+            }
+            while (c < 0 && front_head < front.size()) {
+                if (tile[front[front_head]] < 0) c = front[front_head];
+                front_head++;
+            }
+            if (c < 0) break;
+            add(c);
+        }
+        // cells whose neighbours are all in tiles would become tiles of their own
+        for (size_t k = first; k < member.size(); k++)
+            for (int j = 0; j < 3; j++) {
+                const int o = nbr[3 * (size_t)member[k] + j];
+                const int s = (int)(member.size() - first);
+                if (o < 0 || tile[o] >= 0 || s >= cells || s + halo + 2 > gmost || (3 * s + bfaces) / 2 + 3 > ffaces) continue;
+                bool alone = true;
+                for (int q = 0; q < 3; q++) {
+                    const int r = nbr[3 * (size_t)o + q];
+                    alone = alone && (r < 0 || r == o || tile[r] >= 0);
+                }
+                if (alone) add(o);
+            }
+        for (size_t k = first; k < member.size(); k++)
+            for (int j = 0; j < 3; j++) {
+                const int o = nbr[3 * (size_t)member[k] + j];
+                if (o >= 0 && tile[o] < 0) seeds.push_back(o);
+            }
+        std::sort(member.begin() + first, member.end());
+        start.push_back((int)member.size());
+    }
+    // the tiles along the numbering of their middle cells
+    std::vector<std::pair<int, int>> key(start.size() - 1);
+    for (size_t t = 0; t + 1 < start.size(); t++) key[t] = {member[(start[t] + start[t + 1]) / 2], (int)t};
+    std::sort(key.begin(), key.end());
+    order.clear();
+    order.reserve(n);
+    sizes.clear();
+    for (auto &k : key) {
+        order.insert(order.end(), member.begin() + start[k.second], member.begin() + start[k.second + 1]);
+        sizes.push_back(start[k.second + 1] - start[k.second]);
+    }
+}
+
 bool standard_geometry(const fvmr_mesh_soa *m, const char **why) {
     const double *X = m->node_xy[0], *Y = m->node_xy[1];
     for (int c = 0; c < m->num_element; c++) {
@@ -188,6 +285,8 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
 
     out.case_tile_begin.assign(1, 0);
     int cs = 0;
+    size_t want = 0;
+    int want_end = 0;   // end of the wanted tile that c0 is in
     for (int c0 = 0; c0 < nc;) {
         while (cs + 1 < in.ncases && c0 >= in.case_begin[cs + 1]) {
             cs++;
@@ -195,6 +294,10 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
         }
         const int case_end = (cs + 1 < in.ncases) ? in.case_begin[cs + 1] : nc;
         int s = std::min(caps.cells, case_end - c0), nG = 0, nFF = 0;
+        if (in.sizes) {
+            while (want_end <= c0 && want < in.sizes->size()) want_end += (*in.sizes)[want++];
+            if (want_end > c0) s = std::min(s, want_end - c0);
+        }
         while (!try_tile(c0, s, nG, nFF)) {
             if (s == 1) return set_error(FVMR_ERR_UNSUPPORTED, "one cell and its halo exceed the tile capacity");
             s = std::max(1, s - std::max(1, s / 8));

@@ -68,16 +68,29 @@ struct TileInput {
     const double *elen;   // edge length
     const double *node_x, *node_y;
     const double *vol;    // cell volume
-    const int *dtcode;    // per cell
     const double *cx, *cy;  // cell centroids
     const double *mx, *my;  // edge midpoints
     const double *nx, *ny;  // edge normals
     int ncases;             // cases of a batch: device cells case_begin[c] .. [c+1]-1 (tiles never
     const int *case_begin;  // cross a case boundary)
+    const std::vector<int> *sizes;  // cell counts of the tiles wanted, in order (group_tiles; NULL: as many
+                                    // cells as fit); a tile that exceeds a capacity is split
 };
 
 // Cells sorted along a Hilbert curve over their centroids (ties by index).
 std::vector<int> hilbert_order(int nc, const double *cx, const double *cy);
+
+// Groups n cells into compact tiles of at most `cells` cells, about `gcells` (at most `gmost`) cells with
+// the first halo ring and at most `ffaces` faces; nbr: 3 per cell, the cells across its faces (-1 none), in a locality-preserving
+// numbering (Hilbert).  order: the cells tile after tile; sizes: the tiles' cell counts.
+//
+// A run of consecutive cells of the Hilbert curve is compact where the cells are as wide as long; in
+// boundary-layer meshes it is a strip.  Tiles grown over the cells' neighbours are compact in both: on a
+// 1024x512x2 wedge 1.26 cells with a gradient and 1.54 staged cells per tile cell against 1.32 and 1.66,
+// on a 512x512x2 cylinder O-grid (cells up to 260 times longer than wide) 1.26 and 1.55 against 1.66 and
+// 2.34, with 144 instead of 106 cells per tile.
+void group_tiles(int n, const int *nbr, int cells, int gcells, int gmost, int ffaces, std::vector<int> &order,
+                 std::vector<int> &sizes);
 
 // True when the caller's centroids, midpoints, normals and lengths are exactly what the
 // tile kernels recompute from the node coordinates (centroid ((x0+x1)+x2)/3, midpoint

@@ -63,7 +63,8 @@ extern "C" {
 /* Device cell order (results always cross the ABI in the caller's order). */
 #define FVMR_RENUMBER_NONE      0    /* the caller's order */
 #define FVMR_RENUMBER_RCM       1    /* reverse Cuthill-McKee */
-#define FVMR_RENUMBER_HILBERT   2    /* Hilbert curve over the centroids (default) */
+#define FVMR_RENUMBER_HILBERT   2    /* Hilbert curve over the centroids (default); the tile kernels group
+                                        the cells of each tile along it */
 
 /* Device kernel family.  TILE: one work-group per tile of cells, gradients kept in LDS,
  * every face flux evaluated once; it needs the standard geometry (centroids, midpoints,
@@ -149,7 +150,7 @@ typedef struct fvmr_params {
     int    renumber;         /* device cell order: FVMR_RENUMBER_* */
     int    compat_inv2x2;    /* 1: reproduce the reference inv_2x2 determinant bug (LSQ) */
     int    kernels;          /* FVMR_KERNELS_*: device kernel family */
-    int    tile_cells;       /* cells per tile of the tile kernels (0: the work-group shape's default, 150
+    int    tile_cells;       /* cells per tile of the tile kernels (0: the work-group shape's default, about 150
                                 in FP64 and 300 in mixed precision for the default shapes; at most 400,
                                 capped by the shape's LDS) */
     int    tile_threads;     /* work-items per work-group of the tile kernels (0: the default, 256 in FP64
