@@ -1073,12 +1073,11 @@ int steady_stage(fvmr_solver *h, const S4 *Uin, const S4 *Un, S4 *Uout, double a
     if (h->tiles && h->shape == 0) {   // the tile kernel with per-cell dt (the same residual as the cell kernels)
         TileArgs<double> t = tile_args<double>(h);
         t.dtl = w->dtl;
-        if (h->ph.equation == FVMR_EQ_NS)
-            k_tile<double, double, true, true><<<h->ntiles, TileCfg<double>::kThreads, 0, h->stream>>>(
-                t, h->ph, Uin, Un, Uout, rhs, h->sc, h->bad_list, h->nc, a, b, first, 0);
-        else
-            k_tile<double, double, false, true><<<h->ntiles, TileCfg<double>::kThreads, 0, h->stream>>>(
-                t, h->ph, Uin, Un, Uout, rhs, h->sc, h->bad_list, h->nc, a, b, first, 0);
+        const bool ns = h->ph.equation == FVMR_EQ_NS, gg = tile_scheme(h->ph) != kTileAny;
+        auto *kern = ns ? (gg ? k_tile<double, double, true, true, kTileGg> : k_tile<double, double, true, true, kTileAny>)
+                        : (gg ? k_tile<double, double, false, true, kTileGg> : k_tile<double, double, false, true, kTileAny>);
+        kern<<<h->ntiles, TileCfg<double>::kThreads, 0, h->stream>>>(t, h->ph, Uin, Un, Uout, rhs, h->sc, h->bad_list, h->nc, a,
+                                                                      b, first, 0);
         HIP_OK(hipGetLastError());
         return FVMR_OK;
     }

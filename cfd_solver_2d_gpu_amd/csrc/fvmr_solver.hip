@@ -74,13 +74,6 @@ constexpr int kGroup3 = 3 * kCellsPerGroup;     // one wave64 per face slot
 #ifndef FVMR_XCD_REMAP
 #define FVMR_XCD_REMAP 1
 #endif
-// 1: the stage kernel k_tile loads each local cell's centroid and each face's normal (packed
-// per tile on the host, equal bit for bit to what it would recompute) instead of recomputing
-// them from the node coordinates (about 1% faster at 1M cells).  The time-step kernel always
-// recomputes its normals: it is bound by its loads, and loading them cost it 6%.
-#ifndef FVMR_TILE_GEOM_LOADED
-#define FVMR_TILE_GEOM_LOADED 1
-#endif
 #if FVMR_STAGE_WPE > 0
 #define FVMR_STAGE_ATTR __attribute__((amdgpu_waves_per_eu(FVMR_STAGE_WPE)))
 #else
@@ -1166,13 +1159,14 @@ __global__ __launch_bounds__(kGroup3) FVMR_STAGE_ATTR void k_stage(Mesh<G> m, Ph
 // and the first ring in LDS, evaluates the flux of every face of the tile once, and sums
 // the fluxes per cell in slot order.  Gradients never go to HBM.
 // ---------------------------------------------------------------------------
-// Work-group shapes of the tile kernels per arithmetic precision.  The default (S = 0) is sized
-// so that the LDS of a work-group lets as many work-groups share a CU as the registers allow
-// (FP64: about 104 VGPRs -> 4 waves per SIMD -> 4 work-groups of 4 waves with <= 40 KB LDS each;
-// FP32: about 74 VGPRs -> 6 waves per SIMD -> 3 work-groups of 8 waves with <= 53 KB each).
-// S = 1 halves the work-group (smaller tiles, more work-groups per CU), S = 2 doubles it (FP64
-// only: the FP32 shape's local ids would not fit their 10-bit fields).  A handle uses one shape
-// (fvmr_params.tile_threads); the tuners pick among them.
+// Work-group shapes of the tile kernels per arithmetic precision.  The default (S = 0) is sized so that the
+// LDS of a work-group lets as many work-groups share a CU as the registers allow (FP64: about 107 VGPRs -> 4
+// work-groups of 4 waves, 27 KB LDS each in k_tile and 39 KB in k_run; mixed: about 70 VGPRs -> 7 work-groups of
+// 4 waves with 23 KB each).  The others: half and double the work-items in FP64, double in mixed precision
+// (more cells would not fit the 10-bit local ids).  Stage kernel, events, 1,048,576-cell wedge: FP64 128 / 256 /
+// 512 work-items 69.3 / 48.2 / 50.1 us, mixed 256 / 512 work-items 33.4 / 35.2 us; a batch of 32 cases
+// (690,000 cells) mixed 20.8 / 22.3 us.  A handle uses one shape (fvmr_params.tile_threads); the tuners pick
+// among them.
 template <class C, int S = 0> struct TileCfg;
 template <> struct TileCfg<double, 0> {
     static constexpr int kThreads = 256;
@@ -1194,19 +1188,22 @@ template <> struct TileCfg<double, 2> {
     static constexpr int kCells = 300;
 };
 template <> struct TileCfg<float, 0> {
-    static constexpr int kThreads = 512;
-    static constexpr int kMaxG = 400;
-    static constexpr int kMaxL = 480;
-    static constexpr int kMaxN = 320;
-    static constexpr int kMaxF = 672;
-    static constexpr int kMaxFF = kThreads;
-    static constexpr int kCells = 300;
-};
-template <> struct TileCfg<float, 1> {
     static constexpr int kThreads = 256;
-    static constexpr int kMaxG = 200, kMaxL = 240, kMaxN = 160, kMaxF = 336, kMaxFF = kThreads;
+    static constexpr int kMaxG = 200;
+    static constexpr int kMaxL = 256;
+    static constexpr int kMaxN = 160;
+    static constexpr int kMaxF = 336;
+    static constexpr int kMaxFF = kThreads;
     static constexpr int kCells = 150;
 };
+template <> struct TileCfg<float, 1> {
+    static constexpr int kThreads = 512;
+    static constexpr int kMaxG = 400, kMaxL = 480, kMaxN = 320, kMaxF = 672, kMaxFF = kThreads;
+    static constexpr int kCells = 300;
+};
+// The resident kernel's shape: mixed meshes that fit are better served by the larger tiles, which exchange
+// fewer halo cells (131,070 viscous cells, 50 steps: 1.66 ms against 1.87 ms with 256 work-items).
+template <class C> constexpr int kRunShape = std::is_same<C, float>::value ? 1 : 0;
 constexpr int kTileMaxCells = 400;   // largest tile_cells accepted (the largest shapes' kMaxG)
 constexpr int kNumShapes[2] = {3, 2};   // shapes per precision: FP64, FP32-mixed
 template <class Cfg> constexpr bool tile_cfg_fits() {
@@ -1258,8 +1255,8 @@ struct TileArgs {
     const V4<G> *gcoef;       // per gradient cell: Green-Gauss weights of the 3 slots, volume
     const I3 *face;           // per face: nodes | BC code, L | R | pair face, float length
     const DtRec *dtrec;       // per device cell
-    const V2<G> *lcxy;        // per local cell: centroid (FVMR_TILE_GEOM_LOADED)
-    const V2<G> *fnrm;        // per face: normal (FVMR_TILE_GEOM_LOADED)
+    const V2<G> *lcxy;        // per local cell: centroid
+    const V2<G> *fnrm;        // per face: normal
     const CaseBC *cbc;        // per case of the batch (one case: the handle's)
     double *dtl;              // per-cell steps of a steady solve (k_tile_dt / k_tile with LDT), else NULL
 };
@@ -1391,45 +1388,67 @@ struct TileCells {
     __device__ __forceinline__ bool has(int c) const { return c >= 0; }
 };
 
-// Scheme of a k_tile instantiation: read from Phys at run time, or fixed at compile time for
-// the common Green-Gauss + Barth + Roe + linear reconstruction (the compiler then drops the
-// other branches: 116 -> 99 VGPRs and about 3% of the FP64 kernel's time).
-enum TileScheme { kTileAny = 0, kTileGgBarthRoe = 1 };
-inline bool tile_scheme_fixed(const Phys &ph) {
-    return ph.gradient == FVMR_GRA_GREENGAUSS && ph.limiter == FVMR_LIM_BARTH && ph.scheme == FVMR_SOL_ROE &&
-           ph.reconstruct == FVMR_REC_LINEAR;
+// Scheme of a tile kernel's instantiation: read from Phys at run time; Green-Gauss fixed at compile time
+// (centroids then need not be loaded); or all of the common Green-Gauss + Barth + Roe + linear
+// reconstruction (the compiler drops the other branches: 116 -> 99 VGPRs and about 3% of the FP64 kernel's
+// time).
+enum TileScheme { kTileAny = 0, kTileGgBarthRoe = 1, kTileGg = 2 };
+inline int tile_scheme(const Phys &ph) {
+    if (ph.gradient != FVMR_GRA_GREENGAUSS) return kTileAny;
+    return ph.limiter == FVMR_LIM_BARTH && ph.scheme == FVMR_SOL_ROE && ph.reconstruct == FVMR_REC_LINEAR ? kTileGgBarthRoe
+                                                                                                        : kTileGg;
+}
+template <int SCHEME, bool NS>
+__device__ __forceinline__ void fix_scheme(Phys &ph) {
+    if (!NS) ph.equation = FVMR_EQ_EULER;
+    if (SCHEME != kTileAny) ph.gradient = FVMR_GRA_GREENGAUSS;
+    if (SCHEME == kTileGgBarthRoe) {
+        ph.limiter = FVMR_LIM_BARTH;
+        ph.scheme = FVMR_SOL_ROE;
+        ph.reconstruct = FVMR_REC_LINEAR;
+    }
 }
 
 // LDS of a work-group that computes a tile's stages: states (16-byte columns), node coordinates,
-// centroids, face records and normals; the gradients (16-byte columns of kMaxG), which the face
-// fluxes (columns of kMaxFF) replace once every flux is formed.
-template <class C, class G, class Cfg>
-struct TileLds {
+// centroids; the gradients (16-byte columns of kMaxG), which the face fluxes (columns of kMaxFF) replace once
+// every flux is formed.  GEO: the face records and normals too (the mixed gradients read normals, the
+// resident kernel keeps both; the FP64 k_tile forms each face's normal once, in the thread of its flux).
+template <class Cfg, class G, bool GEO>
+struct TileFaces {
+    I3L face[Cfg::kMaxF];
+    V2<G> nrm[Cfg::kMaxF];
+};
+template <class Cfg, class G>
+struct TileFaces<Cfg, G, false> {};
+template <class C, class G, class Cfg, bool GEO>
+struct TileLds : TileFaces<Cfg, G, GEO> {
     using SU = TileState<C>;
     static_assert(Cfg::kMaxL <= Cfg::kThreads && Cfg::kMaxFF <= Cfg::kThreads, "one local cell and one face per thread");
     static_assert(Cfg::kMaxN <= Cfg::kThreads && Cfg::kMaxF <= 2 * Cfg::kThreads, "one node and two faces per thread");
     static_assert(Cfg::kMaxFF * sizeof(V4<C>) <= Cfg::kMaxG * sizeof(Grad<G>), "flux buffer overlays the gradients");
-    char U[Cfg::kMaxL * sizeof(SU)];
+    alignas(16) char U[Cfg::kMaxL * sizeof(SU)];
     V2<double> N[Cfg::kMaxN];
-    I3L face[Cfg::kMaxF];
     char grfl[Cfg::kMaxG * sizeof(Grad<G>)];
     V2<G> cen[Cfg::kMaxL];
-    V2<G> nrm[Cfg::kMaxF];
 };
 
-// -x where the slot word says that the cell is the face's R: the word's bit 20 into the sign bit.
-static_assert(fvmr::kGsIsR == 1 << 20, "the R flag moves to bit 31");
-__device__ __forceinline__ int sign_of_slot(int sw) { return (sw << 11) & (int)0x80000000; }
-__device__ __forceinline__ float negate_if_R(float x, int sw) { return __int_as_float(__float_as_int(x) ^ sign_of_slot(sw)); }
-__device__ __forceinline__ double negate_if_R(double x, int sw) {
-    return __hiloint2double(__double2hiint(x) ^ sign_of_slot(sw), __double2loint(x));
+// -x where bit FLAG of a slot word is set: the bit into the sign.
+template <int FLAG> __device__ __forceinline__ int sign_of(int sw) {
+    static_assert(FLAG > 0 && (FLAG & (FLAG - 1)) == 0, "one bit");
+    return (int)(((unsigned)sw & (unsigned)FLAG) * (0x80000000u / (unsigned)FLAG));
+}
+template <int FLAG> __device__ __forceinline__ float negate_if(float x, int sw) { return __int_as_float(__float_as_int(x) ^ sign_of<FLAG>(sw)); }
+template <int FLAG> __device__ __forceinline__ double negate_if(double x, int sw) {
+    return __hiloint2double(__double2hiint(x) ^ sign_of<FLAG>(sw), __double2loint(x));
 }
 
 // Limited gradient of local cell i (tile or first ring) into LDS.  gs: its slot words, gco: its
 // Green-Gauss weights and volume, nw: its nodes.  CEN: its centroid is formed here, from the nodes that the
 // limiter reads in any case, and put into LDS for the fluxes (only least squares reads a neighbour's here).
-template <bool CEN, class C, class G, class Cfg>
-__device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg> &s, int i, const I3 gs,
+// In FP64 a slot's area vector is the step between its two nodes, (dy, -dx): the product of the normal
+// (dy, -dx) / L and L up to its two roundings.  In mixed precision it is that product of FP32 values.
+template <bool CEN, class C, class G, class Cfg, bool GEO>
+__device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg, GEO> &s, int i, const I3 gs,
                                               const V4<G> gco, int nw) {
     using SU = TileState<C>;
     const int sw[3] = {gs.x, gs.y, gs.z};
@@ -1458,14 +1477,9 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
     int fl[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        const int f = sw[j] & fvmr::kLocalMask;
         const int out = (sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask;
         const bool has_out = out != fvmr::kLocalNone;
         const bool periodic = (sw[j] & fvmr::kGsPeriodic) != 0;
-        const I3 fr = s.face[f];
-        V4<G> eg;
-        V2<G> em;
-        tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
         {
             const SU v = lds_get<SU>(s.U, Cfg::kMaxL, has_out ? out : i);
             sl.u[j][0] = (C)v.x; sl.u[j][1] = (C)v.y; sl.u[j][2] = (C)v.z; sl.u[j][3] = (C)v.w;
@@ -1474,10 +1488,18 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
         sl.n[j][1] = (C)(G)nd[j].y - yc;
         if (ph.gradient == FVMR_GRA_GREENGAUSS) {
             // weight g_C of the slot precomputed by the host (the device formula in FP64)
-            const C len = (C)eg.z;
             sl.a[j][0] = (C)(j == 0 ? gco.x : (j == 1 ? gco.y : gco.z));
-            sl.a[j][1] = negate_if_R((C)eg.x * len, sw[j]);
-            sl.a[j][2] = negate_if_R((C)eg.y * len, sw[j]);
+            if constexpr (std::is_same<C, double>::value) {
+                const V2<double> p = nd[j], q = nd[(j + 1) % 3];
+                sl.a[j][1] = negate_if<fvmr::kGsTurned>(q.y - p.y, sw[j]);
+                sl.a[j][2] = negate_if<fvmr::kGsTurned>(p.x - q.x, sw[j]);
+            } else {
+                const int f = sw[j] & fvmr::kLocalMask;
+                const V2<G> n = s.nrm[f];
+                const C len = (C)(G)(double)__int_as_float(s.face[f].z);
+                sl.a[j][1] = negate_if<fvmr::kGsIsR>((C)n.x * len, sw[j]);
+                sl.a[j][2] = negate_if<fvmr::kGsIsR>((C)n.y * len, sw[j]);
+            }
         } else {
             C dxn = C(0), dyn = C(0);
             if (has_out && !periodic) {   // element neighbours exclude periodic faces
@@ -1501,25 +1523,22 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg>
     lds_put(s.grfl, Cfg::kMaxG, i, g);
 }
 
-// The canonical L -> R flux of face f of the tile from the states and gradients in LDS.
-template <class C, class G, bool NS, class Cfg>
-__device__ __forceinline__ void tile_flux(const Phys &ph, const CaseBC &bc, double t_rk, const TileLds<C, G, Cfg> &s,
-                                          int f, C F[4]) {
+// The canonical L -> R flux of a face of the tile from the states and gradients in LDS.  fr: its record, eg,
+// em: its geometry, pair(f): the midpoint of local face f (the periodic partner).
+template <class C, class G, bool NS, class Cfg, bool GEO, class Pair>
+__device__ __forceinline__ void tile_flux(const Phys &ph, const CaseBC &bc, double t_rk, const TileLds<C, G, Cfg, GEO> &s,
+                                          const I3 fr, const V4<G> eg, const V2<G> em, Pair &&pair, C F[4]) {
     const TileCells<G, TileState<C>> cells{s.U, Cfg::kMaxL, s.cen, s.grfl, Cfg::kMaxG};
-    const I3 fr = s.face[f];
-    V4<G> eg;
-    V2<G> em;
-    tile_face_geom_n<G>(s.N, s.nrm, f, fr, eg, em);
     const int L = lfield(fr.y, 0), R = lfield(fr.y, 1), pl = lfield(fr.y, 2);
     const int bType = tile_btype(fr);
     const bool has_pair = pl != fvmr::kLocalNone;
-    const V2<G> pm = (bType != -1 && has_pair) ? tile_face_mid<G>(s.N, s.face[pl]) : em;
+    const V2<G> pm = (bType != -1 && has_pair) ? pair(pl) : em;
     face_flux<C, G, NS>(cells, ph, bc, t_rk, L, R == fvmr::kLocalNone ? -1 : R, bType, has_pair, eg, em, pm, F);
 }
 
 // r = -(1/V) sum_j s_j F_j of a tile cell, the fluxes of its faces taken from LDS in slot order.
-template <class C, class G, class Cfg>
-__device__ __forceinline__ void tile_rhs(const TileLds<C, G, Cfg> &s, const I3 gs, const V4<G> gco, double r[4]) {
+template <class C, class G, class Cfg, bool GEO>
+__device__ __forceinline__ void tile_rhs(const TileLds<C, G, Cfg, GEO> &s, const I3 gs, const V4<G> gco, double r[4]) {
     const int sw[3] = {gs.x, gs.y, gs.z};
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -1568,16 +1587,13 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
                                                         S4 *__restrict__ rhs_out, Scalars *__restrict__ sc,
                                                         int *__restrict__ bad_list, int nc, double a, double b,
                                                         int first, int last) {
-    if (SCHEME == kTileGgBarthRoe) {
-        ph.gradient = FVMR_GRA_GREENGAUSS;
-        ph.limiter = FVMR_LIM_BARTH;
-        ph.scheme = FVMR_SOL_ROE;
-        ph.reconstruct = FVMR_REC_LINEAR;
-    }
+    fix_scheme<SCHEME, NS>(ph);
     using Cfg = TileCfg<C, SHAPE>;
     constexpr int kTileThreads = Cfg::kThreads;
+    constexpr bool kGeo = !std::is_same<C, double>::value;
+    constexpr bool kOwnCen = SCHEME != kTileAny;
     using SU = TileState<C>;
-    __shared__ __align__(16) TileLds<C, G, Cfg> lds;
+    __shared__ TileLds<C, G, Cfg, kGeo> lds;
     const int tid = threadIdx.x;
     const int *ti = ta.info + (size_t)xcd_block() * fvmr::kTileInfo;
     const int c0 = ti[fvmr::kTiC0], nT = ti[fvmr::kTiNT], nG = ti[fvmr::kTiNG], nL = ti[fvmr::kTiNL];
@@ -1588,8 +1604,7 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     // thread i owns local cell i (phases 2, 3, 5) and face i (phase 4); its records are
     // fetched with the staging loads
     const int i = tid;
-    constexpr bool kOwnCen = SCHEME == kTileGgBarthRoe && FVMR_TILE_GEOM_LOADED;
-    const int nw = (i < (kOwnCen ? nG : nL)) ? ta.lnodes[offL + i] : 0;
+    const int nw = (i < nG) ? ta.lnodes[offL + i] : 0;
     const I3 gs = (i < nG) ? ta.gslot[offG + i] : I3{0, 0, 0};
     const V4<G> gco = (i < nG) ? ta.gcoef[offG + i] : V4<G>{G(0.5), G(0.5), G(0.5), G(1)};
     // 1. stage nodes, states and face records: every global load is issued before the first
@@ -1597,51 +1612,50 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : -1;
     const S4 uin = (src >= 0) ? Uin[src] : S4{0.0, 0.0, 0.0, 0.0};
     const V2<double> nd = (tid < nN) ? ta.nxy[offN + tid] : V2<double>{0.0, 0.0};
-    const I3 fr0 = (tid < nF) ? ta.face[offF + tid] : I3{0, 0, 0};
-    const I3 fr1 = (tid + kTileThreads < nF) ? ta.face[offF + tid + kTileThreads] : I3{0, 0, 0};
+    const I3 fr0 = (tid < (kGeo ? nF : nFF)) ? ta.face[offF + tid] : I3{0, 0, 0};
+    I3 fr1{0, 0, 0};
+    V2<G> nr0{G(0), G(0)}, nr1{G(0), G(0)};
+    if constexpr (kGeo) {
+        fr1 = (tid + kTileThreads < nF) ? ta.face[offF + tid + kTileThreads] : I3{0, 0, 0};
+        nr0 = (tid < nF) ? ta.fnrm[offF + tid] : V2<G>{G(0), G(0)};
+        nr1 = (tid + kTileThreads < nF) ? ta.fnrm[offF + tid + kTileThreads] : V2<G>{G(0), G(0)};
+    }
     const S4 un = (!first && i < nT) ? Un[c0 + i] : S4{0.0, 0.0, 0.0, 0.0};
-#if FVMR_TILE_GEOM_LOADED
     const V2<G> cc = (!kOwnCen && i < nL) ? ta.lcxy[offL + i] : V2<G>{G(0), G(0)};
-    const V2<G> nr0 = (tid < nF) ? ta.fnrm[offF + tid] : V2<G>{G(0), G(0)};
-    const V2<G> nr1 = (tid + kTileThreads < nF) ? ta.fnrm[offF + tid + kTileThreads] : V2<G>{G(0), G(0)};
-#endif
     if (tid < nN) lds.N[tid] = nd;
-    if (tid < nF) static_cast<I3 &>(lds.face[tid]) = fr0;
-    if (tid + kTileThreads < nF) static_cast<I3 &>(lds.face[tid + kTileThreads]) = fr1;
     if (i < nL) lds_put(lds.U, Cfg::kMaxL, i, SU{(C)uin.x, (C)uin.y, (C)uin.z, (C)uin.w});
-#if FVMR_TILE_GEOM_LOADED
+    if constexpr (kGeo) {
+        if (tid < nF) static_cast<I3 &>(lds.face[tid]) = fr0;
+        if (tid + kTileThreads < nF) static_cast<I3 &>(lds.face[tid + kTileThreads]) = fr1;
+        if (tid < nF) lds.nrm[tid] = nr0;
+        if (tid + kTileThreads < nF) lds.nrm[tid + kTileThreads] = nr1;
+    }
     if (!kOwnCen && i < nL) lds.cen[i] = cc;
-    if (tid < nF) lds.nrm[tid] = nr0;
-    if (tid + kTileThreads < nF) lds.nrm[tid + kTileThreads] = nr1;
     __syncthreads();
-#else
-    __syncthreads();
-    // 2. centroids and face normals
-    if (i < nL) {
-        const V2<double> ct = tile_centroid(lds.N[lfield(nw, 0)], lds.N[lfield(nw, 1)], lds.N[lfield(nw, 2)]);
-        lds.cen[i] = V2<G>{(G)ct.x, (G)ct.y};
-    }
-    for (int k = tid; k < nF; k += kTileThreads) {
-        V4<G> eg;
-        V2<G> em;
-        tile_face_geom<G>(lds.N, lds.face[k], eg, em);
-        lds.nrm[k] = V2<G>{eg.x, eg.y};
-    }
-    __syncthreads();
-#endif
-    // 3. limited gradients of the tile and the first ring
+    // 2. limited gradients of the tile and the first ring
     if (i < nG) tile_gradient<kOwnCen>(ph, lds, i, gs, gco, nw);
     __syncthreads();
-    // 4. one canonical flux per face of the tile (nFF <= threads), written over the gradients
+    // 3. one canonical flux per face of the tile (nFF <= threads), written over the gradients
     const double t_rk = sc[cs].t_rk;
     const CaseBC &bc = ta.cbc[cs];
     C F[4] = {C(0), C(0), C(0), C(0)};
     const int f = tid;
-    if (f < nFF) tile_flux<C, G, NS>(ph, bc, t_rk, lds, f, F);
+    if (f < nFF) {
+        V4<G> eg;
+        V2<G> em;
+        if constexpr (kGeo) {
+            const I3 fr = lds.face[f];
+            tile_face_geom_n<G>(lds.N, lds.nrm, f, fr, eg, em);
+            tile_flux<C, G, NS>(ph, bc, t_rk, lds, fr, eg, em, [&](int pl) { return tile_face_mid<G>(lds.N, lds.face[pl]); }, F);
+        } else {
+            tile_face_geom<G>(lds.N, fr0, eg, em);
+            tile_flux<C, G, NS>(ph, bc, t_rk, lds, fr0, eg, em, [&](int pl) { return tile_face_mid<G>(lds.N, ta.face[offF + pl]); }, F);
+        }
+    }
     __syncthreads();
     if (f < nFF) lds_put(lds.grfl, Cfg::kMaxFF, f, V4<C>{F[0], F[1], F[2], F[3]});
     __syncthreads();
-    // 5. cell-owned sum in slot order, /(-V), RK update (as k_stage); LDT: the cell's own dt
+    // 4. cell-owned sum in slot order, /(-V), RK update (as k_stage); LDT: the cell's own dt
     double dt = sc[cs].dt;
     if (i < nT) {
         const int c = c0 + i;
@@ -1893,17 +1907,6 @@ __device__ __forceinline__ void opaque(int &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void opaque(float &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void opaque(double &x) { asm volatile("" : "+v"(x)); }
 
-template <int SCHEME, bool NS>
-__device__ __forceinline__ void fix_scheme(Phys &ph) {
-    if (!NS) ph.equation = FVMR_EQ_EULER;
-    if (SCHEME == kTileGgBarthRoe) {
-        ph.gradient = FVMR_GRA_GREENGAUSS;
-        ph.limiter = FVMR_LIM_BARTH;
-        ph.scheme = FVMR_SOL_ROE;
-        ph.reconstruct = FVMR_REC_LINEAR;
-    }
-}
-
 __device__ __forceinline__ unsigned long long ll_load(const unsigned long long *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1972,8 +1975,8 @@ __device__ __forceinline__ void run_reduce(const RunArgs &ra) {
 // per-cell steps and no restriction (no reducing work-group).  The arithmetic is that of k_tile_dt
 // and k_tile.
 template <class C, class G, bool NS, bool LDT, int SCHEME, int WAVES>
-__global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKernArg<G> arg) {
-    using Cfg = TileCfg<C, 0>;
+__global__ __launch_bounds__((TileCfg<C, kRunShape<C>>::kThreads), WAVES) void k_run(RunKernArg<G> arg) {
+    using Cfg = TileCfg<C, kRunShape<C>>;
     using SU = TileState<C>;
     constexpr bool kF64 = std::is_same<SU, S4>::value;
     if (!LDT && (int)blockIdx.x == arg.ra.ntiles) {
@@ -1984,7 +1987,7 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
     const RunArgs &ra = arg.ra;
     Scalars *const sc = arg.sc;
     const int nc = arg.nc;
-    __shared__ __align__(16) TileLds<C, G, Cfg> lds;
+    __shared__ TileLds<C, G, Cfg, true> lds;
     __shared__ double sMin[Cfg::kThreads / 64];
     __shared__ double sT, sTrk, sDt;   // t, t at the start of the step, dt
     __shared__ int sStop, sFail, sBad;   // the published flag; a wait of this work-group gave up; a cell to restrict
@@ -2094,7 +2097,13 @@ __global__ __launch_bounds__((TileCfg<C, 0>::kThreads), WAVES) void k_run(RunKer
             if (i < nG) tile_gradient<false>(ph, lds, i, gs, gco, nw);
             __syncthreads();
             C F[4] = {C(0), C(0), C(0), C(0)};
-            if (i < nFF) tile_flux<C, G, NS>(ph, bc, sTrk, lds, i, F);
+            if (i < nFF) {
+                const I3 fr = lds.face[i];
+                V4<G> eg;
+                V2<G> em;
+                tile_face_geom_n<G>(lds.N, lds.nrm, i, fr, eg, em);
+                tile_flux<C, G, NS>(ph, bc, sTrk, lds, fr, eg, em, [&](int pl) { return tile_face_mid<G>(lds.N, lds.face[pl]); }, F);
+            }
             __syncthreads();
             if (i < nFF) lds_put(lds.grfl, Cfg::kMaxFF, i, V4<C>{F[0], F[1], F[2], F[3]});
             if (!LDT && stage == 0 && i == 0) {
@@ -2704,7 +2713,7 @@ struct fvmr_solver {
     V2<double> *t_nxy = nullptr;
     I3 *t_gslot = nullptr, *t_face = nullptr;
     void *t_gcoef = nullptr;
-    void *t_lcxy = nullptr, *t_fnrm = nullptr;   // V2<G> per local cell / per face (FVMR_TILE_GEOM_LOADED)
+    void *t_lcxy = nullptr, *t_fnrm = nullptr;   // V2<G> per local cell / per face
     DtRec *t_dtrec = nullptr;
     // resident kernel (k_run): exchange buffers, allocated by fvmr_create when the handle can use it
     const void *run_step_kernel = nullptr, *run_steady_kernel = nullptr;   // NULL: not on this handle
@@ -2880,11 +2889,16 @@ int launch_tile_stage(fvmr_solver *h, const S4 *Uin, const S4 *Un, S4 *Uout, dou
     hipEvent_t e0{};
     int rc = prof_begin(h, 0, &e0);
     if (rc) return rc;
-    const bool ns = h->ph.equation == FVMR_EQ_NS, fixed = tile_scheme_fixed(h->ph);
+    const bool ns = h->ph.equation == FVMR_EQ_NS;
+    const int scheme = tile_scheme(h->ph);
     with_shape<C>(h, [&](auto sh) {
         constexpr int S = decltype(sh)::value;
-        auto *kern = ns ? (fixed ? k_tile<C, G, true, false, kTileGgBarthRoe, S> : k_tile<C, G, true, false, kTileAny, S>)
-                        : (fixed ? k_tile<C, G, false, false, kTileGgBarthRoe, S> : k_tile<C, G, false, false, kTileAny, S>);
+        auto *kern = ns ? (scheme == kTileGgBarthRoe ? k_tile<C, G, true, false, kTileGgBarthRoe, S>
+                           : scheme == kTileGg       ? k_tile<C, G, true, false, kTileGg, S>
+                                                     : k_tile<C, G, true, false, kTileAny, S>)
+                        : (scheme == kTileGgBarthRoe ? k_tile<C, G, false, false, kTileGgBarthRoe, S>
+                           : scheme == kTileGg       ? k_tile<C, G, false, false, kTileGg, S>
+                                                     : k_tile<C, G, false, false, kTileAny, S>);
         kern<<<h->ntiles, TileCfg<C, S>::kThreads, 0, h->stream>>>(tile_args<G>(h), h->ph, Uin, Un, Uout, rhs_out, h->sc,
                                                                    h->bad_list, h->nc, a, b, first, last);
         return FVMR_OK;
@@ -2945,7 +2959,7 @@ int run_step(fvmr_solver *h, bool store_rhs) {
 // spills a few registers.
 template <class C, class G, int W>
 const void *run_kernel_w(const fvmr_solver *h, bool steady) {
-    const bool ns = h->ph.equation == FVMR_EQ_NS, fixed = tile_scheme_fixed(h->ph);
+    const bool ns = h->ph.equation == FVMR_EQ_NS, fixed = tile_scheme(h->ph) == kTileGgBarthRoe;
     if constexpr (std::is_same<C, double>::value) {
         if (steady) return ns ? (const void *)k_run<C, G, true, true, kTileAny, W> : (const void *)k_run<C, G, false, true, kTileAny, W>;
     }
@@ -2976,7 +2990,7 @@ int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
                    rhs_step, {0.0, 0.75, 1.0 / 3.0}, {1.0, 0.25, 2.0 / 3.0}};
     void *args[] = {&k};
     HIP_OK(hipLaunchCooperativeKernel(steady ? h->run_steady_kernel : h->run_step_kernel, dim3(h->ntiles + (steady ? 0 : 1)),
-                                      dim3(TileCfg<C, 0>::kThreads), args, 0, h->stream));
+                                      dim3(TileCfg<C, kRunShape<C>>::kThreads), args, 0, h->stream));
     h->run_ex += (unsigned)(nsteps * stages);
     if (!steady) h->run_dt += (unsigned)nsteps;
     h->cur = b;
@@ -3062,12 +3076,13 @@ int read_scalars(fvmr_solver *h, Scalars &s) {
 // work-groups on the device at once, tiles that need each other's cells mutually; not mixed precision
 // with periodic faces, whose time step takes FP64 states across a face), and its buffers.
 int run_setup(fvmr_solver *h, const std::vector<int2> &cslot, const std::vector<int> &halo) {
-    if (!h->tiles || h->ncases != 1 || h->shape != 0 || (h->mixed && h->ph.has_periodic)) return FVMR_OK;
+    const int shape = h->mixed ? kRunShape<float> : kRunShape<double>;
+    if (!h->tiles || h->ncases != 1 || h->shape != shape || (h->mixed && h->ph.has_periodic)) return FVMR_OK;
     int coop = 0, cus = 0;
     HIP_OK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, h->device));
     HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
     if (!coop) return FVMR_OK;
-    const int threads = shape_threads(h->mixed, 0);
+    const int threads = shape_threads(h->mixed, shape);
     auto pick = [&](bool steady, int groups) -> const void * {
         for (bool wide : {true, false}) {
             const void *kern = run_kernel(h, steady, wide);
@@ -3268,6 +3283,12 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
                                   Cfg::kMaxG, Cfg::kMaxL, Cfg::kMaxN, Cfg::kMaxF, Cfg::kMaxFF};
         };
         h->shape = shape_of_threads(h->mixed, p->tile_threads);
+        // the default in mixed precision: the resident kernel's shape for the meshes that it can serve (three
+        // work-groups per CU), else the one that is faster in launched kernels
+        if (h->mixed && !p->tile_threads && ncases == 1 &&
+            std::none_of(m->edge_periodicPair, m->edge_periodicPair + nf, [](int e) { return e >= 0; }) &&
+            nc <= 3 * cus * (TileCfg<float, kRunShape<float>>::kCells - 20))
+            h->shape = kRunShape<float>;
         if (h->mixed) caps = (h->shape == 1) ? caps_of(TileCfg<float, 1>{}) : caps_of(TileCfg<float, 0>{});
         else caps = (h->shape == 1) ? caps_of(TileCfg<double, 1>{})
                                     : ((h->shape == 2) ? caps_of(TileCfg<double, 2>{}) : caps_of(TileCfg<double, 0>{}));
@@ -3474,7 +3495,7 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             if ((rc = upload(&d, gcd, h->stream))) return bail(rc);
             h->t_gcoef = d;
         }
-        if (FVMR_TILE_GEOM_LOADED) {
+        {
             // centroids and normals as the kernels would recompute them (standard geometry:
             // the caller's values), rounded to the kernels' geometry type
             auto pack = [&](const std::vector<double> &xy, void **dst) -> int {

@@ -61,6 +61,32 @@ double gg_weight(const TileInput &in, int c, int e, int o, bool periodic) {
     return dFf / dFC;
 }
 
+// The nodes of cell c in the order of its slots: slot j joins v[j] and v[j + 1].  turned[j]: the edge's normal
+// times the cell's sign (out of the cell) is (-dy, dx), not (dy, -dx), of the step v[j] -> v[j + 1].  False
+// when the three edges do not join the cell's three nodes.
+bool slot_nodes(const TileInput &in, int c, int v[3], int turned[3]) {
+    int a[3], b[3];
+    for (int j = 0; j < 3; j++) {
+        const int x = in.cslot_x[(size_t)j * in.nc + c], e = x & ((1 << 28) - 1);
+        a[j] = in.en0[e];
+        b[j] = in.en1[e];
+        if (x & (1 << 30)) std::swap(a[j], b[j]);   // the cell is R: seen from it the edge runs the other way
+    }
+    v[1] = (b[0] == a[1] || b[0] == b[1]) ? b[0] : a[0];
+    v[0] = (v[1] == b[0]) ? a[0] : b[0];
+    v[2] = (a[1] == v[1]) ? b[1] : a[1];
+    for (int j = 0; j < 3; j++) {
+        const int p = v[j], q = v[(j + 1) % 3];
+        if (a[j] == p && b[j] == q) turned[j] = 0;
+        else if (a[j] == q && b[j] == p) turned[j] = 1;
+        else return false;
+        bool mine = false;
+        for (int k = 0; k < 3; k++) mine = mine || in.cnode[(size_t)k * in.nc + c] == p;
+        if (!mine) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 std::vector<int> hilbert_order(int nc, const double *cx, const double *cy) {
@@ -232,7 +258,7 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
     for (int c = 0; c < 3 * nc; c++) nv = std::max(nv, in.cnode[c] + 1);
     for (int e = 0; e < nf; e++) nv = std::max(nv, std::max(in.en0[e], in.en1[e]) + 1);
     std::vector<int> nst(nv, -1), nid(nv, 0);
-    std::vector<int> cells, faces, nodes;
+    std::vector<int> cells, faces, nodes, gturn;
     int stamp = 0;
 
     // Builds the sets of the candidate tile [c0, c0+s); false when a capacity is exceeded.
@@ -308,14 +334,19 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
                                      (int)out.lnodes.size(), (int)(out.gcoef.size() / 4), cs};
         out.info.insert(out.info.end(), info, info + kTileInfo);
         for (int i = s; i < nL; i++) out.halo.push_back(cells[i]);
+        gturn.clear();
         for (int v : nodes) { out.nxy.push_back(in.node_x[v]); out.nxy.push_back(in.node_y[v]); }
         for (int i = 0; i < nL; i++) {
             const int c = cells[i];
             out.lcxy.push_back(in.cx[c]);
             out.lcxy.push_back(in.cy[c]);
+            int v[3], turned[3];
+            if (!slot_nodes(in, c, v, turned))
+                return set_error(FVMR_ERR_UNSUPPORTED, "an element's edges do not join its nodes");
             int w = 0;
-            for (int j = 0; j < 3; j++) w |= nid[in.cnode[(size_t)j * nc + c]] << (kLocalBits * j);
+            for (int j = 0; j < 3; j++) w |= nid[v[j]] << (kLocalBits * j);
             out.lnodes.push_back(w);
+            for (int j = 0; j < 3 && i < nG; j++) gturn.push_back(turned[j]);
         }
         for (int i = 0; i < nG; i++) {
             const int c = cells[i];
@@ -326,6 +357,7 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
                 int w = fid[e] | ((o >= 0 ? lid[o] : kLocalNone) << kGsOutShift);
                 if (x & (1 << 30)) w |= kGsIsR;
                 if (x & (1 << 28)) w |= kGsPeriodic;
+                if (gturn[3 * (size_t)i + j]) w |= kGsTurned;
                 out.gslot.push_back(w);
                 gw[j] = gg_weight(in, c, e, o, (x & (1 << 28)) != 0);
             }

@@ -21,10 +21,12 @@ enum TileInfoField { kTiC0, kTiNT, kTiNG, kTiNL, kTiNN, kTiNF, kTiNFF, kTiOffH, 
                      kTiCase, kTileInfo };
 
 // Gradient-cell slot word: local face (10 bits) | local cell across (10) | cell is the
-// face's R (bit 20) | periodic face (bit 21).
+// face's R (bit 20) | periodic face (bit 21) | the face's normal out of the cell is (-dy, dx) and not
+// (dy, -dx) of the step from local node j to node j + 1 of lnodes (bit 22).
 constexpr int kGsOutShift = 10;
 constexpr int kGsIsR = 1 << 20;
 constexpr int kGsPeriodic = 1 << 21;
+constexpr int kGsTurned = 1 << 22;
 
 // Face record (3 ints): x = node a | node b << 10 | boundary code << 20 (0 interior, else
 // type - 5999); y = L | R << 10 | pair face << 20; z = float bits of the length.
@@ -45,7 +47,7 @@ struct TileMesh {
     std::vector<int> info;        // kTileInfo per tile
     std::vector<int> halo;        // device cell id of local cells nT .. nL-1
     std::vector<double> nxy;      // node coordinates, 2 per local node
-    std::vector<int> lnodes;      // per local cell: 3 local node ids (10 bits each)
+    std::vector<int> lnodes;      // per local cell: 3 local node ids (10 bits each); slot j joins nodes j, j + 1
     std::vector<int> gslot;       // per gradient cell: 3 slot words
     std::vector<double> gcoef;    // per gradient cell: Green-Gauss weight of slots 0-2, volume
     std::vector<double> lcxy;     // per local cell: centroid x, y (the caller's, as lnodes)

@@ -150,11 +150,12 @@ typedef struct fvmr_params {
     int    renumber;         /* device cell order: FVMR_RENUMBER_* */
     int    compat_inv2x2;    /* 1: reproduce the reference inv_2x2 determinant bug (LSQ) */
     int    kernels;          /* FVMR_KERNELS_*: device kernel family */
-    int    tile_cells;       /* cells per tile of the tile kernels (0: the work-group shape's default, about 150
-                                in FP64 and 300 in mixed precision for the default shapes; at most 400,
-                                capped by the shape's LDS) */
-    int    tile_threads;     /* work-items per work-group of the tile kernels (0: the default, 256 in FP64
-                                and 512 in mixed precision; 128 or 512 in FP64, 256 in mixed precision) */
+    int    tile_cells;       /* cells per tile of the tile kernels (0: the work-group shape's default, about 72,
+                                150 and 300 for 128, 256 and 512 work-items, fewer on meshes of less than
+                                one such tile per compute unit; at most 400, capped by the shape's LDS) */
+    int    tile_threads;     /* work-items per work-group of the tile kernels (0: the default, 256 in FP64,
+                                512 or 256 by the mesh's size in mixed precision; 128, 256 or 512 in FP64,
+                                256 or 512 in mixed precision) */
     int    reserved;         /* 0 */
     double inf_ruvp[4];      /* boundaryCondition.2D.inf    (rho,u,v,p) */
     double inlet_ruvp[4];    /* boundaryCondition.2D.inlet  */
