@@ -17,13 +17,11 @@
 // the face physics (primitives, ghost state, Riemann flux, written out by hand) contracted with
 // mu_e gives the adjoints of the face's two reconstructed states.  Per cell (k_adj_vjp):
 // reconstruction passes its three face-state adjoints to U_c and to c's limited gradient; the
-// limited gradient's derivatives in U_c and in the three states across (forward mode: the
-// solver's grad_limit on Dual<4>, one conserved variable at a time, the branch taken by the
-// values) send that on to U_c and to the neighbours: the share of neighbour n goes to a
-// per-(edge, side) slot, which n's gather (k_adj_update) adds in slot order, so the product is
-// deterministic.  The limited gradients of U* (a primal quantity) are formed once per solve;
-// the derivatives of flux, gradient and limiter are recomputed in every product, and no
-// Jacobian is stored.
+// reverse mode of the limited gradient (grad_limit_adj, the branch taken by the values) sends that on
+// to U_c and to the neighbours: the share of neighbour n goes to a per-(edge, side) slot, which n's
+// gather (k_adj_update) adds in slot order, so the product is deterministic.  The limited gradients
+// of U* (a primal quantity) are formed once per solve; the derivatives of flux, gradient and limiter are
+// recomputed in every product, and no Jacobian is stored.
 //
 // Scope: FP64 handles of one case, Euler, no periodic faces and no double Mach reflection
 // boundary (a time-dependent state).  dJ/dX assumes the standard geometry relations (centroid =
@@ -535,32 +533,146 @@ __global__ __launch_bounds__(kBlock) void k_adj_faces(Mesh<double> m, Phys ph, c
     if (interior) st(fadj, 2 * e + 1, URb);
 }
 
-// Gradient slots of grad_limit for one conserved variable with its four derivative directions
-// (0 = the cell's own state, 1 + i = the state across slot i).
-struct SlotsU1 {
-    double a[3][3];
-    Dual<4> uo[3];
-    double n[3][2];
-    __device__ __forceinline__ double A(int i, int q) const { return a[i][q]; }
-    __device__ __forceinline__ Dual<4> Uo(int i, int) const { return uo[i]; }
-    __device__ __forceinline__ double N(int i, int q) const { return n[i][q]; }
-};
+// Reverse mode of grad_limit in the states: the cotangents (gbx, gby) of a cell's limited gradient give
+// those of the cell's own state (self) and of the states across its slots (w).  a, n, fl, vol: the slots as
+// grad_limit takes them; the branch (extremes of bounds and vertices, the limiting vertex) is the one that
+// the values take.  Forward mode (four directions per variable) held k_adj_vjp at 256 VGPRs with spills:
+// 59 us for 393,216 cells of an airfoil O-grid, 45 us with this.
+__device__ __forceinline__ void grad_limit_adj(const Phys &ph, const double Uc[4], const double Uo[3][4],
+                                               const double a[3][3], const double n[3][2], const int fl[3], double vol,
+                                               const double gbx[4], const double gby[4], double self[4], double w[3][4]) {
+    // the unlimited gradient is sum_i (cx_i, cy_i) X_i with X_i = wc_i Uc + wo_i Uo_i
+    double cx[3], cy[3], wc[3], wo[3];
+    if (ph.gradient == FVMR_GRA_GREENGAUSS) {
+        const double inv_vol = frcp(vol);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            cx[i] = inv_vol * a[i][1];
+            cy[i] = inv_vol * a[i][2];
+            wc[i] = (fl[i] & 1) ? a[i][0] : 1.0;
+            wo[i] = (fl[i] & 1) ? 1.0 - a[i][0] : 0.0;
+        }
+    } else {
+        double M[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (fl[i] & 2) {
+                M[0] += a[i][0] * a[i][0];
+                M[1] += a[i][0] * a[i][1];
+                M[2] += a[i][1] * a[i][1];
+            }
+        double det = M[0] * M[2] - M[1] * M[1];
+        const double eps = fvmr::kEPS;
+        if (ph.compat_inv) {   // MatrixKernel.h:48-49 as written
+            if (det >= 0.0 && det < eps) det = eps;
+            else if (det > -eps) det = -eps;
+        } else {
+            if (det >= 0.0 && det < eps) det = eps;
+            else if (det < 0.0 && det > -eps) det = -eps;
+        }
+        const double idet = frcp(det);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const bool in = (fl[i] & 2) != 0;
+            cx[i] = in ? (M[2] * a[i][0] - M[1] * a[i][1]) * idet : 0.0;
+            cy[i] = in ? (M[0] * a[i][1] - M[1] * a[i][0]) * idet : 0.0;
+            wc[i] = -1.0;
+            wo[i] = 1.0;
+        }
+    }
+    double eps2 = 0.0;
+    if (ph.limiter == FVMR_LIM_VENKATAKRISHNAN) {
+        const double Kh = ph.venkat_K * fsqrt(vol);
+        eps2 = Kh * Kh * Kh;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        double gxb = gbx[k], gyb = gby[k], sb = 0.0, ob[3] = {0.0, 0.0, 0.0};
+        if (ph.limiter != FVMR_LIM_NONE) {
+            double gx = 0.0, gy = 0.0, hi = Uc[k], lo = Uc[k];
+            int ih = -1, il = -1;   // the cell that a bound comes from (-1: the cell itself)
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const double X = wc[i] * Uc[k] + wo[i] * Uo[i][k];
+                gx += cx[i] * X;
+                gy += cy[i] * X;
+                if (fl[i] & 2) {
+                    if (hi < Uo[i][k]) { hi = Uo[i][k]; ih = i; }
+                    if (lo > Uo[i][k]) { lo = Uo[i][k]; il = i; }
+                }
+            }
+            const double hrel = hi - Uc[k], lrel = lo - Uc[k];
+            double phi = 1.0, hb = 0.0, lb = 0.0, dxb = 0.0, dyb = 0.0;   // d phi / d (hrel, lrel, gx, gy)
+            if (ph.limiter == FVMR_LIM_BARTH) {
+                double mp = 0.0, mn = 0.0, px = 0.0, py = 0.0, qx = 0.0, qy = 0.0;
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const double rel = (Uc[k] + gx * n[j][0] + gy * n[j][1]) - Uc[k];
+                    if (rel > mp) { mp = rel; px = n[j][0]; py = n[j][1]; }
+                    if (rel < mn) { mn = rel; qx = n[j][0]; qy = n[j][1]; }
+                }
+                const double dpos = mp + fvmr::kEPS, dneg = mn - fvmr::kEPS;
+                if (mp > 0.0 && hrel < dpos) {
+                    const double q = fdiv(hrel, dpos);
+                    if (!(phi < q)) {
+                        const double id = frcp(dpos);
+                        phi = q; hb = id; lb = 0.0; dxb = -q * id * px; dyb = -q * id * py;
+                    }
+                }
+                if (mn < 0.0 && lrel > dneg) {
+                    const double q = fdiv(lrel, dneg);
+                    if (!(phi < q)) {
+                        const double id = frcp(dneg);
+                        phi = q; hb = 0.0; lb = id; dxb = -q * id * qx; dyb = -q * id * qy;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const double d2 = gx * n[j][0] + gy * n[j][1];
+                    if (d2 == 0.0) continue;
+                    const double d1 = (d2 > 0.0) ? hrel : lrel;
+                    const double N = d1 * d1 + eps2 + 2.0 * d1 * d2, D = d1 * d1 + 2.0 * d2 * d2 + d1 * d2 + eps2;
+                    const double iD = frcp(D), q = N * iD;
+                    if (phi < q) continue;
+                    const double q1 = (2.0 * (d1 + d2) - q * (2.0 * d1 + d2)) * iD, q2 = (2.0 * d1 - q * (4.0 * d2 + d1)) * iD;
+                    phi = q;
+                    hb = (d2 > 0.0) ? q1 : 0.0;
+                    lb = (d2 > 0.0) ? 0.0 : q1;
+                    dxb = q2 * n[j][0];
+                    dyb = q2 * n[j][1];
+                }
+            }
+            const double phib = gbx[k] * gx + gby[k] * gy;
+            gxb = phi * gbx[k] + phib * dxb;
+            gyb = phi * gby[k] + phib * dyb;
+            sb = -phib * (hb + lb);
+#pragma unroll
+            for (int i = 0; i < 3; i++) ob[i] = (ih == i ? phib * hb : 0.0) + (il == i ? phib * lb : 0.0);
+            if (ih < 0) sb += phib * hb;
+            if (il < 0) sb += phib * lb;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const double t = gxb * cx[i] + gyb * cy[i];
+            sb += wc[i] * t;
+            ob[i] += wo[i] * t;
+            w[i][k] = ob[i];
+        }
+        self[k] = sb;
+    }
+}
 
 // The product with (dr/dU)^T, part 1 (one thread per cell c): the adjoints of c's three face
 // states (k_adj_faces) pass through the reconstruction to U_c and to c's limited gradient, whose
-// derivatives in U_c and the three states across (grad_limit on Dual<4>, one conserved variable
-// at a time: the variables do not mix) send them on: base[c] = the terms that land on U_c,
-// wedge[2 e + side] = the terms c sends to the cell across its edge e (side 1 when c is the
+// reverse mode (grad_limit_adj) sends them on to U_c and the three states across: base[c] = the terms that
+// land on U_c, wedge[2 e + side] = the terms c sends to the cell across its edge e (side 1 when c is the
 // edge's R).  With gbar, also the adjoint of c's limited gradient.
-#ifndef FVMR_ADJ_WAVES
-#define FVMR_ADJ_WAVES 2   // minimum waves per SIMD k_adj_vjp is compiled for (3 spills: slower)
-#endif
 template <bool GBAR>
-__global__ __launch_bounds__(kAdjBlock, FVMR_ADJ_WAVES) void k_adj_vjp(Mesh<double> m, Phys ph, const S4 *__restrict__ U,
+__global__ __launch_bounds__(kAdjBlock) void k_adj_vjp(Mesh<double> m, Phys ph, const S4 *__restrict__ U,
                                                         const Grad<double> *__restrict__ grad,
                                                         const S4 *__restrict__ fadj, S4 *__restrict__ base,
                                                         S4 *__restrict__ wedge, Grad<double> *__restrict__ gbar) {
-    using D = Dual<4>;
     const int c = blockIdx.x * kAdjBlock + threadIdx.x;
     const int nc = m.nc;
     if (c >= nc) return;
@@ -604,8 +716,7 @@ __global__ __launch_bounds__(kAdjBlock, FVMR_ADJ_WAVES) void k_adj_vjp(Mesh<doub
     }
     double self[4] = {0, 0, 0, 0}, w[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
     if (ph.reconstruct == FVMR_REC_LINEAR) {
-        double Uo[3][4];
-        SlotsU1 S;
+        double Uo[3][4], sa[3][3], sn[3][2];
         int fl[3];
 #pragma unroll
         for (int j = 0; j < 3; j++) {
@@ -614,8 +725,8 @@ __global__ __launch_bounds__(kAdjBlock, FVMR_ADJ_WAVES) void k_adj_vjp(Mesh<doub
             const V2<double> em = m.emid[edges[j]];
             ld(U, out >= 0 ? out : c, Uo[j]);
             const V2<double> nd = m.nxy[m.cnode[j * nc + c]];
-            S.n[j][0] = nd.x - cg.x;
-            S.n[j][1] = nd.y - cg.y;
+            sn[j][0] = nd.x - cg.x;
+            sn[j][1] = nd.y - cg.y;
             double Fx = 0.0, Fy = 0.0;
             if (out >= 0) {
                 const V4<double> og = m.cgeo[out];
@@ -623,20 +734,10 @@ __global__ __launch_bounds__(kAdjBlock, FVMR_ADJ_WAVES) void k_adj_vjp(Mesh<doub
                 Fy = og.y;
             }
             const double sgn = isR[j] ? -1.0 : 1.0;
-            slot_coef<double>(ph, out >= 0, cg.x, cg.y, em.x, em.y, Fx, Fy, eg.x * eg.z * sgn, eg.y * eg.z * sgn, S.a[j]);
+            slot_coef<double>(ph, out >= 0, cg.x, cg.y, em.x, em.y, Fx, Fy, eg.x * eg.z * sgn, eg.y * eg.z * sgn, sa[j]);
             fl[j] = (out >= 0) ? 3 : 0;
         }
-#pragma unroll 1
-        for (int k = 0; k < 4; k++) {
-#pragma unroll
-            for (int j = 0; j < 3; j++) S.uo[j] = D::seed(Uo[j][k], 1 + j);
-            const D Ud[1] = {D::seed(Uc[k], 0)};
-            D gx[1], gy[1];
-            grad_limit<D, SlotsU1, 1, double>(ph, Ud, S, fl, cg.z, gx, gy);
-            self[k] = gbx[k] * gx[0].d[0] + gby[k] * gy[0].d[0];
-#pragma unroll
-            for (int j = 0; j < 3; j++) w[j][k] = gbx[k] * gx[0].d[1 + j] + gby[k] * gy[0].d[1 + j];
-        }
+        grad_limit_adj(ph, Uc, Uo, sa, sn, fl, cg.z, gbx, gby, self, w);
     }
     base[c] = S4{ub[0] + self[0], ub[1] + self[1], ub[2] + self[2], ub[3] + self[3]};
 #pragma unroll
