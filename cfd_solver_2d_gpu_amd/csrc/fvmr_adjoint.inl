@@ -19,7 +19,8 @@
 // reconstruction passes its three face-state adjoints to U_c and to c's limited gradient; the
 // reverse mode of the limited gradient (grad_limit_adj, the branch taken by the values) sends that on
 // to U_c and to the neighbours: the share of neighbour n goes to a per-(edge, side) slot, which n's
-// gather (k_adj_update) adds in slot order, so the product is deterministic.  The limited gradients
+// gather (k_adj_update) adds in slot order, so the product is deterministic; k_adj_tile does all three
+// parts in one launch over the tiles.  The limited gradients
 // of U* (a primal quantity) are formed once per solve; the derivatives of flux, gradient and limiter are
 // recomputed in every product, and no Jacobian is stored.
 //
@@ -238,13 +239,13 @@ __device__ void roe_adj(const FaceState<double> &L, const FaceState<double> &R, 
     const double V2L = uL * uL + vL * vL, V2R = uR * uR + vR * vR;
     const double ga1 = gamma - 1.0;
     const double HL = pL * g_ga1 * L.ir + 0.5 * V2L, HR = pR * g_ga1 * R.ir + 0.5 * V2R;
-    const double rrorl = sqrt(rR * L.ir);
-    const double inv_p1 = 1.0 / (rrorl + 1.0);
-    const double rm = rL * rrorl;
+    const double rrorl = fsqrt(rR * L.ir);
+    const double inv_p1 = frcp(rrorl + 1.0);
+    const double rm = rL * rrorl, inv_rm = frcp(rm);
     const double um = (uL + uR * rrorl) * inv_p1, vm = (vL + vR * rrorl) * inv_p1, Hm = (HL + HR * rrorl) * inv_p1;
     const double Vm2 = um * um + vm * vm;
-    const double am = sqrt(ga1 * (Hm - 0.5 * Vm2));
-    const double inv_am = 1.0 / am;
+    const double am = fsqrt(ga1 * (Hm - 0.5 * Vm2));
+    const double inv_am = frcp(am);
     const double unm = um * nx + vm * ny;
     const double eig1 = fabs(unm), eig2 = fabs(unm + am), eig3 = fabs(unm - am);
     const double ER = HR - pR * R.ir, EL = HL - pL * L.ir;
@@ -255,7 +256,7 @@ __device__ void roe_adj(const FaceState<double> &L, const FaceState<double> &R, 
     const double Mstar = (eig2 - eig3) * 0.5 * inv_am;
     const double dun = nx * (uR - uL) + ny * (vR - vL);
     const double dp = pR - pL;
-    const double B = (astar - eig1) * dp / rm, Cq = inv_am * inv_am;
+    const double B = (astar - eig1) * dp * inv_rm, Cq = inv_am * inv_am;
     const double dUroe = Mstar * dun + B * Cq;
     const double dProe = Mstar * dp + (astar - eig1) * rm * dun;
     // central part 0.5 (F_L + F_R) area
@@ -286,8 +287,8 @@ __device__ void roe_adj(const FaceState<double> &L, const FaceState<double> &R, 
     dunb += dUroeb * Mstar;
     const double Bb = dUroeb * Cq;
     double inv_amb = dUroeb * B * 2.0 * inv_am;
-    const double Ab = Bb / rm;
-    rmb -= Bb * B / rm;
+    const double Ab = Bb * inv_rm;
+    rmb -= Ab * B;
     astarb += Ab * dp;
     eig1b -= Ab * dp;
     dpb += Ab * (astar - eig1);
@@ -319,7 +320,7 @@ __device__ void roe_adj(const FaceState<double> &L, const FaceState<double> &R, 
     vmb += unmb * ny;
     // inv_am, am = sqrt(ga1 (Hm - Vm2 / 2))
     amb -= inv_amb * inv_am * inv_am;
-    const double am2b = amb * 0.5 / am;
+    const double am2b = amb * 0.5 * inv_am;
     Hmb += am2b * ga1;
     Vm2b -= am2b * ga1 * 0.5;
     umb += Vm2b * 2.0 * um;
@@ -332,7 +333,7 @@ __device__ void roe_adj(const FaceState<double> &L, const FaceState<double> &R, 
     rLb += rmb * rrorl;
     rrorlb += rmb * rL;
     rrorlb -= inv_p1b * inv_p1 * inv_p1;
-    const double sb = rrorlb * 0.5 / rrorl;
+    const double sb = fdiv(rrorlb * 0.5, rrorl);
     rRb += sb * L.ir;
     irLb += sb * rR;
     // total enthalpies
@@ -355,7 +356,7 @@ __device__ void llf_adj(const FaceState<double> &L, const FaceState<double> &R, 
                         double gamma, double g_ga1, const double mu[4], PrimBar &Lb, PrimBar &Rb, double ULc[4],
                         double URc[4]) {
     const double unL = nx * L.u + ny * L.v, unR = nx * R.u + ny * R.v;
-    const double cL = sqrt(gamma * L.p * L.ir), cR = sqrt(gamma * R.p * R.ir);
+    const double cL = fsqrt(gamma * L.p * L.ir), cR = fsqrt(gamma * R.p * R.ir);
     const double aL = fabs(unL) + cL, aR = fabs(unR) + cR;
     const double lam = (aL > aR) ? aL : aR;
     const double h = 0.5 * len;
@@ -378,7 +379,7 @@ __device__ void llf_adj(const FaceState<double> &L, const FaceState<double> &R, 
         Sb.v += h * mu[2] * t + hsb * S.v;
         Sb.p += h * (mu[1] * nx + mu[2] * ny) + hsb * g_ga1 * S.ir;
         Sb.ir += hsb * S.p * g_ga1;
-        const double wb = ab * 0.5 / c;
+        const double wb = fdiv(ab * 0.5, c);
         Sb.p += wb * gamma * S.ir;
         Sb.ir += wb * gamma * S.p;
         Sb.u += unb * nx;
@@ -388,65 +389,49 @@ __device__ void llf_adj(const FaceState<double> &L, const FaceState<double> &R, 
     side(R, unR, cR, aRb, Rb);
 }
 
-// ghost_farfield, reverse: Rc = adjoint of the ghost's conserved state; into L's primitives
-__device__ void farfield_adj(const FaceState<double> &L, const double *ruvp_inf, double nx, double ny, double gamma,
-                             const double Rc[4], PrimBar &Lb) {
+// ghost_farfield, reverse: Rc = adjoint of the ghost's conserved state; into L's primitives.  The subsonic
+// ghost's density is rho_s (a_*^2 / a_s^2)^(1 / (gamma - 1)), so its derivatives are quotients of the value
+// that R holds; with the powers formed again a work-group at the far field took about 4 us longer.
+__device__ __forceinline__ void farfield_adj(const FaceState<double> &L, const FaceState<double> &R, const double *ruvp_inf,
+                                             double nx, double ny, double gamma, const double Rc[4], PrimBar &Lb) {
     const double ga1 = gamma - 1;
     const double rho_f = ruvp_inf[0], u_f = ruvp_inf[1], v_f = ruvp_inf[2], p_f = ruvp_inf[3];
-    const double rho_e = L.r, u_e = L.u, v_e = L.v, p_e = L.p;
-    const double af = sqrt(gamma * p_f / rho_f);
-    const double ae = sqrt(gamma * p_e / rho_e);
-    const double qnf = u_f * nx + v_f * ny, qne = u_e * nx + v_e * ny;
-    const double rf = qnf - 2.0 * af / ga1, re = qne + 2.0 * ae / ga1;
+    const double rho_e = L.r, p_e = L.p;
+    const double af = fsqrt(fdiv(gamma * p_f, rho_f));
+    const double ae = fsqrt(fdiv(gamma * p_e, rho_e));
+    const double qnf = u_f * nx + v_f * ny, qne = L.u * nx + L.v * ny;
+    const double rf = qnf - fdiv(2.0 * af, ga1), re = qne + fdiv(2.0 * ae, ga1);
     const double qn = 0.5 * (re + rf), as = ga1 * (re - rf) / 4.0;
     if (qn <= -as) return;   // freestream state: no dependence on L
-    double r0[4];
     const bool sub = qn < as, in = qn < 0;
-    double s_p = 0, s_r = 0, son = 0, X = 0;
-    if (sub) {
-        s_p = in ? p_f : p_e;
-        s_r = in ? rho_f : rho_e;
-        const double s_u = in ? u_f : u_e, s_v = in ? v_f : v_e, s_qn = in ? qnf : qne;
-        son = s_p / pow(s_r, gamma);
-        X = as * as / son / gamma;
-        r0[0] = pow(X, 1.0 / ga1);
-        r0[1] = s_u - s_qn * nx + qn * nx;
-        r0[2] = s_v - s_qn * ny + qn * ny;
-        r0[3] = as * as * r0[0] / gamma;
-    } else {
-        r0[0] = rho_e; r0[1] = u_e; r0[2] = v_e; r0[3] = p_e;
-    }
     // ruvp2u, reverse
     double r0b[4];
-    r0b[0] = Rc[0] + Rc[1] * r0[1] + Rc[2] * r0[2] + Rc[3] * 0.5 * (r0[1] * r0[1] + r0[2] * r0[2]);
-    r0b[1] = Rc[1] * r0[0] + Rc[3] * r0[0] * r0[1];
-    r0b[2] = Rc[2] * r0[0] + Rc[3] * r0[0] * r0[2];
-    r0b[3] = Rc[3] / ga1;
+    r0b[0] = Rc[0] + Rc[1] * R.u + Rc[2] * R.v + Rc[3] * 0.5 * (R.u * R.u + R.v * R.v);
+    r0b[1] = Rc[1] * R.r + Rc[3] * R.r * R.u;
+    r0b[2] = Rc[2] * R.r + Rc[3] * R.r * R.v;
+    r0b[3] = fdiv(Rc[3], ga1);
     if (!sub) {
         Lb.r += r0b[0]; Lb.u += r0b[1]; Lb.v += r0b[2]; Lb.p += r0b[3];
         return;
     }
-    const double r00b = r0b[0] + r0b[3] * as * as / gamma;
-    double asb = r0b[3] * 2.0 * as * r0[0] / gamma;
-    double qnb = r0b[1] * nx + r0b[2] * ny;
-    const double s_ub = r0b[1], s_vb = r0b[2], s_qnb = -r0b[1] * nx - r0b[2] * ny;
-    const double Xb = r00b * (1.0 / ga1) * pow(X, 1.0 / ga1 - 1.0);
-    asb += Xb * 2.0 * as / son / gamma;
-    const double sonb = -Xb * as * as / (son * son) / gamma;
+    // rho = rho_s (as^2 rho_s / (gamma p_s))^(1 / ga1), p = as^2 rho / gamma
+    const double rb = (r0b[0] + fdiv(r0b[3] * as * as, gamma)) * R.r;   // the adjoint of ln rho
+    const double qb = fdiv(rb, ga1);
+    const double asb = fdiv(r0b[3] * 2.0 * as * R.r, gamma) + fdiv(2.0 * qb, as);
+    const double qnb = r0b[1] * nx + r0b[2] * ny;
     double qneb = 0.0;
     if (!in) {
-        const double srg = pow(s_r, gamma);
-        Lb.p += sonb / srg;
-        Lb.r -= sonb * s_p * gamma * pow(s_r, gamma - 1.0) / (srg * srg);
-        Lb.u += s_ub;
-        Lb.v += s_vb;
-        qneb += s_qnb;
+        Lb.p -= fdiv(qb, p_e);
+        Lb.r += fdiv(gamma * qb, rho_e);
+        Lb.u += r0b[1];
+        Lb.v += r0b[2];
+        qneb -= qnb;
     }
     const double reb = 0.5 * qnb + asb * ga1 / 4.0;
     qneb += reb;
-    const double wb = reb * 2.0 / ga1 * 0.5 / ae;
-    Lb.p += wb * gamma / rho_e;
-    Lb.r -= wb * gamma * p_e / (rho_e * rho_e);
+    const double wb = fdiv(fdiv(reb, ga1), ae);
+    Lb.p += fdiv(wb * gamma, rho_e);
+    Lb.r -= fdiv(wb * gamma * p_e, rho_e * rho_e);
     Lb.u += qneb * nx;
     Lb.v += qneb * ny;
 }
@@ -490,7 +475,7 @@ __device__ void face_vjp(const Phys &ph, int bType, const double *ruvp, const do
         ULc[0] += URc[0];
         ULc[3] += URc[3];
     } else {
-        farfield_adj(L, ruvp, nx, ny, gamma, URc, Lb);
+        farfield_adj(L, R, ruvp, nx, ny, gamma, URc, Lb);
     }
     set_prim_adj(L, gamma, Lb, ULc);
 #pragma unroll
@@ -521,11 +506,11 @@ __global__ __launch_bounds__(kBlock) void k_adj_faces(Mesh<double> m, Phys ph, c
     ld(psi, Rs, pR);
     recon_state(ph, UL, grL, gL.x, gL.y, em.x, em.y, ULf);
 #pragma unroll
-    for (int k = 0; k < 4; k++) mu[k] = -pL[k] / gL.z;
+    for (int k = 0; k < 4; k++) mu[k] = fdiv(-pL[k], gL.z);
     if (interior) {
         recon_state(ph, UR, grR, gR.x, gR.y, em.x, em.y, URf);
 #pragma unroll
-        for (int k = 0; k < 4; k++) mu[k] += pR[k] / gR.z;
+        for (int k = 0; k < 4; k++) mu[k] += fdiv(pR[k], gR.z);
     }
     double ULb[4], URb[4];
     face_vjp(ph, bType, bc_state(ph, ph.bc, bType, em.x, em.y, 0.0), ULf, URf, eg.x, eg.y, eg.z, mu, ULb, URb);
@@ -754,9 +739,35 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_vjp(Mesh<double> m, Phys ph, 
     }
 }
 
-// Part 2 (one thread per cell): v = base[c] + the wedge terms of c's neighbours in slot order
-// (+ g[c]).  Without dtl: out = v.  With dtl, one pseudo-time stage: s = psi_in + dt_c v,
-// psi_out = s (first) or a psi_n + b s.  res (optional) = v.
+// The end of a product at cell c: v = the product + g[c].  Without dtl: out = v.  With dtl, one
+// pseudo-time stage: s = psi_in + dt_c v, psi_out = s (first) or a psi_n + b s.  res (optional) = v.
+__device__ __forceinline__ void adj_stage(int c, double v[4], const S4 *__restrict__ g, const S4 *__restrict__ pin,
+                                          const S4 *__restrict__ pn, S4 *__restrict__ pout, const double *__restrict__ dtl,
+                                          double a, double b, int first, S4 *__restrict__ res) {
+    if (g) {
+        double q[4];
+        ld(g, c, q);
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] += q[k];
+    }
+    if (res) st(res, c, v);
+    if (!dtl) {
+        st(pout, c, v);
+        return;
+    }
+    const double dt = dtl[c];
+    double pi[4], pb[4] = {0, 0, 0, 0}, o[4];
+    ld(pin, c, pi);
+    if (!first) ld(pn, c, pb);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double s = pi[k] + dt * v[k];
+        o[k] = first ? s : a * pb[k] + b * s;
+    }
+    st(pout, c, o);
+}
+
+// Part 2 (one thread per cell): base[c] + the wedge terms of c's neighbours in slot order, then adj_stage.
 __global__ __launch_bounds__(kBlock) void k_adj_update(Mesh<double> m, const S4 *__restrict__ base,
                                                         const S4 *__restrict__ wedge, const S4 *__restrict__ g,
                                                         const S4 *__restrict__ pin, const S4 *__restrict__ pn,
@@ -785,27 +796,187 @@ __global__ __launch_bounds__(kBlock) void k_adj_update(Mesh<double> m, const S4 
 #pragma unroll
             for (int k = 0; k < 4; k++) v[k] += q[j][k];
         }
-    if (g) {
+    adj_stage(c, v, g, pin, pn, pout, dtl, a, b, first, res);
+}
+
+// A scheme of k_adj_tile beside kTileAny and kTileGg: Green-Gauss, Roe, linear reconstruction and any limiter
+// (162 against 180 VGPRs: three work-groups to a CU, not two).
+constexpr int kTileGgRoe = 3;
+
+// One product with (dr/dU)^T and its pseudo-time stage over the tiles (the work of k_adj_faces, k_adj_vjp and
+// k_adj_update in one launch): each work-group forms the face adjoints of its tile's and first ring's cells, the
+// cell products of both, and the sums of its tile cells; psi, U and its gradients are staged for the tile and
+// both rings.  Between the three cell kernels 128 bytes per face and 32 per cell are written and read again,
+// which bounds them; here about 0.4 faces more per face of the mesh are formed, and nothing but the next psi is
+// written.  What bounds it is the face phase: about 130 registers live, so three waves per SIMD at best and the
+// latency of its divisions and roots in view.  So the records of the cells are loaded after that phase, and a
+// work-item's second face goes to LDS of its own before the first is formed (held in registers, with the records:
+// 209 VGPRs, 6.9 ms; 384 work-items with one face each 8.4 ms; bounded to 168 VGPRs with spills 9.4 ms).  LDS:
+// the face adjoints replace the staged psi and gradients, and the shares sent across the faces replace those;
+// 46 KB, three work-groups to a CU.  393,216 cells of an airfoil O-grid: one launch 44 us against 36 + 45 +
+// 17 us; 30 RK3 iterations 10.3 -> 5.2 ms.
+template <int SCHEME>
+__global__ __launch_bounds__(TileCfg<double>::kThreads) void k_adj_tile(
+    TileArgs<double> ta, Phys ph, const V4<double> *__restrict__ cgeo, const S4 *__restrict__ U,
+    const Grad<double> *__restrict__ grad, const S4 *__restrict__ psi, const S4 *__restrict__ g,
+    const S4 *__restrict__ pn, S4 *__restrict__ pout, const double *__restrict__ dtl, double a, double b, int first,
+    S4 *__restrict__ res) {
+    fix_scheme<SCHEME == kTileGgRoe ? kTileGg : SCHEME, false>(ph);
+    if (SCHEME == kTileGgRoe) {
+        ph.scheme = FVMR_SOL_ROE;
+        ph.reconstruct = FVMR_REC_LINEAR;
+    }
+    using Cfg = TileCfg<double>;
+    constexpr int T = Cfg::kThreads, kF2 = Cfg::kMaxF - T;   // faces beyond the first per work-item
+    static_assert(kF2 > 0 && kF2 <= T, "at most two faces per work-item");
+    __shared__ struct {
+        alignas(16) char U[Cfg::kMaxL * sizeof(S4)];
+        union {
+            struct {
+                alignas(16) char lam[Cfg::kMaxL * sizeof(S4)];   // -psi / V
+                char grad[Cfg::kMaxL * sizeof(Grad<double>)];
+            };
+            char fadj[2 * T * sizeof(S4)];    // face f: its L state's adjoint at 2 f, its R state's at 2 f + 1
+            char share[2 * Cfg::kMaxFF * sizeof(S4)];  // face f: what L sends to R at 2 f, what R sends to L at 2 f + 1
+        };
+        alignas(16) char fadj2[2 * kF2 * sizeof(S4)];   // the same of face T + f
+        V2<double> N[Cfg::kMaxN];
+        V2<double> cen[Cfg::kMaxL];
+        unsigned char lin[Cfg::kMaxF];   // bit 0: face f's L state is the linear reconstruction, bit 1: R's
+    } lds;
+    const int i = threadIdx.x;
+    const int *ti = ta.info + (size_t)xcd_block() * fvmr::kTileInfo;
+    const int c0 = ti[fvmr::kTiC0], nT = ti[fvmr::kTiNT], nG = ti[fvmr::kTiNG], nL = ti[fvmr::kTiNL];
+    const int nN = ti[fvmr::kTiNN], nF = ti[fvmr::kTiNF], nFF = ti[fvmr::kTiNFF];
+    const int offH = ti[fvmr::kTiOffH], offN = ti[fvmr::kTiOffN], offF = ti[fvmr::kTiOffF];
+    const int offL = ti[fvmr::kTiOffL], offG = ti[fvmr::kTiOffG];
+    // 1. staging, every global load issued before the first LDS store (see k_tile)
+    const I3 fr0 = (i < nF) ? ta.face[offF + i] : I3{0, 0, 0};
+    const I3 fr1 = (i + T < nF) ? ta.face[offF + i + T] : I3{0, 0, 0};
+    const int src = (i < nL) ? (i < nT ? c0 + i : ta.halo[offH + i - nT]) : c0;
+    const V2<double> nd = (i < nN) ? ta.nxy[offN + i] : V2<double>{0.0, 0.0};
+    const S4 u = U[src], p = psi[src];
+    const V4<double> cg = cgeo[src];
+    const Grad<double> gr = grad[src];
+    if (i < nN) lds.N[i] = nd;
+    if (i < nL) {
+        lds_put(lds.U, Cfg::kMaxL, i, u);
+        lds_put(lds.lam, Cfg::kMaxL, i, S4{fdiv(-p.x, cg.z), fdiv(-p.y, cg.z), fdiv(-p.z, cg.z), fdiv(-p.w, cg.z)});
+        lds_put(lds.grad, Cfg::kMaxL, i, gr);
+        lds.cen[i] = V2<double>{cg.x, cg.y};
+    }
+    __syncthreads();
+    // 2. the adjoints of the two reconstructed states of every face (k_adj_faces)
+    const CaseBC &bc = ta.cbc[0];
+    auto face = [&](int f, const I3 fr, S4 &oL, S4 &oR) {
+        V4<double> eg;
+        V2<double> em;
+        tile_face_geom<double>(lds.N, fr, eg, em);
+        const int bType = tile_btype(fr);
+        const bool interior = bType == -1;
+        const int L = lfield(fr.y, 0), R = interior ? lfield(fr.y, 1) : L;
+        double Uc[4], ULf[4], URf[4] = {0, 0, 0, 0}, mu[4], lR[4], ULb[4], URb[4];
+        lds_state(lds.U, Cfg::kMaxL, L, Uc);
+        const V2<double> cL = lds.cen[L], cR = lds.cen[R];
+        int lin = recon_state(ph, Uc, lds_get<Grad<double>>(lds.grad, Cfg::kMaxL, L), cL.x, cL.y, em.x, em.y, ULf) ? 1 : 0;
+        lds_state(lds.lam, Cfg::kMaxL, L, mu);
+        if (interior) {
+            lds_state(lds.U, Cfg::kMaxL, R, Uc);
+            if (recon_state(ph, Uc, lds_get<Grad<double>>(lds.grad, Cfg::kMaxL, R), cR.x, cR.y, em.x, em.y, URf)) lin |= 2;
+            lds_state(lds.lam, Cfg::kMaxL, R, lR);
+#pragma unroll
+            for (int k = 0; k < 4; k++) mu[k] -= lR[k];
+        }
+        face_vjp(ph, bType, bc_state(ph, bc, bType, em.x, em.y, 0.0), ULf, URf, eg.x, eg.y, eg.z, mu, ULb, URb);
+        oL = S4{ULb[0], ULb[1], ULb[2], ULb[3]};
+        oR = S4{URb[0], URb[1], URb[2], URb[3]};
+        lds.lin[f] = (unsigned char)lin;
+    };
+    S4 fL{0, 0, 0, 0}, fR{0, 0, 0, 0};
+    if (i + T < nF) {   // the second face first: its place is not that of what is still read
+        face(i + T, fr1, fL, fR);
+        lds_put(lds.fadj2, 2 * kF2, 2 * i, fL);
+        lds_put(lds.fadj2, 2 * kF2, 2 * i + 1, fR);
+    }
+    if (i < nF) face(i, fr0, fL, fR);
+    __syncthreads();
+    if (i < nF) {
+        lds_put(lds.fadj, 2 * T, 2 * i, fL);
+        lds_put(lds.fadj, 2 * T, 2 * i + 1, fR);
+    }
+    const int nw = (i < nG) ? ta.lnodes[offL + i] : 0;
+    const I3 gs = (i < nG) ? ta.gslot[offG + i] : I3{0, 0, 0};
+    const V4<double> gco = (i < nG) ? ta.gcoef[offG + i] : V4<double>{0.5, 0.5, 0.5, 1.0};
+    __syncthreads();
+    // 3. the products of the tile's and the first ring's cells (k_adj_vjp)
+    const int sw[3] = {gs.x, gs.y, gs.z};
+    double v[4] = {0, 0, 0, 0}, w[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    if (i < nG) {
+        double Uc[4], Uo[3][4], sa[3][3], sn[3][2], gbx[4] = {0, 0, 0, 0}, gby[4] = {0, 0, 0, 0}, self[4];
+        int fl[3];
+        lds_state(lds.U, Cfg::kMaxL, i, Uc);
+        const V2<double> vn[3] = {lds.N[lfield(nw, 0)], lds.N[lfield(nw, 1)], lds.N[lfield(nw, 2)]};
+        const V2<double> cen = lds.cen[i];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int f = sw[j] & fvmr::kLocalMask, side = (sw[j] & fvmr::kGsIsR) ? 1 : 0;
+            const int out = (sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask;
+            const bool has_out = out != fvmr::kLocalNone;
+            const V2<double> P = vn[j], Q = vn[(j + 1) % 3];
+            double ub[4];
+            if (f < T) lds_state(lds.fadj, 2 * T, 2 * f + side, ub);
+            else lds_state(lds.fadj2, 2 * kF2, 2 * (f - T) + side, ub);
+            const bool lin = (lds.lin[f] >> side) & 1;
+            const double dx = (P.x + Q.x) / 2.0 - cen.x, dy = (P.y + Q.y) / 2.0 - cen.y;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] += ub[k];
+                if (lin) {
+                    gbx[k] += ub[k] * dx;
+                    gby[k] += ub[k] * dy;
+                }
+            }
+            lds_state(lds.U, Cfg::kMaxL, has_out ? out : i, Uo[j]);
+            sn[j][0] = P.x - cen.x;
+            sn[j][1] = P.y - cen.y;
+            if (ph.gradient == FVMR_GRA_GREENGAUSS) {
+                sa[j][0] = j == 0 ? gco.x : (j == 1 ? gco.y : gco.z);
+                sa[j][1] = negate_if<fvmr::kGsTurned>(Q.y - P.y, sw[j]);
+                sa[j][2] = negate_if<fvmr::kGsTurned>(P.x - Q.x, sw[j]);
+            } else {
+                const V2<double> co = lds.cen[has_out ? out : i];
+                sa[j][0] = co.x - cen.x;
+                sa[j][1] = co.y - cen.y;
+                sa[j][2] = 0.0;
+            }
+            fl[j] = has_out ? 3 : 0;
+        }
+        if (ph.reconstruct == FVMR_REC_LINEAR) {
+            grad_limit_adj(ph, Uc, Uo, sa, sn, fl, gco.w, gbx, gby, self, w);
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] += self[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int f = sw[j] & fvmr::kLocalMask;
+        if (i < nG && f < nFF)
+            lds_put(lds.share, 2 * Cfg::kMaxFF, 2 * f + ((sw[j] & fvmr::kGsIsR) ? 1 : 0), S4{w[j][0], w[j][1], w[j][2], w[j][3]});
+    }
+    __syncthreads();
+    // 4. the tile's sums and the stage (k_adj_update)
+    if (i >= nT) return;
+    const int c = c0 + i;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        if (((sw[j] >> fvmr::kGsOutShift) & fvmr::kLocalMask) == fvmr::kLocalNone) continue;
         double q[4];
-        ld(g, c, q);
+        lds_state(lds.share, 2 * Cfg::kMaxFF, 2 * (sw[j] & fvmr::kLocalMask) + ((sw[j] & fvmr::kGsIsR) ? 0 : 1), q);
 #pragma unroll
         for (int k = 0; k < 4; k++) v[k] += q[k];
     }
-    if (res) st(res, c, v);
-    if (!dtl) {
-        st(pout, c, v);
-        return;
-    }
-    const double dt = dtl[c];
-    double pi[4], pb[4] = {0, 0, 0, 0}, o[4];
-    ld(pin, c, pi);
-    if (!first) ld(pn, c, pb);
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const double s = pi[k] + dt * v[k];
-        o[k] = first ? s : a * pb[k] + b * s;
-    }
-    st(pout, c, o);
+    adj_stage(c, v, g, psi, pn, pout, dtl, a, b, first, res);
 }
 
 // dJ/dU of J = sum_v W_v Cp_v with Cp_v = (p_v - p_inf) / p_dyn and p_v the mean of the
@@ -1206,35 +1377,54 @@ int field_norm2(fvmr_solver *h, const S4 *f, double out[4]) {
     return FVMR_OK;
 }
 
-// One product with (dr/dU)^T at U (gradients recomputed first): base/wedge, then the gather.
+// The limited gradients of U (a primal quantity), once per solve.
+int adj_gradient(fvmr_solver *h, const S4 *U) {
+    AdjWork *w = (AdjWork *)h->adj;
+    if (w->grad_ready) return FVMR_OK;
+    const int rc = launch_gradient<double, double>(h, U, -1);
+    w->grad_ready = rc == FVMR_OK;
+    return rc;
+}
+
+// The face and cell parts of one product with (dr/dU)^T at U: base/wedge, and with gbar the adjoints of the
+// limited gradients.
 int adj_product(fvmr_solver *h, const S4 *U, const S4 *psi, bool with_gbar) {
     AdjWork *w = (AdjWork *)h->adj;
-    if (!w->grad_ready) {   // the limited gradients of U (a primal quantity) once per solve
-        const int rc = launch_gradient<double, double>(h, U, -1);
-        if (rc) return rc;
-        w->grad_ready = true;
-    }
+    const int rc = adj_gradient(h, U);
+    if (rc) return rc;
     const Mesh<double> m = mesh_args<double>(h);
     k_adj_faces<<<grid_of(h->nf), kBlock, 0, h->stream>>>(m, h->ph, U, (const Grad<double> *)h->grad, psi, w->fadj);
     HIP_OK(hipGetLastError());
-    if (with_gbar) {
-        if (!w->gbar && hipMalloc((void **)&w->gbar, (size_t)h->nc * sizeof(Grad<double>)) != hipSuccess)
-            return set_error(FVMR_ERR_HIP, "hipMalloc adjoint gradient");
-        k_adj_vjp<true><<<adj_grid(h->nc), kAdjBlock, 0, h->stream>>>(m, h->ph, U, (const Grad<double> *)h->grad,
-                                                                                   w->fadj, w->base, w->wedge, w->gbar);
-    } else {
-        k_adj_vjp<false><<<adj_grid(h->nc), kAdjBlock, 0, h->stream>>>(m, h->ph, U, (const Grad<double> *)h->grad,
-                                                                                    w->fadj, w->base, w->wedge, nullptr);
-    }
+    if (with_gbar && !w->gbar && hipMalloc((void **)&w->gbar, (size_t)h->nc * sizeof(Grad<double>)) != hipSuccess)
+        return set_error(FVMR_ERR_HIP, "hipMalloc adjoint gradient");
+    auto *kern = with_gbar ? k_adj_vjp<true> : k_adj_vjp<false>;
+    kern<<<adj_grid(h->nc), kAdjBlock, 0, h->stream>>>(m, h->ph, U, (const Grad<double> *)h->grad, w->fadj, w->base, w->wedge,
+                                                       with_gbar ? w->gbar : nullptr);
     HIP_OK(hipGetLastError());
     return FVMR_OK;
 }
 
-int adj_update(fvmr_solver *h, const S4 *g, const S4 *pin, const S4 *pn, S4 *pout, bool step, double a, double b,
-               int first, S4 *res) {
+// pout = (dr/dU)^T psi + g (without step), or one pseudo-time stage with it (see adj_stage).
+int adj_step(fvmr_solver *h, const S4 *U, const S4 *psi, const S4 *g, const S4 *pn, S4 *pout, bool step, double a, double b,
+             int first, S4 *res) {
     AdjWork *w = (AdjWork *)h->adj;
-    k_adj_update<<<grid_of(h->nc), kBlock, 0, h->stream>>>(mesh_args<double>(h), w->base, w->wedge, g, pin, pn, pout,
-                                                           step ? w->dtl : nullptr, a, b, first, res);
+    int rc;
+    const double *dtl = step ? w->dtl : nullptr;
+    // tiles of the default shape: one launch, 44 us against the cell kernels' 98 at 393,216 cells, 12 against
+    // 30 at 49,152 (the other work-group shapes use the cell kernels here, as the rest of the steady path)
+    if (h->tiles && h->shape == 0) {
+        if ((rc = adj_gradient(h, U))) return rc;
+        const bool gg = h->ph.gradient == FVMR_GRA_GREENGAUSS;
+        const bool roe = h->ph.scheme == FVMR_SOL_ROE && h->ph.reconstruct == FVMR_REC_LINEAR;
+        auto *kern = gg ? (roe ? k_adj_tile<kTileGgRoe> : k_adj_tile<kTileGg>) : k_adj_tile<kTileAny>;
+        kern<<<h->ntiles, TileCfg<double>::kThreads, 0, h->stream>>>(tile_args<double>(h), h->ph, mesh_args<double>(h).cgeo, U,
+                                                                      (const Grad<double> *)h->grad, psi, g, pn, pout, dtl, a, b,
+                                                                      first, res);
+    } else {
+        if ((rc = adj_product(h, U, psi, false))) return rc;
+        k_adj_update<<<grid_of(h->nc), kBlock, 0, h->stream>>>(mesh_args<double>(h), w->base, w->wedge, g, psi, pn, pout, dtl, a,
+                                                               b, first, res);
+    }
     HIP_OK(hipGetLastError());
     return FVMR_OK;
 }
@@ -1329,14 +1519,13 @@ int adj_iteration(fvmr_solver *h, const S4 *U, const S4 *g, const S4 *x, S4 *out
     S4 *Pb = w->psi[2], *Pc = w->psi[3];
     int rc;
     if (h->p.time_advance == FVMR_EVO_RK3) {
-        if ((rc = adj_product(h, U, x, false)) || (rc = adj_update(h, g, x, x, Pb, true, 0.0, 1.0, 1, res)) ||
-            (rc = adj_product(h, U, Pb, false)) || (rc = adj_update(h, g, Pb, x, Pc, true, 0.75, 0.25, 0, nullptr)) ||
-            (rc = adj_product(h, U, Pc, false)) ||
-            (rc = adj_update(h, g, Pc, x, out, true, 1.0 / 3.0, 2.0 / 3.0, 0, nullptr)))
+        if ((rc = adj_step(h, U, x, g, x, Pb, true, 0.0, 1.0, 1, res)) ||
+            (rc = adj_step(h, U, Pb, g, x, Pc, true, 0.75, 0.25, 0, nullptr)) ||
+            (rc = adj_step(h, U, Pc, g, x, out, true, 1.0 / 3.0, 2.0 / 3.0, 0, nullptr)))
             return rc;
         return FVMR_OK;
     }
-    if ((rc = adj_product(h, U, x, false)) || (rc = adj_update(h, g, x, x, out, true, 0.0, 1.0, 1, res))) return rc;
+    if ((rc = adj_step(h, U, x, g, x, out, true, 0.0, 1.0, 1, res))) return rc;
     return FVMR_OK;
 }
 
@@ -1413,8 +1602,7 @@ int fvmr_adjoint_vjp(fvmr_handle *h, const double *const psi[4], double *const o
     const S4 *U = h->Ubuf[h->cur];
     w->grad_ready = false;
     if ((rc = upload_field(h, psi, w->psi[0]))) return rc;
-    if ((rc = adj_product(h, U, w->psi[0], false))) return rc;
-    if ((rc = adj_update(h, nullptr, nullptr, nullptr, w->psi[1], false, 0, 0, 1, nullptr))) return rc;
+    if ((rc = adj_step(h, U, w->psi[0], nullptr, nullptr, w->psi[1], false, 0, 0, 1, nullptr))) return rc;
     if ((rc = read_back(h, w->psi[1], out))) return rc;
     if (dalpha && (rc = adj_alpha(h, U, w->psi[0], dalpha))) return rc;
     if (dxy && (rc = adj_coords(h, U, w->psi[0], dxy))) return rc;
@@ -1479,8 +1667,7 @@ int fvmr_adjoint_solve(fvmr_handle *h, int nsets, const int *set_offsets, const 
     // the residual of the adjoint equation at the start (psi = 0: dJ/dU) and at the end
     if ((rc = field_norm2(h, w->g, nrm))) return rc;
     r0 = std::sqrt(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2] + nrm[3] * nrm[3]);
-    if ((rc = adj_product(h, U, w->psi[a], false)) ||
-        (rc = adj_update(h, w->g, nullptr, nullptr, w->res, false, 0, 0, 1, nullptr)) ||
+    if ((rc = adj_step(h, U, w->psi[a], w->g, nullptr, w->res, false, 0, 0, 1, nullptr)) ||
         (rc = field_norm2(h, w->res, nrm)))
         return rc;
     r = std::sqrt(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2] + nrm[3] * nrm[3]);

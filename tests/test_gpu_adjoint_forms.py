@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 import cfd_solver_2d_gpu_amd as F
-from test_gpu_adjoint import announce, modulated_state, naca_mesh, naca_params, rel
+from test_gpu_adjoint import announce, modulated_state, naca_mesh, naca_params, rel, wall_sets
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,39 @@ def test_vjp_forms_match_residual_differences(form, kernels):
     g.close()
     fd, ad = np.sum(psi * (rp - rm)) / (2 * eps), np.sum(out * v)
     assert rel(fd, ad) < 1e-6, (fd, ad)
+
+
+@pytest.mark.parametrize("tile_cells", [0, 1, 37])
+@pytest.mark.parametrize("form", FORMS + [(F.GRA_LEASTSQUARE, F.LIM_BARTH, F.SOL_ROE, F.REC_LINEAR, 1)])
+def test_vjp_tile_and_cell_kernels_agree(form, tile_cells):
+    """The two kernels add the same terms in the same order from geometry that differs by two
+    roundings: a few hundred operations of 1e-16 on terms that partly cancel, hence 1e-12."""
+    announce(f"adjoint product, tile vs cell kernels, form {form}, tile_cells {tile_cells}")
+    m = naca_mesh(47, 15, 1.2)
+    out = []
+    for kw in ({"kernels": F.KERNELS_TILE, "tile_cells": tile_cells}, {"kernels": F.KERNELS_CELL}):
+        p = form_params(form, **kw)
+        U = modulated_state(m, p)
+        g = F.GPUSolver2(m, p)
+        g.set_state(U)
+        out.append(g.adjoint_vjp(np.random.default_rng(23).standard_normal(U.shape)))
+        g.close()
+    assert np.linalg.norm(out[0] - out[1]) / np.linalg.norm(out[1]) < 1e-12
+
+
+@pytest.mark.parametrize("time_advance", [F.EVO_RK3, F.EVO_EXPLICIT])
+def test_adjoint_iterations_tile_and_cell_kernels_agree(time_advance):
+    announce(f"adjoint iterations, tile vs cell kernels (NACA 47 x 15, 60 iterations), time advance {time_advance}")
+    m = naca_mesh(47, 15, 1.2)
+    out = []
+    for kern in (F.KERNELS_TILE, F.KERNELS_CELL):
+        p = form_params(FORMS[3], kernels=kern, cfl=0.5)
+        p.time_advance = time_advance
+        g = F.GPUSolver2(m, p)
+        g.set_state(modulated_state(m, p))
+        res, _ = g.adjoint_solve(wall_sets(m), 1.0, 60, 0.0)
+        out.append((g.adjoint_state(), res.dJ_dalpha))
+        g.close()
+    (pt, at), (pc, ac) = out
+    assert np.linalg.norm(pt - pc) / np.linalg.norm(pc) < 1e-12
+    assert rel(at, ac) < 1e-11
