@@ -720,27 +720,22 @@ __device__ __forceinline__ void edge_alpha(const Phys &ph, const T ra[4], const 
 // correct 2x2 inverse unless compat; then LimiterBarth_device_kernel, GradientGPU.cu:453-502,
 // or Venkatakrishnan).  Per slot i: fl bit 0 = a cell across, bit 1 = a non-periodic
 // neighbour; A = (gC, Sx s, Sy s) for Green-Gauss or (dx, dy) for least squares; Uo = the
-// state across (own state when none); N = vertex i relative to the centroid.  NV: the number of
-// conserved variables formed (they do not mix; the adjoint forms one at a time).
-template <class C, class Slots, int NV = 4, class V = C>
-__device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[NV], const Slots &S, const int fl[3], V vol,
-                                           C gx[NV], C gy[NV]) {
-    // the slot coefficients and vertex offsets keep the accessor's type (the adjoint's are
-    // plain doubles beside dual states)
-    using A_t = typename std::decay<decltype(S.A(0, 0))>::type;
-    using N_t = typename std::decay<decltype(S.N(0, 0))>::type;
+// state across (own state when none); N = vertex i relative to the centroid.  Its reverse mode is
+// grad_limit_adj.
+template <class C, class Slots>
+__device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[4], const Slots &S, const int fl[3], C vol,
+                                           C gx[4], C gy[4]) {
     if (ph.gradient == FVMR_GRA_GREENGAUSS) {
-        const V inv_vol = frcp(vol);
+        const C inv_vol = frcp(vol);
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
+        for (int k = 0; k < 4; k++) {
             C s0 = C(0), s1 = C(0);
 #pragma unroll
             for (int i = 0; i < 3; i++) {
                 // a slot with no cell across has g = 1/2 and the cell's own state, for which the
-                // blend gives U_C exactly, so the plain types blend every slot
-                const A_t g = S.A(i, 0);
-                const bool blend = std::is_floating_point<C>::value || (fl[i] & 1);
-                const C phif = blend ? g * Uc[k] + (A_t(1.0) - g) * S.Uo(i, k) : Uc[k];
+                // blend gives U_C exactly
+                const C g = S.A(i, 0);
+                const C phif = g * Uc[k] + (C(1.0) - g) * S.Uo(i, k);
                 s0 += phif * S.A(i, 1);
                 s1 += phif * S.A(i, 2);
             }
@@ -748,31 +743,31 @@ __device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[NV], const
             gy[k] = inv_vol * s1;
         }
     } else {
-        A_t M[4];   // A^T A
+        C M[4];   // A^T A
 #pragma unroll
         for (int x = 0; x < 2; x++)
 #pragma unroll
             for (int y = 0; y < 2; y++) {
-                A_t acc = A_t(0);
+                C acc = C(0);
 #pragma unroll
                 for (int i = 0; i < 3; i++)
                     if (fl[i] & 2) acc += S.A(i, x) * S.A(i, y);
                 M[x * 2 + y] = acc;
             }
-        A_t det = M[0] * M[3] - M[1] * M[2];
-        const A_t eps = A_t(fvmr::kEPS);
+        C det = M[0] * M[3] - M[1] * M[2];
+        const C eps = C(fvmr::kEPS);
         if (ph.compat_inv) {  // MatrixKernel.h:48-49 as written
-            if (det >= A_t(0) && det < eps) det = eps;
+            if (det >= C(0) && det < eps) det = eps;
             else if (det > -eps) det = -eps;
         } else {
-            if (det >= A_t(0) && det < eps) det = eps;
-            else if (det < A_t(0) && det > -eps) det = -eps;
+            if (det >= C(0) && det < eps) det = eps;
+            else if (det < C(0) && det > -eps) det = -eps;
         }
-        const A_t idet = frcp(det);
-        const A_t i00 = M[3] * idet, i01 = -M[1] * idet, i10 = -M[2] * idet, i11 = M[0] * idet;
+        const C idet = frcp(det);
+        const C i00 = M[3] * idet, i01 = -M[1] * idet, i10 = -M[2] * idet, i11 = M[0] * idet;
         const bool any = (fl[0] | fl[1] | fl[2]) & 2;
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
+        for (int k = 0; k < 4; k++) {
             C a = C(0), b = C(0);
 #pragma unroll
             for (int i = 0; i < 3; i++)
@@ -787,146 +782,94 @@ __device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[NV], const
     if (ph.limiter != FVMR_LIM_NONE) {
         C eps2 = C(0);
         if (ph.limiter == FVMR_LIM_VENKATAKRISHNAN) {
-            const V Kh = (V)ph.venkat_K * fsqrt(vol);
+            const C Kh = (C)ph.venkat_K * fsqrt(vol);
             eps2 = Kh * Kh * Kh;
         }
-        if constexpr (std::is_floating_point<C>::value) {
-            // Straight-line code over the variables, so that their dependent chains overlap: with one
-            // branch per quotient the gradient phase took 1.9 us at any occupancy, 10 cycles an instruction.
-            // Bounds over the cell and its non-periodic neighbours (a slot without one: the cell's own
-            // state, which leaves both bounds as they are); a NaN bound already makes the gradient NaN.
-            C hrel[NV], lrel[NV], phi[NV];
-            bool nan = false;
+        // Straight-line code over the variables, so that their dependent chains overlap: with one
+        // branch per quotient the gradient phase took 1.9 us at any occupancy, 10 cycles an instruction.
+        // Bounds over the cell and its non-periodic neighbours (a slot without one: the cell's own
+        // state, which leaves both bounds as they are); a NaN bound already makes the gradient NaN.
+        C hrel[4], lrel[4], phi[4];
+        bool nan = false;
 #pragma unroll
-            for (int k = 0; k < NV; k++) {
-                C lo = Uc[k], hi = Uc[k];
+        for (int k = 0; k < 4; k++) {
+            C lo = Uc[k], hi = Uc[k];
 #pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    const C o = (!ph.has_periodic || (fl[i] & 2)) ? C(S.Uo(i, k)) : Uc[k];
-                    lo = vmin(lo, o);
-                    hi = vmax(hi, o);
-                }
-                hrel[k] = hi - Uc[k];
-                lrel[k] = lo - Uc[k];
-                nan = nan || isnan(hrel[k]) || isnan(lrel[k]);
+            for (int i = 0; i < 3; i++) {
+                const C o = (!ph.has_periodic || (fl[i] & 2)) ? C(S.Uo(i, k)) : Uc[k];
+                lo = vmin(lo, o);
+                hi = vmax(hi, o);
             }
-            if (ph.limiter == FVMR_LIM_BARTH) {
-                // min over vertices of min(1, hrel / (rel + eps)) (rel > 0) and of
-                // min(1, lrel / (rel - eps)) (rel < 0): division and addition round monotonically, so each
-                // minimum is one division by the extreme rel plus eps, which counts when it is below 1
+            hrel[k] = hi - Uc[k];
+            lrel[k] = lo - Uc[k];
+            nan = nan || isnan(hrel[k]) || isnan(lrel[k]);
+        }
+        if (ph.limiter == FVMR_LIM_BARTH) {
+            // min over vertices of min(1, hrel / (rel + eps)) (rel > 0) and of
+            // min(1, lrel / (rel - eps)) (rel < 0): division and addition round monotonically, so each
+            // minimum is one division by the extreme rel plus eps, which counts when it is below 1
 #pragma unroll
-                for (int k = 0; k < NV; k++) {
-                    C rel[3];
+            for (int k = 0; k < 4; k++) {
+                C rel[3];
 #pragma unroll
-                    for (int jn = 0; jn < 3; jn++) {
-                        const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                        rel[jn] = Un - Uc[k];
-                    }
-                    const C mp = vmax(vmax(rel[0], rel[1]), rel[2]), mn = vmin(vmin(rel[0], rel[1]), rel[2]);
-                    const C dpos = mp + C(fvmr::kEPS), dneg = mn - C(fvmr::kEPS);
-                    const bool cpos = (mp > C(0)) & (hrel[k] < dpos), cneg = (mn < C(0)) & (lrel[k] > dneg);
-                    if constexpr (std::is_same<C, double>::value) {
-                        // one division, of the smaller of the two quotients (compared crosswise: dpos > 0 >
-                        // dneg); where they agree to a rounding either will do
-                        C num = cpos ? hrel[k] : C(1), den = cpos ? dpos : C(1);
-                        const bool neg = cneg & (lrel[k] * den > num * dneg);
-                        num = neg ? lrel[k] : num;
-                        den = neg ? dneg : den;
-                        phi[k] = fdiv(num, den);
-                    } else {
-                        const C qp = fdiv(hrel[k], dpos), qn = fdiv(lrel[k], dneg);
-                        phi[k] = cpos ? tmin(C(1), qp) : C(1);
-                        phi[k] = cneg ? tmin(phi[k], qn) : phi[k];
-                    }
+                for (int jn = 0; jn < 3; jn++) {
+                    const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
+                    rel[jn] = Un - Uc[k];
                 }
-                if (nan) {
-                    // NaN bounds: the vertex loop as the reference writes it
-#pragma unroll
-                    for (int k = 0; k < NV; k++) {
-                        if (!isnan(hrel[k]) && !isnan(lrel[k])) continue;
-                        phi[k] = C(1);
-#pragma unroll
-                        for (int jn = 0; jn < 3; jn++) {
-                            const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                            C rel = Un - Uc[k];
-                            C pn = C(1.0);
-                            if (rel > C(0)) { rel += C(fvmr::kEPS); pn = tmin(C(1), fdiv(hrel[k], rel)); }
-                            else if (rel < C(0)) { rel -= C(fvmr::kEPS); pn = tmin(C(1), fdiv(lrel[k], rel)); }
-                            phi[k] = tmin(phi[k], pn);
-                        }
-                    }
+                const C mp = vmax(vmax(rel[0], rel[1]), rel[2]), mn = vmin(vmin(rel[0], rel[1]), rel[2]);
+                const C dpos = mp + C(fvmr::kEPS), dneg = mn - C(fvmr::kEPS);
+                const bool cpos = (mp > C(0)) & (hrel[k] < dpos), cneg = (mn < C(0)) & (lrel[k] > dneg);
+                if constexpr (std::is_same<C, double>::value) {
+                    // one division, of the smaller of the two quotients (compared crosswise: dpos > 0 >
+                    // dneg); where they agree to a rounding either will do
+                    C num = cpos ? hrel[k] : C(1), den = cpos ? dpos : C(1);
+                    const bool neg = cneg & (lrel[k] * den > num * dneg);
+                    num = neg ? lrel[k] : num;
+                    den = neg ? dneg : den;
+                    phi[k] = fdiv(num, den);
+                } else {
+                    const C qp = fdiv(hrel[k], dpos), qn = fdiv(lrel[k], dneg);
+                    phi[k] = cpos ? tmin(C(1), qp) : C(1);
+                    phi[k] = cneg ? tmin(phi[k], qn) : phi[k];
                 }
-            } else {
+            }
+            if (nan) {
+                // NaN bounds: the vertex loop as the reference writes it
 #pragma unroll
-                for (int k = 0; k < NV; k++) {
+                for (int k = 0; k < 4; k++) {
+                    if (!isnan(hrel[k]) && !isnan(lrel[k])) continue;
                     phi[k] = C(1);
 #pragma unroll
                     for (int jn = 0; jn < 3; jn++) {
-                        const N_t ndx = S.N(jn, 0), ndy = S.N(jn, 1);
-                        const C d2 = gx[k] * ndx + gy[k] * ndy;
-                        const C d1 = (d2 > C(0)) ? hrel[k] : lrel[k];
-                        const C num = (d1 * d1 + eps2) * d2 + C(2.0) * d2 * d2 * d1;
-                        const C den = d1 * d1 + C(2.0) * d2 * d2 + d1 * d2 + eps2;
-                        const C q = fdiv(num, den * d2);
-                        phi[k] = tmin(phi[k], (d2 != C(0)) ? q : C(1));
+                        const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
+                        C rel = Un - Uc[k];
+                        C pn = C(1.0);
+                        if (rel > C(0)) { rel += C(fvmr::kEPS); pn = tmin(C(1), fdiv(hrel[k], rel)); }
+                        else if (rel < C(0)) { rel -= C(fvmr::kEPS); pn = tmin(C(1), fdiv(lrel[k], rel)); }
+                        phi[k] = tmin(phi[k], pn);
                     }
                 }
             }
+        } else {
 #pragma unroll
-            for (int k = 0; k < NV; k++) {
-                gx[k] *= phi[k];
-                gy[k] *= phi[k];
+            for (int k = 0; k < 4; k++) {
+                phi[k] = C(1);
+#pragma unroll
+                for (int jn = 0; jn < 3; jn++) {
+                    const C ndx = S.N(jn, 0), ndy = S.N(jn, 1);
+                    const C d2 = gx[k] * ndx + gy[k] * ndy;
+                    const C d1 = (d2 > C(0)) ? hrel[k] : lrel[k];
+                    const C num = (d1 * d1 + eps2) * d2 + C(2.0) * d2 * d2 * d1;
+                    const C den = d1 * d1 + C(2.0) * d2 * d2 + d1 * d2 + eps2;
+                    const C q = fdiv(num, den * d2);
+                    phi[k] = tmin(phi[k], (d2 != C(0)) ? q : C(1));
+                }
             }
-            return;
         }
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
-            // the dual types, whose derivatives follow the branch that the values take
-            C lo = Uc[k], hi = Uc[k];
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-                if (fl[i] & 2) { lo = fmin(lo, S.Uo(i, k)); hi = fmax(hi, S.Uo(i, k)); }
-            C phi = C(1.0);
-            const C hrel = hi - Uc[k], lrel = lo - Uc[k];
-            if (ph.limiter == FVMR_LIM_BARTH && !isnan(hrel) && !isnan(lrel)) {
-                C dpos = C(0), dneg = C(0);
-#pragma unroll
-                for (int jn = 0; jn < 3; jn++) {
-                    const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                    const C rel = Un - Uc[k];
-                    if (rel > C(0)) dpos = fmax(dpos, rel + C(fvmr::kEPS));
-                    else if (rel < C(0)) dneg = fmin(dneg, rel - C(fvmr::kEPS));
-                }
-                if (dpos > C(0) && hrel < dpos) phi = tmin(phi, fdiv(hrel, dpos));
-                if (dneg < C(0) && lrel > dneg) phi = tmin(phi, fdiv(lrel, dneg));
-            } else if (ph.limiter == FVMR_LIM_BARTH) {
-                // NaN bounds: the vertex loop as the reference writes it
-#pragma unroll
-                for (int jn = 0; jn < 3; jn++) {
-                    const C Un = Uc[k] + gx[k] * S.N(jn, 0) + gy[k] * S.N(jn, 1);
-                    C rel = Un - Uc[k];
-                    C pn = C(1.0);
-                    if (rel > C(0)) { rel += C(fvmr::kEPS); pn = tmin(C(1), fdiv(hrel, rel)); }
-                    else if (rel < C(0)) { rel -= C(fvmr::kEPS); pn = tmin(C(1), fdiv(lrel, rel)); }
-                    phi = tmin(phi, pn);
-                }
-            } else {
-#pragma unroll
-                for (int jn = 0; jn < 3; jn++) {
-                    const N_t ndx = S.N(jn, 0), ndy = S.N(jn, 1);
-                    C pn = C(1.0);
-                    const C d2 = gx[k] * ndx + gy[k] * ndy;
-                    if (d2 != C(0)) {
-                        const C d1 = (d2 > C(0)) ? (hi - Uc[k]) : (lo - Uc[k]);
-                        const C num = (d1 * d1 + eps2) * d2 + C(2.0) * d2 * d2 * d1;
-                        const C den = d1 * d1 + C(2.0) * d2 * d2 + d1 * d2 + eps2;
-                        pn = fdiv(num, den * d2);
-                    }
-                    phi = tmin(phi, pn);
-                }
-            }
-            gx[k] *= phi;
-            gy[k] *= phi;
+        for (int k = 0; k < 4; k++) {
+            gx[k] *= phi[k];
+            gy[k] *= phi[k];
         }
     }
 }

@@ -3,7 +3,9 @@ import numpy as np
 import pytest
 
 import cfd_solver_2d_gpu_amd as F
-from test_gpu_adjoint import announce, modulated_state, naca_mesh, naca_params, rel, wall_sets
+from helpers import SoaMesh
+from test_gpu_adjoint import (announce, modulated_state, naca_mesh, naca_params, rel, standard_geometry_arrays,
+                              wall_sets)
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +82,36 @@ def test_adjoint_iterations_tile_and_cell_kernels_agree(time_advance):
     (pt, at), (pc, ac) = out
     assert np.linalg.norm(pt - pc) / np.linalg.norm(pc) < 1e-12
     assert rel(at, ac) < 1e-11
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_vjp_coordinates_forms_match_differences(form):
+    """Central differences over FP64 geometry with a step of 1e-7 of the local spacing: the areas of the
+    thinnest cells carry 1e-16 / 1e-7 relative, ten times that where edge lengths cancel, hence 1e-5."""
+    announce(f"adjoint coordinate product vs central differences, form {form}")
+    m = naca_mesh(31, 9, 1.3)
+    p = form_params(form)
+    U = modulated_state(m, p)
+    a = F.soa_arrays(m.soa)
+    xy = a["node_xy"].copy()
+    rng = np.random.default_rng(29)
+    psi = rng.standard_normal(U.shape)
+    g = F.GPUSolver2(SoaMesh(standard_geometry_arrays(a, xy)), p)
+    g.set_state(U)
+    _, dxy = g.adjoint_vjp(psi, coords=True)
+    g.close()
+    e0, e1 = a["edge_nodes"]
+    L = np.hypot(xy[0][e1] - xy[0][e0], xy[1][e1] - xy[1][e0])
+    hloc = np.full(xy.shape[1], np.inf)
+    np.minimum.at(hloc, e0, L)
+    np.minimum.at(hloc, e1, L)
+    d = rng.standard_normal(xy.shape) * hloc
+    eps = 1e-7
+    r = []
+    for s in (1, -1):
+        gg = F.GPUSolver2(SoaMesh(standard_geometry_arrays(a, xy + s * eps * d)), p)
+        gg.set_state(U)
+        r.append(gg.stage_rhs())
+        gg.close()
+    fd, ad = np.sum(psi * (r[0] - r[1])) / (2 * eps), np.sum(dxy * d)
+    assert rel(fd, ad) < 1e-5, (fd, ad)
