@@ -1,7 +1,7 @@
 // Forward-mode dual numbers for the adjoint kernels: a value and N directional derivatives.
 // The solver's face-physics templates are instantiated with Dual<N> in place of double where few
-// directions are wanted (the freestream angle, a face's normal).  Branches (min/max, limiter cases, the out-of-range fallback, the farfield regimes)
-// are taken on the values, so derivatives follow the branch the value takes.
+// directions are wanted (the freestream angle, a face's normal).  Branches (min/max, the out-of-range
+// fallback, the farfield regimes) are taken on the values, so derivatives follow the branch the value takes.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -3411,6 +3411,12 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
                            ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin,
                            tile_sizes.empty() ? nullptr : &tile_sizes};
         if ((rc = fvmr::build_tiles(ti, caps, tm))) return bail(rc);
+        // elements whose edges are not the sides of their nodes: the tile kernels take each side from its two
+        // nodes, the cell kernels take the edges' own geometry
+        use_tiles = tm.joined;
+        if (!use_tiles) tm = fvmr::TileMesh();
+    }
+    if (use_tiles) {
         h->tiles = true;
         h->ntiles = tm.ntiles;
         std::vector<V2<double>> txy(tm.nxy.size() / 2);
@@ -3462,8 +3468,10 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             if ((rc = pack(tm.lcxy, &h->t_lcxy)) || (rc = pack(tm.fnrm, &h->t_fnrm))) return bail(rc);
         }
         std::vector<DtRec> dtr(nc);
-        for (int i = 0; i < nc; i++)
-            dtr[i] = DtRec{dtcode[i], tm.dtface[i], h->mixed ? (double)(float)vol[i] : vol[i]};
+        for (int i = 0; i < nc; i++) {
+            const double vol = m->element_volume[h->perm[i]];
+            dtr[i] = DtRec{dtcode[i], tm.dtface[i], h->mixed ? (double)(float)vol : vol};
+        }
         if ((rc = upload(&h->t_dtrec, dtr, h->stream))) return bail(rc);
         if ((rc = upload(&h->tile_case_begin, tm.case_tile_begin, h->stream))) return bail(rc);
         // the host vectors of these uploads end with this block

@@ -341,8 +341,10 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
             out.lcxy.push_back(in.cx[c]);
             out.lcxy.push_back(in.cy[c]);
             int v[3], turned[3];
-            if (!slot_nodes(in, c, v, turned))
-                return set_error(FVMR_ERR_UNSUPPORTED, "an element's edges do not join its nodes");
+            if (!slot_nodes(in, c, v, turned)) {
+                out.joined = false;
+                return FVMR_OK;
+            }
             int w = 0;
             for (int j = 0; j < 3; j++) w |= nid[v[j]] << (kLocalBits * j);
             out.lnodes.push_back(w);

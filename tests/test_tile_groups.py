@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import cfd_solver_2d_gpu_amd as F
-from helpers import vortex_case, wedge_case
+from helpers import SoaMesh, vortex_case, wedge_case
 
 
 def ogrid_case(ni=96, nj=60):
@@ -41,3 +41,27 @@ def test_grouped_tiles_give_the_same_fields(case, tile_cells, precision):
         g.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernels", [F.KERNELS_AUTO, F.KERNELS_TILE])
+def test_edges_that_are_not_sides_use_the_cell_kernels(kernels):
+    """An edge that holds another edge's nodes and geometry: every edge is still standard by itself, but two
+    elements have a side that does not join their nodes, so the tiles cannot form it from them."""
+    print(f"[gpu-case] an edge that is no side of its elements, kernels {kernels}", flush=True)
+    m, p, U = vortex_case(20)
+    a = {k: v.copy() for k, v in F.soa_arrays(m.soa).items()}
+    inner = np.flatnonzero((a["edge_elementR"] >= 0) & (a["edge_periodicPair"] < 0))
+    e, f = inner[7], inner[180]
+    for key in ("edge_nodes", "edge_xy", "edge_normal"):
+        a[key][:, e] = a[key][:, f]
+    a["edge_length"][e] = a["edge_length"][f]
+    out = []
+    for kern in (kernels, F.KERNELS_CELL):
+        p.kernels = kern
+        g = F.GPUSolver2(SoaMesh(a), p)
+        g.set_state(U)
+        g.advance(5, 0.0, 1e9)
+        out.append(g.get_state())
+        g.close()
+    assert np.array_equal(*out)
