@@ -3405,11 +3405,10 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
     // tile records
     fvmr::TileMesh tm;
     if (use_tiles) {
-        std::vector<int> sx(3 * (size_t)nc), sy(3 * (size_t)nc), eL(nf), eR(nf), et(nf), ep(nf), en0(nf), en1(nf);
+        static_assert(sizeof(int2) == sizeof(fvmr::TileSlot) && sizeof(int4) == sizeof(fvmr::TileEdge), "records of ints");
+        std::vector<int> en0(nf), en1(nf);
         std::vector<double> elen(nf), vol(nc);
-        for (size_t k = 0; k < sx.size(); k++) { sx[k] = cslot[k].x; sy[k] = cslot[k].y; }
         for (int e = 0; e < nf; e++) {
-            eL[e] = eint[e].x; eR[e] = eint[e].y; et[e] = eint[e].z; ep[e] = eint[e].w;
             en0[e] = m->edge_nodes[0][eperm[e]]; en1[e] = m->edge_nodes[1][eperm[e]];
             elen[e] = m->edge_length[eperm[e]];
         }
@@ -3420,8 +3419,8 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             emx[e] = m->edge_xy[0][eperm[e]]; emy[e] = m->edge_xy[1][eperm[e]];
             enx[e] = m->edge_normal[0][eperm[e]]; eny[e] = m->edge_normal[1][eperm[e]];
         }
-        fvmr::TileInput ti{nc, nf, sx.data(), sy.data(), cnode.data(), eL.data(), eR.data(), et.data(), ep.data(),
-                           en0.data(), en1.data(), elen.data(), m->node_xy[0], m->node_xy[1], vol.data(),
+        fvmr::TileInput ti{nc, nf, reinterpret_cast<const fvmr::TileSlot *>(cslot.data()), cnode.data(),
+                           reinterpret_cast<const fvmr::TileEdge *>(eint.data()), en0.data(), en1.data(), elen.data(), m->node_xy[0], m->node_xy[1], vol.data(),
                            ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin,
                            tile_sizes.empty() ? nullptr : &tile_sizes};
         if ((rc = fvmr::build_tiles(ti, caps, tm))) return bail(rc);
@@ -3433,54 +3432,25 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
     if (use_tiles) {
         h->tiles = true;
         h->ntiles = tm.ntiles;
-        std::vector<V2<double>> txy(tm.nxy.size() / 2);
-        for (size_t k = 0; k < txy.size(); k++) txy[k] = V2<double>{tm.nxy[2 * k], tm.nxy[2 * k + 1]};
-        std::vector<I3> tgs(tm.gslot.size() / 3), tfc(tm.face.size() / 3);
-        for (size_t k = 0; k < tgs.size(); k++) tgs[k] = I3{tm.gslot[3 * k], tm.gslot[3 * k + 1], tm.gslot[3 * k + 2]};
-        for (size_t k = 0; k < tfc.size(); k++) tfc[k] = I3{tm.face[3 * k], tm.face[3 * k + 1], tm.face[3 * k + 2]};
+        static_assert(sizeof(I3) == 3 * sizeof(int) && sizeof(V4<double>) == 4 * sizeof(double), "packed records");
+        // the packed records as they are; coefficients, centroids and normals rounded to the kernels' geometry type
+        auto put = [&](const auto &v, auto **dst) -> int {
+            HIP_OK(hipMalloc((void **)dst, std::max<size_t>(1, v.size()) * sizeof(v[0])));
+            if (!v.empty()) HIP_OK(hipMemcpyAsync((void *)*dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, h->stream));
+            return FVMR_OK;
+        };
+        std::vector<float> f32[3];
+        auto geo = [&](const std::vector<double> &v, std::vector<float> &f, void **dst) -> int {
+            if (!h->mixed) return put(v, dst);
+            f.assign(v.begin(), v.end());
+            return put(f, dst);
+        };
         if ((rc = upload(&h->t_info, tm.info, h->stream)) || (rc = upload(&h->t_halo, tm.halo, h->stream)) ||
-            (rc = upload(&h->t_lnodes, tm.lnodes, h->stream)) || (rc = upload(&h->t_nxy, txy, h->stream)) ||
-            (rc = upload(&h->t_gslot, tgs, h->stream)) || (rc = upload(&h->t_face, tfc, h->stream)))
+            (rc = upload(&h->t_lnodes, tm.lnodes, h->stream)) || (rc = put(tm.nxy, &h->t_nxy)) ||
+            (rc = put(tm.gslot, &h->t_gslot)) || (rc = put(tm.face, &h->t_face)) ||
+            (rc = geo(tm.gcoef, f32[0], &h->t_gcoef)) || (rc = geo(tm.lcxy, f32[1], &h->t_lcxy)) ||
+            (rc = geo(tm.fnrm, f32[2], &h->t_fnrm)))
             return bail(rc);
-        std::vector<V4<float>> gcf;
-        std::vector<V4<double>> gcd(tm.gcoef.size() / 4);
-        for (size_t k = 0; k < gcd.size(); k++)
-            gcd[k] = V4<double>{tm.gcoef[4 * k], tm.gcoef[4 * k + 1], tm.gcoef[4 * k + 2], tm.gcoef[4 * k + 3]};
-        if (h->mixed) {
-            gcf.resize(gcd.size());
-            for (size_t k = 0; k < gcd.size(); k++)
-                gcf[k] = V4<float>{(float)gcd[k].x, (float)gcd[k].y, (float)gcd[k].z, (float)gcd[k].w};
-            V4<float> *d = nullptr;
-            if ((rc = upload(&d, gcf, h->stream))) return bail(rc);
-            h->t_gcoef = d;
-        } else {
-            V4<double> *d = nullptr;
-            if ((rc = upload(&d, gcd, h->stream))) return bail(rc);
-            h->t_gcoef = d;
-        }
-        {
-            // centroids and normals as the kernels would recompute them (standard geometry:
-            // the caller's values), rounded to the kernels' geometry type
-            auto pack = [&](const std::vector<double> &xy, void **dst) -> int {
-                if (h->mixed) {
-                    std::vector<V2<float>> v(xy.size() / 2);
-                    for (size_t k = 0; k < v.size(); k++) v[k] = V2<float>{(float)xy[2 * k], (float)xy[2 * k + 1]};
-                    V2<float> *d = nullptr;
-                    int r = upload(&d, v, h->stream);
-                    *dst = d;
-                    if (!r && hipStreamSynchronize(h->stream) != hipSuccess) r = set_error(FVMR_ERR_HIP, "tile upload failed");
-                    return r;
-                }
-                std::vector<V2<double>> v(xy.size() / 2);
-                for (size_t k = 0; k < v.size(); k++) v[k] = V2<double>{xy[2 * k], xy[2 * k + 1]};
-                V2<double> *d = nullptr;
-                int r = upload(&d, v, h->stream);
-                *dst = d;
-                if (!r && hipStreamSynchronize(h->stream) != hipSuccess) r = set_error(FVMR_ERR_HIP, "tile upload failed");
-                return r;
-            };
-            if ((rc = pack(tm.lcxy, &h->t_lcxy)) || (rc = pack(tm.fnrm, &h->t_fnrm))) return bail(rc);
-        }
         std::vector<DtRec> dtr(nc);
         for (int i = 0; i < nc; i++) {
             const double vol = m->element_volume[h->perm[i]];

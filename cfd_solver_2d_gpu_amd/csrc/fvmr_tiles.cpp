@@ -20,21 +20,19 @@ namespace fvmr {
 
 namespace {
 
-// Hilbert index of (x, y) on an n x n grid, n = 2^order (the textbook xy -> d walk).
-uint64_t hilbert_d(uint32_t x, uint32_t y, int order) {
-    const uint32_t n = 1u << order;
-    uint64_t d = 0;
-    for (uint32_t s = n >> 1; s > 0; s >>= 1) {
-        const uint32_t rx = (x & s) ? 1u : 0u;
-        const uint32_t ry = (y & s) ? 1u : 0u;
-        d += (uint64_t)s * s * ((3u * rx) ^ ry);
-        if (ry == 0) {
-            if (rx == 1) {
-                x = n - 1 - x;
-                y = n - 1 - y;
-            }
-            std::swap(x, y);
-        }
+// Hilbert index of (x, y) on an n x n grid, n = 2^order (the textbook xy -> d walk, without its branches).
+uint32_t hilbert_d(uint32_t x, uint32_t y, int order) {
+    const uint32_t all = (1u << order) - 1;
+    uint32_t d = 0;
+    for (int b = order - 1; b >= 0; b--) {
+        const uint32_t rx = (x >> b) & 1u, ry = (y >> b) & 1u;
+        d = (d << 2) | ((3u * rx) ^ ry);
+        const uint32_t flip = (0u - (rx & ~ry & 1u)) & all;   // turn the quadrant
+        x ^= flip;
+        y ^= flip;
+        const uint32_t t = (x ^ y) & (ry - 1u);               // and swap its axes
+        x ^= t;
+        y ^= t;
     }
     return d;
 }
@@ -49,7 +47,7 @@ double gg_weight(const TileInput &in, int c, int e, int o, bool periodic) {
     if (o < 0) return 0.5;
     const double fx = in.mx[e], fy = in.my[e];
     double Fx = in.cx[o], Fy = in.cy[o];
-    const int pe = in.epair[e];
+    const int pe = in.edge[e].pair;
     if (periodic && pe >= 0) {
         Fx += fx - in.mx[pe];
         Fy += fy - in.my[pe];
@@ -67,7 +65,7 @@ double gg_weight(const TileInput &in, int c, int e, int o, bool periodic) {
 bool slot_nodes(const TileInput &in, int c, int v[3], int turned[3]) {
     int a[3], b[3];
     for (int j = 0; j < 3; j++) {
-        const int x = in.cslot_x[(size_t)j * in.nc + c], e = x & ((1 << 28) - 1);
+        const int x = in.cslot[(size_t)j * in.nc + c].x, e = x & ((1 << 28) - 1);
         a[j] = in.en0[e];
         b[j] = in.en1[e];
         if (x & (1 << 30)) std::swap(a[j], b[j]);   // the cell is R: seen from it the edge runs the other way
@@ -98,15 +96,33 @@ std::vector<int> hilbert_order(int nc, const double *cx, const double *cy) {
     const int order = 16;
     const double span = std::max(std::max(x1 - x0, y1 - y0), 1e-300);
     const double scale = ((1u << order) - 1) / span;
-    std::vector<std::pair<uint64_t, int>> key(nc);
+    struct Key {
+        uint32_t d;
+        int c;
+    };
+    std::vector<Key> key(nc), next(nc);
     for (int c = 0; c < nc; c++) {
         const uint32_t ix = (uint32_t)std::min<double>((cx[c] - x0) * scale, (1u << order) - 1);
         const uint32_t iy = (uint32_t)std::min<double>((cy[c] - y0) * scale, (1u << order) - 1);
         key[c] = {hilbert_d(ix, iy, order), c};
     }
-    std::sort(key.begin(), key.end());
+    // by 11 bits at a time, each pass stable (393,216 cells: 31 ms with a comparison sort of the walk's branches,
+    // 12 ms so)
+    constexpr int kBits = 11;
+    for (int shift = 0; shift < 2 * order; shift += kBits) {
+        size_t at[1 << kBits] = {0};
+        for (const Key &k : key) at[(k.d >> shift) & ((1u << kBits) - 1)]++;
+        size_t sum = 0;
+        for (size_t &n : at) {
+            const size_t m = n;
+            n = sum;
+            sum += m;
+        }
+        for (const Key &k : key) next[at[(k.d >> shift) & ((1u << kBits) - 1)]++] = k;
+        key.swap(next);
+    }
     std::vector<int> order_out(nc);
-    for (int i = 0; i < nc; i++) order_out[i] = key[i].second;
+    for (int i = 0; i < nc; i++) order_out[i] = key[i].c;
     return order_out;
 }
 
@@ -246,19 +262,48 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
         caps.lcells > kLocalNone || caps.nodes > kLocalNone || caps.faces > kLocalNone)
         return set_error(FVMR_ERR_INVALID_ARG, "bad tile capacities");
     for (int e = 0; e < nf; e++) {
-        const int t = in.etype[e];
+        const int t = in.edge[e].type;
         if (t != -1 && (t <= kBcBase || t - kBcBase > 127))
             return set_error(FVMR_ERR_UNSUPPORTED, "boundary type outside the tile kernels' code range");
     }
     out = TileMesh();
     out.dtface.assign(nc, 0);
+    // room for tiles of the usual halo (no page is touched before it is written)
+    out.halo.reserve(nc);
+    out.nxy.reserve(2 * (size_t)nc);
+    out.lnodes.reserve(2 * (size_t)nc);
+    out.lcxy.reserve(4 * (size_t)nc);
+    out.gslot.reserve(4 * (size_t)nc + nc / 2);
+    out.gcoef.reserve(6 * (size_t)nc);
+    out.face.reserve(7 * (size_t)nc);
+    out.fnrm.reserve(5 * (size_t)nc);
+    auto grow = [](auto &v, size_t n) {
+        v.resize(v.size() + n);
+        return v.data() + v.size() - n;
+    };
     // stamps: lid valid when lst == current tile
     std::vector<int> lst(nc, -1), lid(nc, 0), fst(nf, -1), fid(nf, 0);
     int nv = 0;
     for (int c = 0; c < 3 * nc; c++) nv = std::max(nv, in.cnode[c] + 1);
     for (int e = 0; e < nf; e++) nv = std::max(nv, std::max(in.en0[e], in.en1[e]) + 1);
     std::vector<int> nst(nv, -1), nid(nv, 0);
-    std::vector<int> cells, faces, nodes, gturn;
+    std::vector<int> cells, faces, nodes;
+    // what every tile that holds a cell packs of it
+    struct Cell {
+        int v[3], turned[3];
+        double gw[3];
+    };
+    std::vector<Cell> rec(nc);
+    for (int c = 0; c < nc; c++) {
+        if (!slot_nodes(in, c, rec[c].v, rec[c].turned)) {
+            out.joined = false;
+            return FVMR_OK;
+        }
+        for (int j = 0; j < 3; j++) {
+            const TileSlot sl = in.cslot[(size_t)j * nc + c];
+            rec[c].gw[j] = gg_weight(in, c, sl.x & ((1 << 28) - 1), sl.y, (sl.x & (1 << 28)) != 0);
+        }
+    }
     int stamp = 0;
 
     // Builds the sets of the candidate tile [c0, c0+s); false when a capacity is exceeded.
@@ -280,25 +325,25 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
         for (int i = 0; i < s; i++) add_cell(c0 + i);
         for (int i = 0; i < s; i++)
             for (int j = 0; j < 3; j++) {
-                const int o = in.cslot_y[(size_t)j * nc + c0 + i];
+                const int o = in.cslot[(size_t)j * nc + c0 + i].y;
                 if (o >= 0) add_cell(o);
             }
         nG = (int)cells.size();
         if (nG > caps.gcells) return false;
         for (int i = s; i < nG; i++)
             for (int j = 0; j < 3; j++) {
-                const int o = in.cslot_y[(size_t)j * nc + cells[i]];
+                const int o = in.cslot[(size_t)j * nc + cells[i]].y;
                 if (o >= 0) add_cell(o);
             }
         if ((int)cells.size() > caps.lcells) return false;
         for (int i = 0; i < s; i++)
-            for (int j = 0; j < 3; j++) add_face(in.cslot_x[(size_t)j * nc + c0 + i] & ((1 << 28) - 1));
+            for (int j = 0; j < 3; j++) add_face(in.cslot[(size_t)j * nc + c0 + i].x & ((1 << 28) - 1));
         nFF = (int)faces.size();
         if (nFF > caps.ffaces) return false;
         for (int i = s; i < nG; i++)
-            for (int j = 0; j < 3; j++) add_face(in.cslot_x[(size_t)j * nc + cells[i]] & ((1 << 28) - 1));
+            for (int j = 0; j < 3; j++) add_face(in.cslot[(size_t)j * nc + cells[i]].x & ((1 << 28) - 1));
         for (size_t k = 0; k < faces.size(); k++) {
-            const int pe = in.epair[faces[k]];
+            const int pe = in.edge[faces[k]].pair;
             if (pe >= 0) add_face(pe);
             if ((int)faces.size() > caps.faces) return false;
         }
@@ -333,58 +378,55 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
                                      (int)out.halo.size(), (int)(out.nxy.size() / 2), (int)(out.face.size() / 3),
                                      (int)out.lnodes.size(), (int)(out.gcoef.size() / 4), cs};
         out.info.insert(out.info.end(), info, info + kTileInfo);
-        for (int i = s; i < nL; i++) out.halo.push_back(cells[i]);
-        gturn.clear();
-        for (int v : nodes) { out.nxy.push_back(in.node_x[v]); out.nxy.push_back(in.node_y[v]); }
+        out.halo.insert(out.halo.end(), cells.begin() + s, cells.end());
+        double *nxy = grow(out.nxy, 2 * (size_t)nN);
+        for (int k = 0; k < nN; k++) {
+            nxy[2 * k] = in.node_x[nodes[k]];
+            nxy[2 * k + 1] = in.node_y[nodes[k]];
+        }
+        double *lcxy = grow(out.lcxy, 2 * (size_t)nL);
+        int *lnodes = grow(out.lnodes, nL);
         for (int i = 0; i < nL; i++) {
             const int c = cells[i];
-            out.lcxy.push_back(in.cx[c]);
-            out.lcxy.push_back(in.cy[c]);
-            int v[3], turned[3];
-            if (!slot_nodes(in, c, v, turned)) {
-                out.joined = false;
-                return FVMR_OK;
-            }
+            lcxy[2 * i] = in.cx[c];
+            lcxy[2 * i + 1] = in.cy[c];
             int w = 0;
-            for (int j = 0; j < 3; j++) w |= nid[v[j]] << (kLocalBits * j);
-            out.lnodes.push_back(w);
-            for (int j = 0; j < 3 && i < nG; j++) gturn.push_back(turned[j]);
+            for (int j = 0; j < 3; j++) w |= nid[rec[c].v[j]] << (kLocalBits * j);
+            lnodes[i] = w;
         }
+        int *gslot = grow(out.gslot, 3 * (size_t)nG);
+        double *gcoef = grow(out.gcoef, 4 * (size_t)nG);
         for (int i = 0; i < nG; i++) {
             const int c = cells[i];
-            double gw[3];
+            int fw = 0;
             for (int j = 0; j < 3; j++) {
-                const int x = in.cslot_x[(size_t)j * nc + c], o = in.cslot_y[(size_t)j * nc + c];
+                const int x = in.cslot[(size_t)j * nc + c].x, o = in.cslot[(size_t)j * nc + c].y;
                 const int e = x & ((1 << 28) - 1);
                 int w = fid[e] | ((o >= 0 ? lid[o] : kLocalNone) << kGsOutShift);
+                fw |= fid[e] << (kLocalBits * j);
                 if (x & (1 << 30)) w |= kGsIsR;
                 if (x & (1 << 28)) w |= kGsPeriodic;
-                if (gturn[3 * (size_t)i + j]) w |= kGsTurned;
-                out.gslot.push_back(w);
-                gw[j] = gg_weight(in, c, e, o, (x & (1 << 28)) != 0);
+                if (rec[c].turned[j]) w |= kGsTurned;
+                gslot[3 * i + j] = w;
+                gcoef[4 * i + j] = rec[c].gw[j];
             }
-            if (i < s) {
-                int w = 0;
-                for (int j = 0; j < 3; j++) w |= fid[in.cslot_x[(size_t)j * nc + c] & ((1 << 28) - 1)] << (kLocalBits * j);
-                out.dtface[c] = w;
-            }
-            out.gcoef.insert(out.gcoef.end(), {gw[0], gw[1], gw[2], in.vol[c]});
+            if (i < s) out.dtface[c] = fw;
+            gcoef[4 * i + 3] = in.vol[c];
         }
+        int *face = grow(out.face, 3 * (size_t)nF);
+        double *fnrm = grow(out.fnrm, 2 * (size_t)nF);
         for (int k = 0; k < nF; k++) {
             const int e = faces[k];
-            const int t = in.etype[e];
-            const int bc = (t == -1) ? 0 : t - kBcBase;
+            const TileEdge &ed = in.edge[e];
+            const int bc = (ed.type == -1) ? 0 : ed.type - kBcBase;
             auto loc = [&](int c) { return (c >= 0 && lst[c] == stamp) ? lid[c] : kLocalNone; };
-            const int pe = in.epair[e];
-            const int pl = (pe >= 0 && fst[pe] == stamp) ? fid[pe] : kLocalNone;
+            const int pl = (ed.pair >= 0 && fst[ed.pair] == stamp) ? fid[ed.pair] : kLocalNone;
             const float lf = (float)in.elen[e];
-            int lbits;
-            std::memcpy(&lbits, &lf, sizeof(int));
-            out.face.push_back(nid[in.en0[e]] | (nid[in.en1[e]] << kLocalBits) | (bc << kBcShift));
-            out.face.push_back(loc(in.eL[e]) | (loc(in.eR[e]) << kLocalBits) | (pl << (2 * kLocalBits)));
-            out.face.push_back(lbits);
-            out.fnrm.push_back(in.nx[e]);
-            out.fnrm.push_back(in.ny[e]);
+            face[3 * k] = nid[in.en0[e]] | (nid[in.en1[e]] << kLocalBits) | (bc << kBcShift);
+            face[3 * k + 1] = loc(ed.L) | (loc(ed.R) << kLocalBits) | (pl << (2 * kLocalBits));
+            std::memcpy(&face[3 * k + 2], &lf, sizeof(int));
+            fnrm[2 * k] = in.nx[e];
+            fnrm[2 * k + 1] = in.ny[e];
         }
         out.max_nL = std::max(out.max_nL, nL); out.max_nG = std::max(out.max_nG, nG);
         out.max_nF = std::max(out.max_nF, nF); out.max_nFF = std::max(out.max_nFF, nFF);

@@ -60,13 +60,20 @@ struct TileMesh {
     int64_t sum_nL = 0, sum_nG = 0, sum_nF = 0, sum_nN = 0;
 };
 
+// A cell's slot: edge | flags (bit 30 cell is R, bit 28 periodic); the cell across the face, -1 none.
+struct TileSlot {
+    int x, y;
+};
+struct TileEdge {
+    int L, R, type, pair;
+};
+
 // Device-order inputs of the tile builder (all in the device numbering).
 struct TileInput {
     int nc, nf;
-    const int *cslot_x;   // [3][nc] edge | flags (bit 30 cell is R, bit 28 periodic)
-    const int *cslot_y;   // [3][nc] cell across the face, -1 none
+    const TileSlot *cslot;  // [3][nc]
     const int *cnode;     // [3][nc] global node id of vertex j
-    const int *eL, *eR, *etype, *epair;  // per edge
+    const TileEdge *edge;   // per edge
     const int *en0, *en1; // edge nodes (reference edge order)
     const double *elen;   // edge length
     const double *node_x, *node_y;
