@@ -290,8 +290,7 @@ class GPUSolver2:
         check(lib().fvmr_set_state(self._h, rows), "fvmr_set_state")
 
     def get_state(self):
-        U = np.zeros((4, self.n))
-        U, rows = _rows(U)
+        U, rows = _rows(np.empty((4, self.n)))
         check(lib().fvmr_get_state(self._h, rows), "fvmr_get_state")
         return U
 
@@ -343,9 +342,9 @@ class GPUSolver2:
         """FieldWriter::update_nodeField on the device: (ruvp 4 x num_node, Cp, Ma) of the
         current state (FVMR/src/output/FieldWriter.cpp:371-452)."""
         nv = self.mesh.soa.num_node
-        R = np.zeros((4, nv))
-        cp = np.zeros(nv)
-        ma = np.zeros(nv)
+        R = np.empty((4, nv))
+        cp = np.empty(nv)
+        ma = np.empty(nv)
         R, rows = _rows(R)
         check(lib().fvmr_node_field(self._h, rows, _dptr(cp), _dptr(ma)), "fvmr_node_field")
         return R, cp, ma
@@ -449,7 +448,7 @@ class GPUSolver2:
         return out, (dxy.reshape(-1, 2).T.copy() if coords else None)
 
     def adjoint_state(self):
-        P, rows = _rows(np.zeros((4, self.n)))
+        P, rows = _rows(np.empty((4, self.n)))
         check(lib().fvmr_adjoint_state(self._h, rows), "fvmr_adjoint_state")
         return P
 
@@ -508,8 +507,7 @@ class BatchSolver:
         check(lib().fvmr_batch_set_state(self._h, c, rows), "fvmr_batch_set_state")
 
     def get_state(self, c):
-        U = np.zeros((4, self.meshes[c].num_element))
-        U, rows = _rows(U)
+        U, rows = _rows(np.empty((4, self.meshes[c].num_element)))
         check(lib().fvmr_batch_get_state(self._h, c, rows), "fvmr_batch_get_state")
         return U
 

@@ -1613,9 +1613,7 @@ int adj_coords(fvmr_solver *h, const S4 *U, const S4 *psi, double *dxy) {
     HIP_OK(hipGetLastError());
     k_adj_coords_sum<<<grid_of(h->nv), kBlock, 0, h->stream>>>(m, h->nv, h->nc_off, h->nc_cells, w->enode, w->xval, w->dxy);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(dxy, w->dxy, nv * sizeof(V2<double>), hipMemcpyDeviceToHost, h->stream));
-    HIP_OK(hipStreamSynchronize(h->stream));
-    return FVMR_OK;
+    return to_host(h, &w->dxy->x, 2 * nv, 1, &dxy);
 }
 
 // Host copy of a caller-order field into device order.
@@ -1766,8 +1764,8 @@ int fvmr_adjoint_solve(fvmr_handle *h, int nsets, const int *set_offsets, const 
     // J and its explicit parts from the node Cp of U
     if ((rc = node_field_device(h))) return rc;
     std::vector<double> Cp(nv);
-    HIP_OK(hipMemcpyAsync(Cp.data(), h->node_buf + 4 * (size_t)nv, nv * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_OK(hipStreamSynchronize(h->stream));
+    double *cp_row = Cp.data();
+    if ((rc = to_host(h, h->node_buf + 4 * (size_t)nv, nv, 1, &cp_row))) return rc;
     const double *inf = h->p.inf_ruvp;
     const double alpha = std::atan2(inf[2], inf[1]), sa = std::sin(alpha), ca = std::cos(alpha);
     const double p_dyn = 0.5 * inf[0] * (inf[1] * inf[1] + inf[2] * inf[2]);
