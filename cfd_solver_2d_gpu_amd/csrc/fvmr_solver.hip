@@ -2270,24 +2270,41 @@ __global__ __launch_bounds__(kBlock) void k_vertex_colors(int nv, const int *__r
     vertices[(size_t)6 * v + 5] = c.z;
 }
 
-// ReferenceData::calculate_edgeSet_force (FieldWriter.cpp:174-205): one thread per set, its
-// edges in set order.  edge e: nodes en[2e], en[2e+1], geometry eg[3e..3e+2] = nx, ny, L.
-__global__ void k_surface_force(int nsets, const int *__restrict__ off, const int *__restrict__ en,
-                                const double *__restrict__ eg, const double *__restrict__ Cp, double S_ref,
-                                double *__restrict__ out) {
+// cd, cl += the terms (x, y) of the wave's first n lanes, one after another in lane order.
+__device__ __forceinline__ void add_in_order(double x, double y, int n, double &cd, double &cl) {
 #pragma clang fp contract(off)
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsets) return;
+    for (int l = 0; l < n; l++) {
+        cd += __shfl(x, l);
+        cl += __shfl(y, l);
+    }
+}
+
+// ReferenceData::calculate_edgeSet_force (FieldWriter.cpp:174-205): one wave per set, its edges added in set
+// order.  edge e: nodes en[2e], en[2e+1], geometry eg[3e..3e+2] = nx, ny, L.  The chain of sums is what the
+// result's bits depend on; the loads before each term do not have to be in it: 64 edges' terms are formed side
+// by side (the boundary of a 131,406-cell wedge: the call 193 us with one thread per set, so 98 us).
+__global__ __launch_bounds__(64) void k_surface_force(const int *__restrict__ off, const int *__restrict__ en,
+                                                      const double *__restrict__ eg, const double *__restrict__ Cp, double S_ref,
+                                                      double *__restrict__ out) {
+#pragma clang fp contract(off)
+    const int s = blockIdx.x;
     const double one_on_Sref = 1 / S_ref;
     double cd = 0.0, cl = 0.0;
-    for (int k = off[s]; k < off[s + 1]; k++) {
-        const double cp = 0.5 * (Cp[en[2 * k]] + Cp[en[2 * k + 1]]);
-        const double dC = cp * one_on_Sref * eg[3 * k + 2];
-        cd += dC * eg[3 * k];
-        cl += dC * eg[3 * k + 1];
+    for (int k0 = off[s], k1 = off[s + 1]; k0 < k1; k0 += 64) {
+        const int k = k0 + threadIdx.x;
+        double x = 0.0, y = 0.0;
+        if (k < k1) {
+            const double cp = 0.5 * (Cp[en[2 * k]] + Cp[en[2 * k + 1]]);
+            const double dC = cp * one_on_Sref * eg[3 * k + 2];
+            x = dC * eg[3 * k];
+            y = dC * eg[3 * k + 1];
+        }
+        add_in_order(x, y, min(64, k1 - k0), cd, cl);
     }
-    out[2 * s] = cd;
-    out[2 * s + 1] = cl;
+    if (threadIdx.x == 0) {
+        out[2 * s] = cd;
+        out[2 * s + 1] = cl;
+    }
 }
 
 // k_surface_force without the node-field buffer: the caller's edge ids of set s,
@@ -2295,35 +2312,40 @@ __global__ void k_surface_force(int nsets, const int *__restrict__ off, const in
 // ascending, nb entries; every id was checked on the host to be there) and the Cp of each
 // edge node is formed where it is used, with the arithmetic of k_node_field, so the sums
 // equal k_surface_force's bit for bit.  Results: cx[s], cy[s].
-__global__ void k_surface_force_direct(int nsets, const int *__restrict__ off, const int *__restrict__ edges, int nb,
+__global__ __launch_bounds__(64) void k_surface_force_direct(const int *__restrict__ off, const int *__restrict__ edges, int nb,
                                        const int *__restrict__ bref, const int2 *__restrict__ bnodes,
                                        const V4<double> *__restrict__ bgeo, const int *__restrict__ noff,
                                        const int *__restrict__ ncells, const S4 *__restrict__ U, double gamma,
                                        double p_inf, double p_dyn, double S_ref, double *__restrict__ cx,
                                        double *__restrict__ cy) {
 #pragma clang fp contract(off)
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsets) return;
+    const int s = blockIdx.x;
     const double one_on_Sref = 1 / S_ref;
     double cd = 0.0, cl = 0.0;
-    for (int k = off[s]; k < off[s + 1]; k++) {
-        const int e = edges[k];
-        int lo = 0, hi = nb - 1;   // bref[lo] <= e <= bref[hi] holds for every listed id
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (bref[mid] < e) lo = mid + 1;
-            else hi = mid;
+    for (int k0 = off[s], k1 = off[s + 1]; k0 < k1; k0 += 64) {
+        const int k = k0 + threadIdx.x;
+        double x = 0.0, y = 0.0;
+        if (k < k1) {
+            const int e = edges[k];
+            int lo = 0, hi = nb - 1;   // bref[lo] <= e <= bref[hi] holds for every listed id
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (bref[mid] < e) lo = mid + 1;
+                else hi = mid;
+            }
+            const int2 nd = bnodes[lo];
+            const V4<double> g = bgeo[lo];
+            double m0[4], m1[4];
+            node_mean_ruvp(nd.x, noff, ncells, U, gamma, m0);
+            node_mean_ruvp(nd.y, noff, ncells, U, gamma, m1);
+            const double cp = 0.5 * (node_cp(m0[3], p_inf, p_dyn) + node_cp(m1[3], p_inf, p_dyn));
+            const double dC = cp * one_on_Sref * g.z;
+            x = dC * g.x;
+            y = dC * g.y;
         }
-        const int2 nd = bnodes[lo];
-        const V4<double> g = bgeo[lo];
-        double m0[4], m1[4];
-        node_mean_ruvp(nd.x, noff, ncells, U, gamma, m0);
-        node_mean_ruvp(nd.y, noff, ncells, U, gamma, m1);
-        const double cp = 0.5 * (node_cp(m0[3], p_inf, p_dyn) + node_cp(m1[3], p_inf, p_dyn));
-        const double dC = cp * one_on_Sref * g.z;
-        cd += dC * g.x;
-        cl += dC * g.y;
+        add_in_order(x, y, min(64, k1 - k0), cd, cl);
     }
+    if (threadIdx.x != 0) return;
     cx[s] = cd;
     cy[s] = cl;
 }
@@ -4029,7 +4051,7 @@ int fvmr_surface_force(fvmr_handle *h, int nsets, const int *set_offsets, const 
         release();
         return rc ? rc : set_error(FVMR_ERR_HIP, "hipMalloc surface force");
     }
-    k_surface_force<<<(nsets + 63) / 64, 64, 0, h->stream>>>(nsets, d_off, d_en, d_eg, h->node_buf + 4 * (size_t)h->nv,
+    k_surface_force<<<nsets, 64, 0, h->stream>>>(d_off, d_en, d_eg, h->node_buf + 4 * (size_t)h->nv,
                                                            S_ref, d_out);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(out.data(), d_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream);
@@ -4070,8 +4092,8 @@ int fvmr_surface_force_noalloc(fvmr_handle *h, int nsets, const int *set_offsets
     if (ne > 0) HIP_OK(hipMemcpyAsync(d_edges, set_edges, (size_t)ne * sizeof(int), hipMemcpyHostToDevice, h->stream));
     const double *inf = h->p.inf_ruvp;
     const double V2 = inf[1] * inf[1] + inf[2] * inf[2];
-    k_surface_force_direct<<<(nsets + 63) / 64, 64, 0, h->stream>>>(
-        nsets, d_off, d_edges, (int)h->bedge_ref.size(), h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev,
+    k_surface_force_direct<<<nsets, 64, 0, h->stream>>>(
+        d_off, d_edges, (int)h->bedge_ref.size(), h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev,
         h->nc_off, h->nc_cells, h->Ubuf[h->cur], h->p.gamma, inf[3], 0.5 * inf[0] * V2, S_ref, d_cx, d_cy);
     HIP_OK(hipGetLastError());
     HIP_OK(hipMemcpyAsync(Cx, d_cx, (size_t)nsets * sizeof(double), hipMemcpyDeviceToHost, h->stream));
