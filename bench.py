@@ -415,14 +415,12 @@ def config_c4(ncases=256, steps=500, seed=0):
 
 
 def adjoint_product_bytes(nc, nf, nv):
-    """Algorithmic bytes of one adjoint product (k_adj_faces, k_adj_vjp, k_adj_update), every array
-    once, intermediates written and read: per cell the state (32), the steady state's gradients
-    (64), psi in, psi of the stage start and psi out (3 x 32), cell geometry (32), face slots (24),
-    vertices (12), the per-cell share written and read (2 x 32), dJ/dU (32) and the pseudo-time
-    step (8); per face the L/R/BC record (16), normal and length (32), midpoint (16), the two
-    sides' face adjoints written and read (2 x 64) and the two per-side shares written and read
-    (2 x 64); per node its coordinates (16)."""
-    return nc * (32 + 64 + 3 * 32 + 32 + 24 + 12 + 2 * 32 + 32 + 8) + nf * (16 + 32 + 16 + 2 * 64 + 2 * 64) + nv * 16
+    """Algorithmic bytes of one adjoint product and its stage (k_adj_tile), every array once and
+    nothing in between: per cell the state (32), the steady state's gradients (64), psi in, psi of
+    the stage start and psi out (3 x 32), cell geometry (32), face slots (24), vertices (12), dJ/dU
+    (32) and the pseudo-time step (8); per face the L/R/BC record (16), normal and length (32) and
+    midpoint (16); per node its coordinates (16)."""
+    return nc * (32 + 64 + 3 * 32 + 32 + 24 + 12 + 32 + 8) + nf * (16 + 32 + 16) + nv * 16
 
 
 def config_c5(primal_iters=260000, adjoint_iters=150000, fd_iters=140000, h=1e-6):
