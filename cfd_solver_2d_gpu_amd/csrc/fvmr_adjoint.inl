@@ -872,7 +872,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_update(Mesh<double> m, const S4 
 }
 
 // A scheme of k_adj_tile beside kTileAny and kTileGg: Green-Gauss, Roe, linear reconstruction and any limiter
-// (162 against 180 VGPRs: three work-groups to a CU, not two).
+// (164 against 180 VGPRs: three work-groups to a CU, not two).
 constexpr int kTileGgRoe = 3;
 
 // One product with (dr/dU)^T and its pseudo-time stage over the tiles (the work of k_adj_faces, k_adj_vjp and
