@@ -338,6 +338,17 @@ class GPUSolver2:
         """Replay runs of three steps from captured HIP graphs (default off)."""
         check(lib().fvmr_use_graphs(self._h, 1 if on else 0), "fvmr_use_graphs")
 
+    def use_resident(self, on=True, max_polls=-1):
+        """Let the resident kernel serve runs of steps where it can (default on); max_polls: polls after
+        which a wait inside it gives up (-1: the default)."""
+        check(lib().fvmr_use_resident(self._h, 1 if on else 0, max_polls), "fvmr_use_resident")
+
+    def resident_steps(self):
+        """Steps and pseudo-time iterations that the resident kernel has done on this handle."""
+        n = C.c_longlong()
+        check(lib().fvmr_resident_steps(self._h, C.byref(n)), "fvmr_resident_steps")
+        return n.value
+
     def node_field(self):
         """FieldWriter::update_nodeField on the device: (ruvp 4 x num_node, Cp, Ma) of the
         current state (FVMR/src/output/FieldWriter.cpp:371-452)."""

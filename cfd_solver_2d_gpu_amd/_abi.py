@@ -117,6 +117,8 @@ SIGNATURES = {
     "fvmr_device_division": (C.c_int, [C.c_int, _dp, _dp, _dp, _dp]),
     "fvmr_node_field": (C.c_int, [C.c_void_p, _dp * 4, _dp, _dp]),
     "fvmr_use_graphs": (C.c_int, [C.c_void_p, C.c_int]),
+    "fvmr_use_resident": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
+    "fvmr_resident_steps": (C.c_int, [C.c_void_p, C.POINTER(C.c_longlong)]),
     "fvmr_autotune": (C.c_int, [C.POINTER(MeshSoA), C.POINTER(Params), C.c_int, _ip, _ip, _dp]),
     "fvmr_autotune_batch": (C.c_int, [C.c_int, C.POINTER(C.POINTER(MeshSoA)), C.POINTER(Params), C.c_int, _ip, _ip,
                                       _dp, _dp]),

@@ -1699,9 +1699,10 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
         const int a = h->cur, b = (a + 1) % 3, c = (a + 2) % 3;
         S4 *Ua = h->Ubuf[a], *Ub = h->Ubuf[b], *Uc = h->Ubuf[c];
         const bool check = (it % kAdjCheck == 0);
-        if (h->run_steady_kernel && !check) {   // the iterations up to the next check in one launch
+        if (h->run_on && h->run_steady_kernel && !check) {   // the iterations up to the next check in one launch
             const int n = std::min(kAdjCheck - it % kAdjCheck, max_iters - it);
             if ((rc = launch_run<double, double>(h, n, -1, true))) return rc;
+            h->run_steps += n;
             it += n;
             continue;
         }

@@ -1814,7 +1814,7 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
 // slots and states stay in LDS and registers, the new states of the cells that other tiles need
 // are exchanged through global memory after each stage, and the time step's minimum goes through
 // one more work-group, which only reduces.  The launch is cooperative, so all work-groups run at
-// once or the launch fails; every wait ends after kRunSpin polls at the latest.
+// once or the launch fails; every wait ends after RunArgs::polls polls at the latest.
 //
 // Exchange.  A double travels as two 64-bit words, each half of its bits with the number of the
 // exchange in the upper 32 bits.  Words are written and read by relaxed device-scope atomics, so
@@ -1825,7 +1825,7 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
 // mutually; the host checks that).  The partial minima and the published minimum have one buffer
 // each: a tile posts the next minimum only after it has read the last published one.
 // ---------------------------------------------------------------------------
-constexpr int kRunSpin = 1 << 21;     // polls before a wait gives up (about 1 us each)
+constexpr int kRunPolls = 1 << 21;    // polls before a wait gives up (about 1 us each), by default
 constexpr int kRunCopies = 32;        // copies of the published time step, kRunStride words apart
 constexpr int kRunStride = 16;
 struct RunArgs {
@@ -1835,6 +1835,7 @@ struct RunArgs {
     const unsigned char *need;  // per device cell: another tile reads it
     unsigned ex0, dt0;          // numbers of the last exchange and time step before this launch
     int nsteps, stages, ntiles;
+    int polls;                  // polls after which a wait gives up (0: every wait gives up)
     int rhs_step;               // the step whose first-stage rhs is kept (-1: none)
     double a[3], b[3];          // stage s > 0: Uout = a Un + b (Uin + dt rhs)
 };
@@ -1899,8 +1900,8 @@ __device__ __forceinline__ void run_reduce(const RunArgs &ra) {
                 lo = ll_load(ra.part + k);
                 hi = ll_load(ra.part + n + k);
                 fl = ll_load(ra.part + 2 * n + k);
-            } while (!(ll_is(lo, tag) && ll_is(hi, tag) && ll_is(fl, tag)) && ++spin < kRunSpin);
-            if (spin >= kRunSpin) stop = 2;
+            } while (!(ll_is(lo, tag) && ll_is(hi, tag) && ll_is(fl, tag)) && ++spin < ra.polls);
+            if (spin >= ra.polls) stop = 2;
             else {
                 d = fmin(d, ll_double(lo, hi));
                 stop |= (int)(fl & 3u);
@@ -2074,11 +2075,11 @@ __global__ __launch_bounds__((TileCfg<C, kRunShape<C>>::kThreads), WAVES) void k
                     lo = ll_load(q);
                     hi = ll_load(q + 1);
                     fl = ll_load(q + 2);
-                } while (!(ll_is(lo, dtag) && ll_is(hi, dtag) && ll_is(fl, dtag)) && ++spin < kRunSpin);
+                } while (!(ll_is(lo, dtag) && ll_is(hi, dtag) && ll_is(fl, dtag)) && ++spin < ra.polls);
                 const double t = sT, T = run_args<G>().sc->T;
                 double d = ll_double(lo, hi);
                 if (t + d > T) d = T - t;
-                const int stop = spin >= kRunSpin ? 2 : (int)(fl & 3u);
+                const int stop = spin >= ra.polls ? 2 : (int)(fl & 3u);
                 if (!stop) {
                     sDt = d;
                     sT = t + d;
@@ -2125,15 +2126,15 @@ __global__ __launch_bounds__((TileCfg<C, kRunShape<C>>::kThreads), WAVES) void k
                 bool ok;
                 // one word is polled until it is there, then all are read (and read again while any is
                 // not): polling all eight took 35.6 instead of 30.0 us per step at 131k cells
-                while (!ll_is(ll_load(q + 7 * (size_t)nc), ex) && ++spin < kRunSpin) {}
+                while (!ll_is(ll_load(q + 7 * (size_t)nc), ex) && ++spin < ra.polls) {}
                 do {
                     ok = true;
 #pragma unroll
                     for (int k = 0; k < 8; k++) w[k] = ll_load(q + (size_t)k * nc);
 #pragma unroll
                     for (int k = 0; k < 8; k++) ok = ok && ll_is(w[k], ex);
-                } while (!ok && ++spin < kRunSpin);
-                if (!ok) sFail = 1;
+                } while (!ok && ++spin < ra.polls);
+                if (!ok || ra.polls <= 0) sFail = 1;
                 lds_put(lds.U, Cfg::kMaxL, i, SU{(C)ll_double(w[0], w[1]), (C)ll_double(w[2], w[3]),
                                                  (C)ll_double(w[4], w[5]), (C)ll_double(w[6], w[7])});
             }
@@ -2705,6 +2706,9 @@ struct fvmr_solver {
     unsigned long long *run_ll = nullptr, *run_part = nullptr, *run_pub = nullptr;
     unsigned char *run_need = nullptr;
     unsigned run_ex = 0, run_dt = 0;      // numbers of the last exchange and time step
+    bool run_on = true;                   // fvmr_use_resident
+    int run_polls = kRunPolls;
+    long long run_steps = 0;              // steps and pseudo-time iterations it has done
     // output quantities: node -> cells (caller's element order), node buffers, boundary edges
     int *nc_off = nullptr, *nc_cells = nullptr;
     double *node_buf = nullptr;               // 6 x nv: ruvp, Cp, Ma
@@ -2972,7 +2976,7 @@ int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
     k.nc = h->nc;
     const int stages = h->p.time_advance == FVMR_EVO_RK3 ? 3 : 1;
     k.ra = RunArgs{h->run_ll, h->run_part, h->run_pub, h->run_need, h->run_ex, h->run_dt, nsteps, stages, h->ntiles,
-                   rhs_step, {0.0, 0.75, 1.0 / 3.0}, {1.0, 0.25, 2.0 / 3.0}};
+                   h->run_polls, rhs_step, {0.0, 0.75, 1.0 / 3.0}, {1.0, 0.25, 2.0 / 3.0}};
     void *args[] = {&k};
     HIP_OK(hipLaunchCooperativeKernel(steady ? h->run_steady_kernel : h->run_step_kernel, dim3(h->ntiles + (steady ? 0 : 1)),
                                       dim3(TileCfg<C, kRunShape<C>>::kThreads), args, 0, h->stream));
@@ -2998,6 +3002,7 @@ int run_resident(fvmr_solver *h, int n, bool store_rhs_last, int *done) {
         if ((rc = read_scalars(h, s))) return rc;
         if (s.run_failed) return set_error(FVMR_ERR_HIP, "resident step kernel: a work-group waited too long for its neighbours");
         *done += (int)s.run_done;
+        h->run_steps += (int)s.run_done;
         if (s.bad_count > 0) {
             if ((rc = h->mixed ? launch_restrict<float>(h, h->Ubuf[h->cur]) : launch_restrict<double>(h, h->Ubuf[h->cur]))) return rc;
         }
@@ -3015,7 +3020,7 @@ int run_steps(fvmr_solver *h, int n, bool store_rhs_last) {
     // 8-12 us less than a launched one (8,192 to 120,000 cells: 3 steps 143 / 201 against 143 / 208 us,
     // 5 steps 182 / 274 against 199 / 301 us)
     constexpr int kRunMin = 4;
-    if (h->run_step_kernel && !h->use_graphs && !h->profiling && n >= kRunMin) {
+    if (h->run_on && h->run_step_kernel && !h->use_graphs && !h->profiling && n >= kRunMin) {
         // (after a step with cells to restrict the rest runs by the kernels below, so that a flow
         // which needs it in every step is not stopped at each)
         if ((rc = run_resident(h, n, store_rhs_last, &done))) return rc;
@@ -4244,6 +4249,19 @@ int fvmr_autotune_candidates(int precision, int *n, int *tile_threads, int *tile
 int fvmr_use_graphs(fvmr_handle *h, int on) {
     if (!h) return set_error(FVMR_ERR_INVALID_ARG, "null handle");
     h->use_graphs = (on != 0);
+    return FVMR_OK;
+}
+
+int fvmr_use_resident(fvmr_handle *h, int on, int max_polls) {
+    if (!h) return set_error(FVMR_ERR_INVALID_ARG, "null handle");
+    h->run_on = (on != 0);
+    h->run_polls = max_polls < 0 ? kRunPolls : std::min(max_polls, kRunPolls);
+    return FVMR_OK;
+}
+
+int fvmr_resident_steps(fvmr_handle *h, long long *steps) {
+    if (!h || !steps) return set_error(FVMR_ERR_INVALID_ARG, "null argument");
+    *steps = h->run_steps;
     return FVMR_OK;
 }
 

@@ -385,6 +385,13 @@ int fvmr_adjoint_state(fvmr_handle *h, double *const psi[4]);
  * (default off; never while profiling).  No reference counterpart: the reference launches
  * every kernel from the host each step. */
 int fvmr_use_graphs(fvmr_handle *h, int on);
+/* The resident kernel: many steps (or pseudo-time iterations) of a small mesh in one launch, with the
+ * results of the launched kernels bit for bit (default on).  on: 0 keeps the handle on the launched
+ * kernels, 1 lets it use the resident one where it can.  max_polls: polls after which a wait between
+ * its work-groups gives up (< 0: the default, about 2 s; 0: at once).  No reference counterpart. */
+int fvmr_use_resident(fvmr_handle *h, int on, int max_polls);
+/* Steps and pseudo-time iterations that h has done in resident launches so far. */
+int fvmr_resident_steps(fvmr_handle *h, long long *steps);
 /* Autotuner of the tile kernels (no reference counterpart): times `steps` steps of the uniform
  * freestream of p on mesh m for every candidate work-group shape and tile size (fvmr_autotune_
  * candidates) and returns the fastest pair (set them as p->tile_threads, p->tile_cells) and its
