@@ -1695,19 +1695,52 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
     const Mesh<double> m = mesh_args<double>(h);
     double r0 = -1.0, r = -1.0, nrm[4];
     int it = 0;
-    while (it < max_iters) {
+    // The iterations of a resident launch that is not yet known to have finished, and the buffer it started from,
+    // which nothing writes until the flag of its waits has been read with the next residual.
+    int pending = 0, from = 0;
+    Scalars s{};
+    auto redo = [&]() -> int {   // a wait gave up: these iterations again, with the launched kernels
+        it -= pending;
+        pending = 0;
+        return run_leave(h, from, s);
+    };
+    while (it < max_iters || pending) {
+        if (it == max_iters) {
+            if ((rc = read_scalars(h, s))) return rc;
+            if (s.run_failed) {
+                if ((rc = redo())) return rc;
+                continue;
+            }
+            h->run_steps += pending;
+            break;
+        }
         const int a = h->cur, b = (a + 1) % 3, c = (a + 2) % 3;
         S4 *Ua = h->Ubuf[a], *Ub = h->Ubuf[b], *Uc = h->Ubuf[c];
         const bool check = (it % kAdjCheck == 0);
         if (h->run_on && h->run_steady_kernel && !check) {   // the iterations up to the next check in one launch
             const int n = std::min(kAdjCheck - it % kAdjCheck, max_iters - it);
             if ((rc = launch_run<double, double>(h, n, -1, true))) return rc;
-            h->run_steps += n;
+            from = a;
+            pending = n;
             it += n;
             continue;
         }
         if ((rc = local_dt(h, Ua))) return rc;
         if ((rc = steady_stage(h, Ua, Ua, Ub, 0.0, 1.0, 1, check ? h->rhs : nullptr))) return rc;
+        if (check) {
+            Scalars *const q = h->pin ? reinterpret_cast<Scalars *>(h->pin) : &s;
+            if (pending) HIP_OK(hipMemcpyAsync(q, h->sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
+            if ((rc = field_norm2(h, h->rhs, nrm))) return rc;
+            if (pending) {
+                s = *q;
+                if (s.run_failed) {
+                    if ((rc = redo())) return rc;
+                    continue;
+                }
+                h->run_steps += pending;
+                pending = 0;
+            }
+        }
         if (h->p.time_advance == FVMR_EVO_RK3) {
             if ((rc = steady_stage(h, Ub, Ua, Uc, 0.75, 0.25, 0, nullptr)) ||
                 (rc = steady_stage(h, Uc, Ua, Ub, 1.0 / 3.0, 2.0 / 3.0, 0, nullptr)))
@@ -1716,7 +1749,6 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
         h->cur = b;
         it++;
         if (check) {
-            if ((rc = field_norm2(h, h->rhs, nrm))) return rc;
             r = nrm[0];
             if (r0 < 0) r0 = r;
             if (!std::isfinite(r)) return set_error(FVMR_ERR_NUMERIC, "steady solve: the residual is not finite");
@@ -1725,11 +1757,6 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
     }
     h->rhs_valid = false;
     free_graphs(h);
-    if (h->run_steady_kernel) {
-        Scalars s{};
-        if ((rc = read_scalars(h, s))) return rc;
-        if (s.run_failed) return set_error(FVMR_ERR_HIP, "resident step kernel: a work-group waited too long for its neighbours");
-    }
     if (iters) *iters = it;
     if (res) { res[0] = r0; res[1] = r; }
     return FVMR_OK;

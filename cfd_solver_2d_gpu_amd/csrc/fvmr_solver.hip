@@ -2988,23 +2988,36 @@ int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
 
 int read_scalars(fvmr_solver *h, Scalars &s);
 
-// n steps by the resident kernel; *done: the steps done (fewer when a step left cells to restrict,
-// which are restricted here).
-int run_resident(fvmr_solver *h, int n, bool store_rhs_last, int *done) {
+// The resident kernel could not finish: the handle goes back to the buffer (never written by the kernel) and the
+// scalars that its last launch started from, and stays with the launched kernels, since the next launch would
+// wait as long (fvmr_use_resident turns it on again).
+int run_leave(fvmr_solver *h, int cur, Scalars s) {
+    h->cur = cur;
+    h->run_on = false;
+    s.run_done = s.run_failed = 0;
+    HIP_OK(hipMemcpyAsync(h->sc, &s, sizeof(Scalars), hipMemcpyHostToDevice, h->stream));
+    HIP_OK(hipStreamSynchronize(h->stream));
+    return FVMR_OK;
+}
+
+// n steps by the resident kernel from the scalars s; *done: the steps done (fewer when a step left cells to
+// restrict, which are restricted here, and when the kernel could not finish).
+int run_resident(fvmr_solver *h, int n, bool store_rhs_last, Scalars s, int *done) {
     constexpr int kMost = 10000;   // steps per launch: a fraction of a second
     int rc;
     for (*done = 0; *done < n;) {
-        const int k = std::min(n - *done, kMost);
+        const int k = std::min(n - *done, kMost), from = h->cur;
+        const Scalars before = s;
         const int rhs_step = (store_rhs_last && *done + k == n) ? k - 1 : -1;
         rc = h->mixed ? launch_run<float, float>(h, k, rhs_step, false) : launch_run<double, double>(h, k, rhs_step, false);
         if (rc) return rc;
-        Scalars s{};
         if ((rc = read_scalars(h, s))) return rc;
-        if (s.run_failed) return set_error(FVMR_ERR_HIP, "resident step kernel: a work-group waited too long for its neighbours");
+        if (s.run_failed) return run_leave(h, from, before);
         *done += (int)s.run_done;
         h->run_steps += (int)s.run_done;
         if (s.bad_count > 0) {
             if ((rc = h->mixed ? launch_restrict<float>(h, h->Ubuf[h->cur]) : launch_restrict<double>(h, h->Ubuf[h->cur]))) return rc;
+            s.bad_count = 0;
         }
         if ((int)s.run_done < k) return FVMR_OK;
     }
@@ -3012,9 +3025,9 @@ int run_resident(fvmr_solver *h, int n, bool store_rhs_last, int *done) {
     return FVMR_OK;
 }
 
-// n steps; the last one keeps its stage-1 rhs when store_rhs_last.  Without profiling, runs of
-// three steps replay a captured graph (the same launches with the same arguments).
-int run_steps(fvmr_solver *h, int n, bool store_rhs_last) {
+// n steps from the scalars s (of the first case); the last one keeps its stage-1 rhs when store_rhs_last.
+// Without profiling, runs of three steps replay a captured graph (the same launches with the same arguments).
+int run_steps(fvmr_solver *h, int n, bool store_rhs_last, const Scalars &s) {
     int rc, done = 0;
     // from 4 steps on: a cooperative launch costs about 40 us more than an ordinary one, a resident step
     // 8-12 us less than a launched one (8,192 to 120,000 cells: 3 steps 143 / 201 against 143 / 208 us,
@@ -3023,7 +3036,7 @@ int run_steps(fvmr_solver *h, int n, bool store_rhs_last) {
     if (h->run_on && h->run_step_kernel && !h->use_graphs && !h->profiling && n >= kRunMin) {
         // (after a step with cells to restrict the rest runs by the kernels below, so that a flow
         // which needs it in every step is not stopped at each)
-        if ((rc = run_resident(h, n, store_rhs_last, &done))) return rc;
+        if ((rc = run_resident(h, n, store_rhs_last, s, &done))) return rc;
     }
     if (h->use_graphs && !h->profiling) {
         const int eager_tail = store_rhs_last ? 1 : 0;
@@ -3776,7 +3789,7 @@ int fvmr_advance(fvmr_handle *h, int nsteps, double *t, double T, fvmr_step_info
     s.T = T;
     s.run_done = s.run_failed = 0; s.bad_count = 0; s.n_restricted = 0;
     HIP_OK(hipMemcpyAsync(h->sc, &s, sizeof(Scalars), hipMemcpyHostToDevice, h->stream));
-    if ((rc = run_steps(h, nsteps, true))) return rc;
+    if ((rc = run_steps(h, nsteps, true, s))) return rc;
     if ((rc = read_scalars(h, s))) return rc;
     if (info) {
         info->t = s.t;
@@ -3835,10 +3848,10 @@ int fvmr_batch_advance(fvmr_handle *h, int nsteps, double *t, const double *T) {
     HIP_OK(hipMemcpyAsync(s.data(), h->sc, s.size() * sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));
     for (int c = 0; c < h->ncases; c++) { s[c].t = t[c]; s[c].T = T[c]; }
-    s[0].bad_count = 0; s[0].n_restricted = 0;
+    s[0].run_done = s[0].run_failed = 0; s[0].bad_count = 0; s[0].n_restricted = 0;
     HIP_OK(hipMemcpyAsync(h->sc, s.data(), s.size() * sizeof(Scalars), hipMemcpyHostToDevice, h->stream));
     int rc;
-    if ((rc = run_steps(h, nsteps, false))) return rc;
+    if ((rc = run_steps(h, nsteps, false, s[0]))) return rc;
     HIP_OK(hipMemcpyAsync(s.data(), h->sc, s.size() * sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));
     if (h->profiling && (rc = prof_collect(h))) return rc;
