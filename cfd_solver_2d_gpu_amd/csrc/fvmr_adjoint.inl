@@ -1719,7 +1719,7 @@ int fvmr_steady_solve(fvmr_handle *h, int max_iters, double tol, int *iters, dou
         const bool check = (it % kAdjCheck == 0);
         if (h->run_on && h->run_steady_kernel && !check) {   // the iterations up to the next check in one launch
             const int n = std::min(kAdjCheck - it % kAdjCheck, max_iters - it);
-            if ((rc = launch_run<double, double>(h, n, -1, true))) return rc;
+            if (!launch_run<double, double>(h, n, -1, true)) continue;
             from = a;
             pending = n;
             it += n;

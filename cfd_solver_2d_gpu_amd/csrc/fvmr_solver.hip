@@ -2961,9 +2961,10 @@ const void *run_kernel(const fvmr_solver *h, bool steady, bool wide) {
 }
 
 // Launches nsteps steps (steady: pseudo-time iterations) of the resident kernel from buffer cur to
-// the next one.
+// the next one.  False when the device refuses the launch, as it does to a second process that would launch
+// cooperatively: nothing has run then, and the handle stays with the launched kernels.
 template <class C, class G>
-int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
+bool launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
     const int a = h->cur, b = (a + 1) % 3;
     RunKernArg<G> k{};
     k.ta = tile_args<G>(h);
@@ -2978,12 +2979,16 @@ int launch_run(fvmr_solver *h, int nsteps, int rhs_step, bool steady) {
     k.ra = RunArgs{h->run_ll, h->run_part, h->run_pub, h->run_need, h->run_ex, h->run_dt, nsteps, stages, h->ntiles,
                    h->run_polls, rhs_step, {0.0, 0.75, 1.0 / 3.0}, {1.0, 0.25, 2.0 / 3.0}};
     void *args[] = {&k};
-    HIP_OK(hipLaunchCooperativeKernel(steady ? h->run_steady_kernel : h->run_step_kernel, dim3(h->ntiles + (steady ? 0 : 1)),
-                                      dim3(TileCfg<C, kRunShape<C>>::kThreads), args, 0, h->stream));
+    if (hipLaunchCooperativeKernel(steady ? h->run_steady_kernel : h->run_step_kernel, dim3(h->ntiles + (steady ? 0 : 1)),
+                                   dim3(TileCfg<C, kRunShape<C>>::kThreads), args, 0, h->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        h->run_on = false;
+        return false;
+    }
     h->run_ex += (unsigned)(nsteps * stages);
     if (!steady) h->run_dt += (unsigned)nsteps;
     h->cur = b;
-    return FVMR_OK;
+    return true;
 }
 
 int read_scalars(fvmr_solver *h, Scalars &s);
@@ -3001,7 +3006,7 @@ int run_leave(fvmr_solver *h, int cur, Scalars s) {
 }
 
 // n steps by the resident kernel from the scalars s; *done: the steps done (fewer when a step left cells to
-// restrict, which are restricted here, and when the kernel could not finish).
+// restrict, which are restricted here, and when the kernel could not start or finish).
 int run_resident(fvmr_solver *h, int n, bool store_rhs_last, Scalars s, int *done) {
     constexpr int kMost = 10000;   // steps per launch: a fraction of a second
     int rc;
@@ -3009,8 +3014,8 @@ int run_resident(fvmr_solver *h, int n, bool store_rhs_last, Scalars s, int *don
         const int k = std::min(n - *done, kMost), from = h->cur;
         const Scalars before = s;
         const int rhs_step = (store_rhs_last && *done + k == n) ? k - 1 : -1;
-        rc = h->mixed ? launch_run<float, float>(h, k, rhs_step, false) : launch_run<double, double>(h, k, rhs_step, false);
-        if (rc) return rc;
+        if (!(h->mixed ? launch_run<float, float>(h, k, rhs_step, false) : launch_run<double, double>(h, k, rhs_step, false)))
+            return FVMR_OK;
         if ((rc = read_scalars(h, s))) return rc;
         if (s.run_failed) return run_leave(h, from, before);
         *done += (int)s.run_done;

@@ -1,10 +1,17 @@
 """Runs that the resident kernel cannot finish go on with the launched kernels from the state they had: a wait
 between its work-groups that gives up (forced by a limit of 0 polls, with which every work-group leaves at its
-first wait)."""
+first wait) and a cooperative launch that the device refuses (a child process with a layer in front of the
+runtime's calls)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 import cfd_solver_2d_gpu_amd as F
+from cfd_solver_2d_gpu_amd.build import C_API_DIR
+from conftest import ROOT
 from helpers import vortex_case, wedge_case
 from test_gpu_resident import naca_case
 
@@ -97,3 +104,76 @@ def test_batch_of_one_case_goes_on_after_a_wait_that_gives_up():
         out.append((b.get_state(0), t))
         b.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+REFUSED = r"""
+import ctypes as C, sys
+sys.path[:0] = [sys.argv[2], sys.argv[2] + "/tests"]
+front = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)   # before the library, which then calls it
+import numpy as np
+import cfd_solver_2d_gpu_amd as F
+from helpers import wedge_case
+from test_gpu_resident import naca_case
+
+def var(name):
+    return C.c_int.in_dll(front, name)
+
+def run(case, launched=False):
+    m, p, U = case()
+    g = F.GPUSolver2(m, p)
+    g.use_resident(not launched)
+    g.set_state(U)
+    out = []
+    t = 0.0
+    for _ in range(2):
+        t, info = g.advance(9, t, 1e9, F.NORM_INF)
+        out += [g.get_state(), t, info.dt, np.array(info.residual[:])]
+    if p.limiter == F.LIM_VENKATAKRISHNAN:
+        out += [*g.steady_solve(77, 0.0), g.get_state()]
+    n = g.resident_steps()
+    g.close()
+    return out, n
+
+cases = {"wedge": lambda: wedge_case(65, 33, scheme=F.SOL_ROE), "naca": lambda: naca_case(48, 21)}
+for name, case in cases.items():
+    want, n = run(case, launched=True)
+    assert n == 0
+    got, n = run(case)   # resident, unless the device itself refuses: this process is its second one here
+    assert var("refused").value == 0
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    if sys.argv[3] == "launch":
+        var("refuse_cooperative").value = 1
+    else:   # the last allocation of a handle's creation: the resident kernel's
+        m, p, U = case()
+        var("mallocs").value = 0
+        F.GPUSolver2(m, p).close()
+        var("refuse_malloc").value = var("mallocs").value
+        var("mallocs").value = 0
+    got, n = run(case)
+    assert n == 0 and var("refused").value >= 1
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    for v in ("refuse_cooperative", "refuse_malloc", "refused"):
+        var(v).value = 0
+    print("ok", name, flush=True)
+"""
+
+
+@pytest.fixture(scope="module")
+def front(tmp_path_factory):
+    """The layer in front of the runtime (tests/c_api/hip_refuse.cpp)."""
+    out = str(tmp_path_factory.mktemp("front") / "libhip_refuse.so")
+    rocm = "/opt/rocm"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                    os.path.join(C_API_DIR, "hip_refuse.cpp"), f"-L{rocm}/lib", "-Wl,--no-as-needed", "-lamdhip64",
+                    f"-Wl,-rpath,{rocm}/lib", "-o", out], check=True)
+    return out
+
+
+def refused(front, what):
+    r = subprocess.run([sys.executable, "-c", REFUSED, front, ROOT, what], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split() == ["ok", "wedge", "ok", "naca"], r.stdout + r.stderr
+
+
+def test_refused_launch_goes_on_with_the_launched_kernels(front):
+    announce("cooperative launches that the device refuses")
+    refused(front, "launch")
