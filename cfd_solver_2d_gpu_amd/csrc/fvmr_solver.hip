@@ -2703,7 +2703,7 @@ struct fvmr_solver {
     DtRec *t_dtrec = nullptr;
     // resident kernel (k_run): exchange buffers, allocated by fvmr_create when the handle can use it
     const void *run_step_kernel = nullptr, *run_steady_kernel = nullptr;   // NULL: not on this handle
-    unsigned long long *run_ll = nullptr, *run_part = nullptr, *run_pub = nullptr;
+    unsigned long long *run_ll = nullptr, *run_part = nullptr, *run_pub = nullptr;   // one allocation: run_ll
     unsigned char *run_need = nullptr;
     unsigned run_ex = 0, run_dt = 0;      // numbers of the last exchange and time step
     bool run_on = true;                   // fvmr_use_resident
@@ -3113,14 +3113,20 @@ int run_setup(fvmr_solver *h, const std::vector<int2> &cslot, const std::vector<
         }
     std::vector<unsigned char> need(nc, 0);
     for (int c : halo) need[c] = 1;
-    int rc;
-    if ((rc = upload(&h->run_need, need, h->stream))) return rc;
-    const size_t words[3] = {16 * (size_t)nc, 3 * (size_t)h->ntiles, (size_t)kRunCopies * kRunStride};
-    unsigned long long **dst[3] = {&h->run_ll, &h->run_part, &h->run_pub};
-    for (int k = 0; k < 3; k++) {
-        HIP_OK(hipMalloc((void **)dst[k], words[k] * sizeof(unsigned long long)));
-        HIP_OK(hipMemsetAsync(*dst[k], 0, words[k] * sizeof(unsigned long long), h->stream));
+    // one allocation, its parts on 128-byte lines of their own: exchanged states, partial minima, published minimum,
+    // and which cells are exchanged
+    const size_t ll = 16 * (size_t)nc, part = (3 * (size_t)h->ntiles + 15) / 16 * 16, pub = (size_t)kRunCopies * kRunStride;
+    const size_t words = ll + part + pub;
+    if (hipMalloc((void **)&h->run_ll, words * sizeof(unsigned long long) + nc) != hipSuccess) {
+        (void)hipGetLastError();   // no memory for it: the launched kernels
+        h->run_ll = nullptr;
+        return FVMR_OK;
     }
+    h->run_part = h->run_ll + ll;
+    h->run_pub = h->run_part + part;
+    h->run_need = reinterpret_cast<unsigned char *>(h->run_pub + pub);
+    HIP_OK(hipMemsetAsync(h->run_ll, 0, words * sizeof(unsigned long long), h->stream));
+    HIP_OK(hipMemcpyAsync(h->run_need, need.data(), nc, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));   // need goes out of scope
     h->run_step_kernel = run;
     h->run_steady_kernel = steady;
@@ -3240,8 +3246,7 @@ void free_all(fvmr_solver *h) {
                     h->eint, h->partial, h->norm_out, h->bad_list, h->sc, h->t_info, h->t_halo, h->t_lnodes,
                     h->t_nxy, h->t_gslot, h->t_face, h->t_gcoef, h->t_dtrec, h->t_lcxy, h->t_fnrm,
                     h->nc_off, h->nc_cells, h->node_buf, h->cbc, h->tile_case_begin, h->perm_dev, h->io_soa,
-                    h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev, h->run_ll, h->run_part, h->run_pub,
-                    h->run_need};
+                    h->bedge_ref_dev, h->bedge_nodes_dev, h->bedge_geo_dev, h->run_ll};
     for (void *q : ptrs) if (q) (void)hipFree(q);
     if (h->pin) (void)hipHostFree(h->pin);
     for (auto &e : h->pin_ev) if (e) (void)hipEventDestroy(e);

@@ -1,7 +1,7 @@
 """Runs that the resident kernel cannot finish go on with the launched kernels from the state they had: a wait
 between its work-groups that gives up (forced by a limit of 0 polls, with which every work-group leaves at its
-first wait) and a cooperative launch that the device refuses (a child process with a layer in front of the
-runtime's calls)."""
+first wait) and a cooperative launch or an allocation that the device refuses (a child process with a layer in front of
+the runtime's calls)."""
 import os
 import subprocess
 import sys
@@ -177,3 +177,8 @@ def refused(front, what):
 def test_refused_launch_goes_on_with_the_launched_kernels(front):
     announce("cooperative launches that the device refuses")
     refused(front, "launch")
+
+
+def test_refused_allocation_leaves_the_launched_kernels(front):
+    announce("the resident kernel's memory refused at creation")
+    refused(front, "memory")
