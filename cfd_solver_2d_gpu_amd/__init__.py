@@ -202,7 +202,7 @@ def _rows(U, n=None):
 
 def autotune(mesh, params, steps=20):
     """fvmr_autotune: (best tile_threads, best tile_cells, ms per step) over the candidate
-    work-group shapes and tile sizes on this mesh."""
+    work-group shapes and tile sizes on this mesh (tile_cells 0: the library's choice)."""
     th, best = C.c_int(), C.c_int()
     ms = C.c_double()
     check(lib().fvmr_autotune(C.byref(mesh.soa), C.byref(params), steps, C.byref(th), C.byref(best), C.byref(ms)),
@@ -337,6 +337,12 @@ class GPUSolver2:
     def use_graphs(self, on=True):
         """Replay runs of three steps from captured HIP graphs (default off)."""
         check(lib().fvmr_use_graphs(self._h, 1 if on else 0), "fvmr_use_graphs")
+
+    def tile_shape(self):
+        """(tile_threads, tile_cells) of the handle's tiles; (0, 0) with the cell kernels."""
+        th, cells = C.c_int(), C.c_int()
+        check(lib().fvmr_tile_shape(self._h, C.byref(th), C.byref(cells)), "fvmr_tile_shape")
+        return th.value, cells.value
 
     def use_resident(self, on=True, max_polls=-1):
         """Let the resident kernel serve runs of steps where it can (default on); max_polls: polls after

@@ -123,6 +123,7 @@ SIGNATURES = {
     "fvmr_autotune_batch": (C.c_int, [C.c_int, C.POINTER(C.POINTER(MeshSoA)), C.POINTER(Params), C.c_int, _ip, _ip,
                                       _dp, _dp]),
     "fvmr_autotune_candidates": (C.c_int, [C.c_int, _ip, _ip, _ip]),
+    "fvmr_tile_shape": (C.c_int, [C.c_void_p, _ip, _ip]),
     "fvmr_set_boundary_states": (C.c_int, [C.c_void_p, _dp, _dp, _dp]),
     "fvmr_vertex_colors": (C.c_int, [C.c_void_p, C.c_int, C.c_float, C.c_float, C.c_int, C.POINTER(C.c_float),
                                      C.POINTER(C.c_float), C.c_int]),

@@ -595,6 +595,8 @@ class Driver:
         if not c.useGPU:
             self.log("basic.useGPU = 0: the device path runs the case")
         solver = GPUSolver2(self.mesh, self.params)
+        if c.tile_cells == -1:   # what the tuner left to the library
+            self.params.tile_threads, self.params.tile_cells = solver.tile_shape()
         try:
             if c.use_graphs:
                 solver.use_graphs(True)

@@ -394,8 +394,8 @@ int fvmr_use_resident(fvmr_handle *h, int on, int max_polls);
 int fvmr_resident_steps(fvmr_handle *h, long long *steps);
 /* Autotuner of the tile kernels (no reference counterpart): times `steps` steps of the uniform
  * freestream of p on mesh m for every candidate work-group shape and tile size (fvmr_autotune_
- * candidates) and returns the fastest pair (set them as p->tile_threads, p->tile_cells) and its
- * ms per step (best_ms may be NULL).  It holds one handle per candidate at once, keeps the GPU
+ * candidates) and returns the fastest pair (set them as p->tile_threads, p->tile_cells; a tile size
+ * of 0 leaves it to fvmr_create) and its ms per step (best_ms may be NULL).  It holds one handle per candidate at once, keeps the GPU
  * busy for at least 40 ms before timing (clocks rise under load) and takes the faster of two
  * timed runs per candidate, one pass forward and one backward. */
 int fvmr_autotune(const fvmr_mesh_soa *m, const fvmr_params *p, int steps, int *best_tile_threads,
@@ -405,8 +405,11 @@ int fvmr_autotune(const fvmr_mesh_soa *m, const fvmr_params *p, int steps, int *
 int fvmr_autotune_batch(int ncases, const fvmr_mesh_soa *const *meshes, const fvmr_params *params, int steps,
                         int *best_tile_threads, int *best_tile_cells, double *best_ms, double *timings);
 /* The tuners' candidates for a precision (FVMR_PREC_*): *n pairs (at most 16) of work-group size
- * and tile size. */
+ * and tile size, every work-group size with the default tile size (0) among them. */
 int fvmr_autotune_candidates(int precision, int *n, int *tile_threads, int *tile_cells);
+/* Work-items per work-group and most cells per tile of the handle's tile kernels; given as
+ * tile_threads and tile_cells they make a handle with the same tiles.  0, 0: it runs the cell kernels. */
+int fvmr_tile_shape(fvmr_handle *h, int *tile_threads, int *tile_cells);
 /* 1: record HIP events around every kernel launch on the handle's stream. */
 int fvmr_profile_enable(fvmr_handle *h, int on);
 /* Average ms per launch and launch count of a kernel class since the last reset:
