@@ -335,7 +335,7 @@ class GPUSolver2:
         return p
 
     def use_graphs(self, on=True):
-        """Replay runs of three steps from captured HIP graphs (default off)."""
+        """Replay runs of three steps from captured HIP graphs (default off) where they are not resident."""
         check(lib().fvmr_use_graphs(self._h, 1 if on else 0), "fvmr_use_graphs")
 
     def tile_shape(self):

@@ -3032,14 +3032,16 @@ int run_resident(fvmr_solver *h, int n, bool store_rhs_last, Scalars s, int *don
 }
 
 // n steps from the scalars s (of the first case); the last one keeps its stage-1 rhs when store_rhs_last.
-// Without profiling, runs of three steps replay a captured graph (the same launches with the same arguments).
+// Without profiling, runs of three steps that are not resident replay a captured graph (the same launches with the
+// same arguments).
 int run_steps(fvmr_solver *h, int n, bool store_rhs_last, const Scalars &s) {
     int rc, done = 0;
     // from 4 steps on: a cooperative launch costs about 40 us more than an ordinary one, a resident step
     // 8-12 us less than a launched one (8,192 to 120,000 cells: 3 steps 143 / 201 against 143 / 208 us,
     // 5 steps 182 / 274 against 199 / 301 us)
     constexpr int kRunMin = 4;
-    if (h->run_on && h->run_step_kernel && !h->use_graphs && !h->profiling && n >= kRunMin) {
+    // also before graphs, whose replays are the same launches (8,192 cells: 27 to 30 us a step against 16)
+    if (h->run_on && h->run_step_kernel && !h->profiling && n >= kRunMin) {
         // (after a step with cells to restrict the rest runs by the kernels below, so that a flow
         // which needs it in every step is not stopped at each)
         if ((rc = run_resident(h, n, store_rhs_last, s, &done))) return rc;

@@ -382,8 +382,8 @@ int fvmr_adjoint_state(fvmr_handle *h, double *const psi[4]);
 /* measurement                                                             */
 /* ---------------------------------------------------------------------- */
 /* Replay runs of three steps of fvmr_advance / fvmr_batch_advance from captured HIP graphs
- * (default off; never while profiling).  No reference counterpart: the reference launches
- * every kernel from the host each step. */
+ * (default off; never while profiling; runs that the resident kernel serves stay with it).  No
+ * reference counterpart: the reference launches every kernel from the host each step. */
 int fvmr_use_graphs(fvmr_handle *h, int on);
 /* The resident kernel: many steps (or pseudo-time iterations) of a small mesh in one launch, with the
  * results of the launched kernels bit for bit (default on).  on: 0 keeps the handle on the launched
