@@ -1496,6 +1496,7 @@ int steady_stage(fvmr_solver *h, const S4 *Uin, const S4 *Un, S4 *Uout, double a
         const bool ns = h->ph.equation == FVMR_EQ_NS, gg = tile_scheme(h->ph) != kTileAny;
         auto *kern = ns ? (gg ? k_tile<double, double, true, true, kTileGg> : k_tile<double, double, true, true, kTileAny>)
                         : (gg ? k_tile<double, double, false, true, kTileGg> : k_tile<double, double, false, true, kTileAny>);
+        if (!h->tile_sides) kern = ns ? k_tile<double, double, true, true, kTileFaces> : k_tile<double, double, false, true, kTileFaces>;
         kern<<<h->ntiles, TileCfg<double>::kThreads, 0, h->stream>>>(t, h->ph, Uin, Un, Uout, rhs, h->sc, h->bad_list, h->nc, a,
                                                                       b, first, 0);
         HIP_OK(hipGetLastError());
@@ -1560,7 +1561,7 @@ int adj_step(fvmr_solver *h, const S4 *U, const S4 *psi, const S4 *g, const S4 *
     const double *dtl = step ? w->dtl : nullptr;
     // tiles of the default shape: one launch, 44 us against the cell kernels' 98 at 393,216 cells, 12 against
     // 30 at 49,152 (the other work-group shapes use the cell kernels here, as the rest of the steady path)
-    if (h->tiles && h->shape == 0) {
+    if (h->tiles && h->tile_sides && h->shape == 0) {
         if ((rc = adj_gradient(h, U))) return rc;
         const bool gg = h->ph.gradient == FVMR_GRA_GREENGAUSS;
         const bool roe = h->ph.scheme == FVMR_SOL_ROE && h->ph.reconstruct == FVMR_REC_LINEAR;

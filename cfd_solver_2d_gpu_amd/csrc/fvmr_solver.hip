@@ -1351,7 +1351,9 @@ struct TileCells {
 // (centroids then need not be loaded); or all of the common Green-Gauss + Barth + Roe + linear
 // reconstruction (the compiler drops the other branches: 116 -> 99 VGPRs and about 3% of the FP64 kernel's
 // time).
-enum TileScheme { kTileAny = 0, kTileGgBarthRoe = 1, kTileGg = 2 };
+// kTileFaces: any scheme, on a mesh whose edges are not all the sides of their elements' nodes (FP64; in mixed
+// precision the gradients take the faces' records in any case).
+enum TileScheme { kTileAny = 0, kTileGgBarthRoe = 1, kTileGg = 2, kTileFaces = 4 };
 inline int tile_scheme(const Phys &ph) {
     if (ph.gradient != FVMR_GRA_GREENGAUSS) return kTileAny;
     return ph.limiter == FVMR_LIM_BARTH && ph.scheme == FVMR_SOL_ROE && ph.reconstruct == FVMR_REC_LINEAR ? kTileGgBarthRoe
@@ -1360,7 +1362,7 @@ inline int tile_scheme(const Phys &ph) {
 template <int SCHEME, bool NS>
 __device__ __forceinline__ void fix_scheme(Phys &ph) {
     if (!NS) ph.equation = FVMR_EQ_EULER;
-    if (SCHEME != kTileAny) ph.gradient = FVMR_GRA_GREENGAUSS;
+    if (SCHEME == kTileGg || SCHEME == kTileGgBarthRoe) ph.gradient = FVMR_GRA_GREENGAUSS;
     if (SCHEME == kTileGgBarthRoe) {
         ph.limiter = FVMR_LIM_BARTH;
         ph.scheme = FVMR_SOL_ROE;
@@ -1370,7 +1372,7 @@ __device__ __forceinline__ void fix_scheme(Phys &ph) {
 
 // LDS of a work-group that computes a tile's stages: states (16-byte columns), node coordinates,
 // centroids; the gradients (16-byte columns of kMaxG), which the face fluxes (columns of kMaxFF) replace once
-// every flux is formed.  GEO: the face records and normals too (the mixed gradients read normals, the
+// every flux is formed.  GEO: the face records and normals too (the mixed gradients and kTileFaces read them, the
 // resident kernel keeps both; the FP64 k_tile forms each face's normal once, in the thread of its flux).
 template <class Cfg, class G, bool GEO>
 struct TileFaces {
@@ -1404,9 +1406,9 @@ template <int FLAG> __device__ __forceinline__ double negate_if(double x, int sw
 // Limited gradient of local cell i (tile or first ring) into LDS.  gs: its slot words, gco: its
 // Green-Gauss weights and volume, nw: its nodes.  CEN: its centroid is formed here, from the nodes that the
 // limiter reads in any case, and put into LDS for the fluxes (only least squares reads a neighbour's here).
-// In FP64 a slot's area vector is the step between its two nodes, (dy, -dx): the product of the normal
-// (dy, -dx) / L and L up to its two roundings.  In mixed precision it is that product of FP32 values.
-template <bool CEN, class C, class G, class Cfg, bool GEO>
+// FACES: a slot's area vector is the product of its face's normal and length.  Without (FP64), it is the step between
+// the slot's two nodes, (dy, -dx), which is that product of (dy, -dx) / L and L up to its two roundings.
+template <bool CEN, bool FACES, class C, class G, class Cfg, bool GEO>
 __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg, GEO> &s, int i, const I3 gs,
                                               const V4<G> gco, int nw) {
     using SU = TileState<C>;
@@ -1448,7 +1450,7 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg,
         if (ph.gradient == FVMR_GRA_GREENGAUSS) {
             // weight g_C of the slot precomputed by the host (the device formula in FP64)
             sl.a[j][0] = (C)(j == 0 ? gco.x : (j == 1 ? gco.y : gco.z));
-            if constexpr (std::is_same<C, double>::value) {
+            if constexpr (!FACES) {
                 const V2<double> p = nd[j], q = nd[(j + 1) % 3];
                 sl.a[j][1] = negate_if<fvmr::kGsTurned>(q.y - p.y, sw[j]);
                 sl.a[j][2] = negate_if<fvmr::kGsTurned>(p.x - q.x, sw[j]);
@@ -1549,8 +1551,8 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     fix_scheme<SCHEME, NS>(ph);
     using Cfg = TileCfg<C, SHAPE>;
     constexpr int kTileThreads = Cfg::kThreads;
-    constexpr bool kGeo = !std::is_same<C, double>::value;
-    constexpr bool kOwnCen = SCHEME != kTileAny;
+    constexpr bool kGeo = !std::is_same<C, double>::value || SCHEME == kTileFaces;
+    constexpr bool kOwnCen = SCHEME == kTileGg || SCHEME == kTileGgBarthRoe;
     using SU = TileState<C>;
     __shared__ TileLds<C, G, Cfg, kGeo> lds;
     const int tid = threadIdx.x;
@@ -1592,7 +1594,7 @@ __global__ __launch_bounds__((TileCfg<C, SHAPE>::kThreads)) void k_tile(TileArgs
     if (!kOwnCen && i < nL) lds.cen[i] = cc;
     __syncthreads();
     // 2. limited gradients of the tile and the first ring
-    if (i < nG) tile_gradient<kOwnCen>(ph, lds, i, gs, gco, nw);
+    if (i < nG) tile_gradient<kOwnCen, kGeo>(ph, lds, i, gs, gco, nw);
     __syncthreads();
     // 3. one canonical flux per face of the tile (nFF <= threads), written over the gradients
     const double t_rk = sc[cs].t_rk;
@@ -2054,7 +2056,7 @@ __global__ __launch_bounds__((TileCfg<C, kRunShape<C>>::kThreads), WAVES) void k
             opaque(nw);
             opaque(gs.x); opaque(gs.y); opaque(gs.z);
             opaque(gco.x); opaque(gco.y); opaque(gco.z); opaque(gco.w);
-            if (i < nG) tile_gradient<false>(ph, lds, i, gs, gco, nw);
+            if (i < nG) tile_gradient<false, !kF64>(ph, lds, i, gs, gco, nw);
             __syncthreads();
             C F[4] = {C(0), C(0), C(0), C(0)};
             if (i < nFF) {
@@ -2696,6 +2698,7 @@ struct fvmr_solver {
     int ntiles = 0;
     int shape = 0;                        // work-group shape of the tile kernels (TileCfg<., shape>)
     int tile_cells = 0;                   // most cells of a tile
+    bool tile_sides = true;               // every edge is the side of its elements' nodes, or mixed (see kTileFaces)
     int *t_info = nullptr, *t_halo = nullptr, *t_lnodes = nullptr;
     V2<double> *t_nxy = nullptr;
     I3 *t_gslot = nullptr, *t_face = nullptr;
@@ -2880,7 +2883,7 @@ int launch_tile_stage(fvmr_solver *h, const S4 *Uin, const S4 *Un, S4 *Uout, dou
     int rc = prof_begin(h, 0, &e0);
     if (rc) return rc;
     const bool ns = h->ph.equation == FVMR_EQ_NS;
-    const int scheme = tile_scheme(h->ph);
+    const int scheme = h->tile_sides ? tile_scheme(h->ph) : kTileFaces;
     with_shape<C>(h, [&](auto sh) {
         constexpr int S = decltype(sh)::value;
         auto *kern = ns ? (scheme == kTileGgBarthRoe ? k_tile<C, G, true, false, kTileGgBarthRoe, S>
@@ -2889,6 +2892,9 @@ int launch_tile_stage(fvmr_solver *h, const S4 *Uin, const S4 *Un, S4 *Uout, dou
                         : (scheme == kTileGgBarthRoe ? k_tile<C, G, false, false, kTileGgBarthRoe, S>
                            : scheme == kTileGg       ? k_tile<C, G, false, false, kTileGg, S>
                                                      : k_tile<C, G, false, false, kTileAny, S>);
+        if constexpr (std::is_same<C, double>::value) {
+            if (scheme == kTileFaces) kern = ns ? k_tile<C, G, true, false, kTileFaces, S> : k_tile<C, G, false, false, kTileFaces, S>;
+        }
         kern<<<h->ntiles, TileCfg<C, S>::kThreads, 0, h->stream>>>(tile_args<G>(h), h->ph, Uin, Un, Uout, rhs_out, h->sc,
                                                                    h->bad_list, h->nc, a, b, first, last);
         return FVMR_OK;
@@ -3088,7 +3094,7 @@ int read_scalars(fvmr_solver *h, Scalars &s) {
 // with periodic faces, whose time step takes FP64 states across a face), and its buffers.
 int run_setup(fvmr_solver *h, const std::vector<int2> &cslot, const std::vector<int> &halo) {
     const int shape = h->mixed ? kRunShape<float> : kRunShape<double>;
-    if (!h->tiles || h->ncases != 1 || h->shape != shape || (h->mixed && h->ph.has_periodic)) return FVMR_OK;
+    if (!h->tiles || !h->tile_sides || h->ncases != 1 || h->shape != shape || (h->mixed && h->ph.has_periodic)) return FVMR_OK;
     int coop = 0, cus = 0;
     HIP_OK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, h->device));
     HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
@@ -3555,9 +3561,10 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
                            ccx.data(), ccy.data(), emx.data(), emy.data(), enx.data(), eny.data(), ncases, case_begin,
                            tile_sizes.empty() ? nullptr : &tile_sizes};
         if ((rc = fvmr::build_tiles(ti, caps, tm))) return bail(rc);
-        // elements whose edges are not the sides of their nodes: the tile kernels take each side from its two
-        // nodes, the cell kernels take the edges' own geometry
-        use_tiles = tm.joined;
+        // some element's edges are not the sides of its nodes: FP64 handles of fvmr_create take the cell kernels, which
+        // have the edges' own geometry; batches, which have no cell kernels, take kTileFaces
+        h->tile_sides = h->mixed || tm.joined;
+        use_tiles = h->tile_sides || case_params;
         if (!use_tiles) tm = fvmr::TileMesh();
     }
     if (use_tiles) {
@@ -3857,7 +3864,7 @@ int fvmr_batch_get_state(fvmr_handle *h, int c, double *const U[4]) {
 
 int fvmr_batch_advance(fvmr_handle *h, int nsteps, double *t, const double *T) {
     if (!h || !t || !T || nsteps < 0) return set_error(FVMR_ERR_INVALID_ARG, "invalid argument");
-    if (!h->tiles) return set_error(FVMR_ERR_UNSUPPORTED, "fvmr_batch_advance needs the tile kernels");
+    if (!h->tiles && h->tile_sides) return set_error(FVMR_ERR_UNSUPPORTED, "fvmr_batch_advance needs the tile kernels");
     std::vector<Scalars> s(h->ncases);
     HIP_OK(hipMemcpyAsync(s.data(), h->sc, s.size() * sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));

@@ -294,11 +294,13 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
         double gw[3];
     };
     std::vector<Cell> rec(nc);
+    for (int c = 0; c < nc && out.joined; c++) out.joined = slot_nodes(in, c, rec[c].v, rec[c].turned);
     for (int c = 0; c < nc; c++) {
-        if (!slot_nodes(in, c, rec[c].v, rec[c].turned)) {
-            out.joined = false;
-            return FVMR_OK;
-        }
+        if (!out.joined)   // the vertices as they are
+            for (int j = 0; j < 3; j++) {
+                rec[c].v[j] = in.cnode[(size_t)j * nc + c];
+                rec[c].turned[j] = 0;
+            }
         for (int j = 0; j < 3; j++) {
             const TileSlot sl = in.cslot[(size_t)j * nc + c];
             rec[c].gw[j] = gg_weight(in, c, sl.x & ((1 << 28) - 1), sl.y, (sl.x & (1 << 28)) != 0);

@@ -44,7 +44,7 @@ struct TileCaps {
 
 struct TileMesh {
     int ntiles = 0;
-    bool joined = true;           // false: an element's edges do not join its nodes, no tiles were built
+    bool joined = true;           // false: some element's edges do not join its nodes; lnodes are its vertices then
     std::vector<int> info;        // kTileInfo per tile
     std::vector<int> halo;        // device cell id of local cells nT .. nL-1
     std::vector<double> nxy;      // node coordinates, 2 per local node

@@ -70,7 +70,9 @@ extern "C" {
  * every face flux evaluated once; it needs the standard geometry (centroids, midpoints,
  * normals recomputable from the nodes, float-valued lengths, as fvmr_mesh_* produce).
  * CELL: one gradient and one stage kernel per RK stage over packed per-cell records.
- * AUTO: TILE when the geometry allows it, else CELL.  Both give the same results. */
+ * AUTO: TILE when the geometry allows it, else CELL.  Both give the same results.  An FP64 handle of
+ * fvmr_create on a mesh in which some element's edges are not the sides of its nodes runs the cell
+ * kernels also under TILE (fvmr_tile_shape gives 0, 0). */
 #define FVMR_KERNELS_AUTO       0
 #define FVMR_KERNELS_CELL       1
 #define FVMR_KERNELS_TILE       2
