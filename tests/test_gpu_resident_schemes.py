@@ -1,0 +1,53 @@
+"""Resident runs equal single steps (the launched kernels) bit for bit in every scheme: gradient, limiter, flux,
+reconstruction, equation and precision."""
+import numpy as np
+import pytest
+
+import cfd_solver_2d_gpu_amd as F
+from helpers import wedge_case
+from test_gpu_resident import naca_case
+
+pytestmark = pytest.mark.gpu
+
+
+def wedge():
+    return wedge_case(65, 33)
+
+
+def naca():
+    m, p, U = naca_case(48, 21)
+    p.CFL = 0.4
+    return m, p, U
+
+
+def viscous():
+    m, p, U = naca()
+    p.equation = F.EQ_NS
+    p.mu0 = 1e-3 * p.inf_ruvp[0] * np.hypot(p.inf_ruvp[1], p.inf_ruvp[2])
+    return m, p, U
+
+
+@pytest.mark.parametrize("precision", [F.PREC_FP64, F.PREC_MIXED])
+@pytest.mark.parametrize("limiter", [F.LIM_NONE, F.LIM_BARTH, F.LIM_VENKATAKRISHNAN])
+@pytest.mark.parametrize("gradient", [F.GRA_GREENGAUSS, F.GRA_LEASTSQUARE])
+@pytest.mark.parametrize("case", [wedge, naca, viscous])
+def test_resident_runs_equal_single_steps(case, gradient, limiter, precision):
+    print(f"[gpu-case] resident run: {case.__name__}, gradient {gradient}, limiter {limiter}, precision {precision}", flush=True)
+    m, p, U = case()
+    a = m.arrays()["element_xy"]
+    U[0] *= 1.0 + 0.05 * np.sin(3 * a[0]) * np.cos(4 * a[1])
+    p.gradient, p.limiter, p.precision = gradient, limiter, precision
+    for p.flux_scheme in (F.SOL_LLF, F.SOL_ROE):
+        for p.reconstruct in (F.REC_CONSTANT, F.REC_LINEAR):
+            out = []
+            for runs in ((9,), (1,) * 9):
+                g = F.GPUSolver2(m, p)
+                g.set_state(U)
+                t = 0.0
+                for n in runs:
+                    t, info = g.advance(n, t, 1e9, F.NORM_INF)
+                out.append((g.get_state(), t, info.dt, np.array(info.residual[:])))
+                assert g.resident_steps() == (9 if len(runs) == 1 else 0)
+                g.close()
+            for x, y in zip(*out):
+                assert np.array_equal(x, y), (p.flux_scheme, p.reconstruct)
