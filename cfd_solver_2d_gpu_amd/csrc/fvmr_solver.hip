@@ -1212,7 +1212,7 @@ struct TileArgs {
     const int *info;          // fvmr::kTileInfo ints per tile
     const int *halo;          // device cell ids of halo cells
     const V2<double> *nxy;    // node coordinates per tile
-    const int *lnodes;        // per local cell: 3 local node ids
+    const int *lnodes;        // per local cell: 3 local node ids, and which of them the centroid adds last
     const I3 *gslot;          // per gradient cell: 3 slot words
     const V4<G> *gcoef;       // per gradient cell: Green-Gauss weights of the 3 slots, volume
     const I3 *face;           // per face: nodes | BC code, L | R | pair face, float length
@@ -1425,7 +1425,13 @@ __device__ __forceinline__ void tile_gradient(const Phys &ph, TileLds<C, G, Cfg,
     const V2<double> nd[3] = {s.N[lfield(nw, 0)], s.N[lfield(nw, 1)], s.N[lfield(nw, 2)]};
     V2<G> cen;
     if (CEN) {
-        const V2<double> ct = tile_centroid(nd[0], nd[1], nd[2]);
+        V2<double> ct = tile_centroid(nd[0], nd[1], nd[2]);
+        // the sum in the order of the element's nodes where the slots' order is another (no mesh of this library)
+        const int last = (int)((unsigned)nw >> fvmr::kLnLastShift);
+        if (__builtin_expect(__any(last), 0)) {
+            if (last == 1) ct = tile_centroid(nd[0], nd[2], nd[1]);
+            if (last == 2) ct = tile_centroid(nd[1], nd[2], nd[0]);
+        }
         cen = V2<G>{(G)ct.x, (G)ct.y};
         s.cen[i] = cen;
     } else {

@@ -290,7 +290,7 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
     std::vector<int> cells, faces, nodes;
     // what every tile that holds a cell packs of it
     struct Cell {
-        int v[3], turned[3];
+        int v[3], turned[3], last;
         double gw[3];
     };
     std::vector<Cell> rec(nc);
@@ -301,6 +301,7 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
                 rec[c].v[j] = in.cnode[(size_t)j * nc + c];
                 rec[c].turned[j] = 0;
             }
+        rec[c].last = rec[c].v[2] == in.cnode[2 * (size_t)nc + c] ? 0 : (rec[c].v[1] == in.cnode[2 * (size_t)nc + c] ? 1 : 2);
         for (int j = 0; j < 3; j++) {
             const TileSlot sl = in.cslot[(size_t)j * nc + c];
             rec[c].gw[j] = gg_weight(in, c, sl.x & ((1 << 28) - 1), sl.y, (sl.x & (1 << 28)) != 0);
@@ -392,9 +393,9 @@ int build_tiles(const TileInput &in, const TileCaps &caps, TileMesh &out) {
             const int c = cells[i];
             lcxy[2 * i] = in.cx[c];
             lcxy[2 * i + 1] = in.cy[c];
-            int w = 0;
-            for (int j = 0; j < 3; j++) w |= nid[rec[c].v[j]] << (kLocalBits * j);
-            lnodes[i] = w;
+            unsigned w = (unsigned)rec[c].last << kLnLastShift;
+            for (int j = 0; j < 3; j++) w |= (unsigned)nid[rec[c].v[j]] << (kLocalBits * j);
+            lnodes[i] = (int)w;
         }
         int *gslot = grow(out.gslot, 3 * (size_t)nG);
         double *gcoef = grow(out.gcoef, 4 * (size_t)nG);

@@ -28,6 +28,10 @@ constexpr int kGsIsR = 1 << 20;
 constexpr int kGsPeriodic = 1 << 21;
 constexpr int kGsTurned = 1 << 22;
 
+// Local nodes of a cell in lnodes (10 bits each), and in the two bits above them which one the caller's centroid
+// adds last: 0 the third, 1 the second, 2 the first.
+constexpr int kLnLastShift = 3 * kLocalBits;
+
 // Face record (3 ints): x = node a | node b << 10 | boundary code << 20 (0 interior, else
 // type - 5999); y = L | R << 10 | pair face << 20; z = float bits of the length.
 constexpr int kBcShift = 20;
