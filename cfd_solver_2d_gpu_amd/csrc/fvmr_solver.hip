@@ -3175,8 +3175,8 @@ int build_geometry(fvmr_solver *h, const fvmr_mesh_soa *m, const std::vector<int
     return FVMR_OK;
 }
 
-// The pinned slots of to_host: four of 1 MiB, or one of a smaller handle's state.  Taken with the state transfers'
-// other buffers, before the first state is set.  131,406 cells to the host: 4 x 256 KiB 323 us, 4 x 512 KiB 224 us,
+// The pinned slots of to_host: four of 1 MiB, or one of a smaller handle's state.  Taken at
+// the handle's creation: mapped later, between large host arrays, their pages took 1.7 ms.  131,406 cells to the host: 4 x 256 KiB 323 us, 4 x 512 KiB 224 us,
 // 4 x 1 MiB 176 us.
 constexpr size_t kPinSlot = size_t(1) << 20;
 bool pin_init(fvmr_solver *h) {
@@ -3348,6 +3348,7 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
     (void)hipGetDevice(&h->device);
     auto bail = [&](int code) { free_all(h); delete h; return code; };
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) return bail(set_error(FVMR_ERR_HIP, "hipStreamCreate failed"));
+    (void)pin_init(h);   // (without pinned memory copies to the host are slower)
     const int nc = h->nc, nf = h->nf;
     // physics constants
     Phys &ph = h->ph;
@@ -3687,36 +3688,38 @@ int fvmr_create_batch(int ncases, const fvmr_mesh_soa *const *meshes, const fvmr
         tn += meshes[c]->num_node; tc += meshes[c]->num_element; tf += meshes[c]->num_edge; tb += meshes[c]->num_boundary_set;
     }
     if (tn > INT32_MAX || tc > INT32_MAX || tf > INT32_MAX) return set_error(FVMR_ERR_UNSUPPORTED, "batch too large");
-    std::vector<double> nxy[2], exy[2], evol, elen, gxy[2], gnrm[2];
-    std::vector<int> en[4], ee[4], enb[4], gn[2], gset, gpair, gL, gR, btype;
+    std::vector<double> nxy[2], exy[2], evol(tc), elen(tf), gxy[2], gnrm[2];
+    std::vector<int> en[4], ee[4], enb[4], gn[2], gset(tf), gpair(tf), gL(tf), gR(tf), btype(tb);
+    for (int k = 0; k < 2; k++) { nxy[k].resize(tn); exy[k].resize(tc); gxy[k].resize(tf); gnrm[k].resize(tf); gn[k].resize(tf); }
+    for (int j = 0; j < 4; j++) { en[j].resize(tc); ee[j].resize(tc); enb[j].resize(tc); }
     std::vector<int> case_begin{0};
     int noff = 0, coff = 0, foff = 0, soff = 0;
-    auto add = [](int v, int off) { return v < 0 ? v : v + off; };
+    // whole arrays one after the other, indices offset (-1 stays)
+    auto copy = [](const auto *src, int n, auto *dst) { std::copy(src, src + n, dst); };
+    auto shift = [](const int *src, int n, int off, int *dst) {
+        for (int i = 0; i < n; i++) dst[i] = src[i] < 0 ? src[i] : src[i] + off;
+    };
     for (int c = 0; c < ncases; c++) {
         const fvmr_mesh_soa &q = *meshes[c];
-        for (int k = 0; k < 2; k++) nxy[k].insert(nxy[k].end(), q.node_xy[k], q.node_xy[k] + q.num_node);
-        for (int i = 0; i < q.num_element; i++) {
-            for (int j = 0; j < 4; j++) {
-                en[j].push_back(add(q.element_nodes[j][i], noff));
-                ee[j].push_back(add(q.element_edges[j][i], foff));
-                enb[j].push_back(add(q.element_neighbors[j][i], coff));
-            }
-            for (int k = 0; k < 2; k++) exy[k].push_back(q.element_xy[k][i]);
-            evol.push_back(q.element_volume[i]);
+        for (int k = 0; k < 2; k++) {
+            copy(q.node_xy[k], q.num_node, &nxy[k][noff]);
+            copy(q.element_xy[k], q.num_element, &exy[k][coff]);
+            copy(q.edge_xy[k], q.num_edge, &gxy[k][foff]);
+            copy(q.edge_normal[k], q.num_edge, &gnrm[k][foff]);
+            for (int e = 0; e < q.num_edge; e++) gn[k][foff + e] = q.edge_nodes[k][e] + noff;
         }
-        for (int e = 0; e < q.num_edge; e++) {
-            for (int k = 0; k < 2; k++) {
-                gn[k].push_back(q.edge_nodes[k][e] + noff);
-                gxy[k].push_back(q.edge_xy[k][e]);
-                gnrm[k].push_back(q.edge_normal[k][e]);
-            }
-            gset.push_back(add(q.edge_setID[e], soff));
-            gpair.push_back(add(q.edge_periodicPair[e], foff));
-            gL.push_back(q.edge_elementL[e] + coff);
-            gR.push_back(add(q.edge_elementR[e], coff));
-            elen.push_back(q.edge_length[e]);
+        for (int j = 0; j < 4; j++) {
+            shift(q.element_nodes[j], q.num_element, noff, &en[j][coff]);
+            shift(q.element_edges[j], q.num_element, foff, &ee[j][coff]);
+            shift(q.element_neighbors[j], q.num_element, coff, &enb[j][coff]);
         }
-        btype.insert(btype.end(), q.boundary_type, q.boundary_type + q.num_boundary_set);
+        copy(q.element_volume, q.num_element, &evol[coff]);
+        copy(q.edge_length, q.num_edge, &elen[foff]);
+        shift(q.edge_setID, q.num_edge, soff, &gset[foff]);
+        shift(q.edge_periodicPair, q.num_edge, foff, &gpair[foff]);
+        for (int e = 0; e < q.num_edge; e++) gL[foff + e] = q.edge_elementL[e] + coff;
+        shift(q.edge_elementR, q.num_edge, coff, &gR[foff]);
+        copy(q.boundary_type, q.num_boundary_set, btype.data() + soff);
         noff += q.num_node; coff += q.num_element; foff += q.num_edge; soff += q.num_boundary_set;
         case_begin.push_back(coff);
     }
@@ -3772,7 +3775,6 @@ static int ensure_io(fvmr_handle *h) {
         release();
         return set_error(FVMR_ERR_HIP, std::string("permutation upload: ") + hipGetErrorString(e));
     }
-    (void)pin_init(h);   // (without them copies to the host are slower)
     h->io_ready = true;
     return FVMR_OK;
 }

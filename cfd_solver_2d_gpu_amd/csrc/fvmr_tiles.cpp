@@ -20,22 +20,40 @@ namespace fvmr {
 
 namespace {
 
-// Hilbert index of (x, y) on an n x n grid, n = 2^order (the textbook xy -> d walk, without its branches).
-uint32_t hilbert_d(uint32_t x, uint32_t y, int order) {
-    const uint32_t all = (1u << order) - 1;
-    uint32_t d = 0;
-    for (int b = order - 1; b >= 0; b--) {
-        const uint32_t rx = (x >> b) & 1u, ry = (y >> b) & 1u;
-        d = (d << 2) | ((3u * rx) ^ ry);
-        const uint32_t flip = (0u - (rx & ~ry & 1u)) & all;   // turn the quadrant
-        x ^= flip;
-        y ^= flip;
-        const uint32_t t = (x ^ y) & (ry - 1u);               // and swap its axes
-        x ^= t;
-        y ^= t;
+// Hilbert index of (x, y) on a 2^16 x 2^16 grid: the textbook xy -> d walk, four bits of x and y at a time.  The walk
+// turns and flips the quadrants below the one it enters; both coordinates flip together, so its state is two
+// bits: axes swapped, coordinates flipped.
+class HilbertWalk {
+public:
+    HilbertWalk() {
+        for (int state = 0; state < 4; state++)
+            for (int xy = 0; xy < 256; xy++) {
+                int swap = state & 1, flip = state >> 1, d = 0;
+                for (int b = 3; b >= 0; b--) {
+                    const int x = (xy >> (4 + b)) & 1, y = (xy >> b) & 1;
+                    const int rx = (swap ? y : x) ^ flip, ry = (swap ? x : y) ^ flip;
+                    d = (d << 2) | ((3 * rx) ^ ry);
+                    if (!ry) {
+                        flip ^= rx;
+                        swap ^= 1;
+                    }
+                }
+                step_[state][xy] = (uint16_t)(d << 2 | flip << 1 | swap);
+            }
     }
-    return d;
-}
+    uint32_t index(uint32_t x, uint32_t y) const {
+        uint32_t d = 0, state = 0;
+        for (int b = 12; b >= 0; b -= 4) {
+            const uint32_t q = step_[state][((x >> b) & 15u) << 4 | ((y >> b) & 15u)];
+            d = d << 8 | q >> 2;
+            state = q & 3u;
+        }
+        return d;
+    }
+
+private:
+    uint16_t step_[4][256];
+};
 
 bool same_bits(double a, double b) { return std::memcmp(&a, &b, sizeof(double)) == 0; }
 
@@ -93,7 +111,8 @@ std::vector<int> hilbert_order(int nc, const double *cx, const double *cy) {
         x0 = std::min(x0, cx[c]); x1 = std::max(x1, cx[c]);
         y0 = std::min(y0, cy[c]); y1 = std::max(y1, cy[c]);
     }
-    const int order = 16;
+    constexpr int order = 16;   // HilbertWalk's
+    static const HilbertWalk walk;
     const double span = std::max(std::max(x1 - x0, y1 - y0), 1e-300);
     const double scale = ((1u << order) - 1) / span;
     struct Key {
@@ -104,10 +123,9 @@ std::vector<int> hilbert_order(int nc, const double *cx, const double *cy) {
     for (int c = 0; c < nc; c++) {
         const uint32_t ix = (uint32_t)std::min<double>((cx[c] - x0) * scale, (1u << order) - 1);
         const uint32_t iy = (uint32_t)std::min<double>((cy[c] - y0) * scale, (1u << order) - 1);
-        key[c] = {hilbert_d(ix, iy, order), c};
+        key[c] = {walk.index(ix, iy), c};
     }
-    // by 11 bits at a time, each pass stable (393,216 cells: 31 ms with a comparison sort of the walk's branches,
-    // 12 ms so)
+    // by 11 bits at a time, each pass stable (a comparison sort takes 2.5 times as long at 393,216 cells)
     constexpr int kBits = 11;
     for (int shift = 0; shift < 2 * order; shift += kBits) {
         size_t at[1 << kBits] = {0};
