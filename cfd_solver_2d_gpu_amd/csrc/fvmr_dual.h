@@ -1,7 +1,7 @@
 // Forward-mode dual numbers for the adjoint kernels: a value and N directional derivatives.
 // The solver's face-physics templates are instantiated with Dual<N> in place of double where few
-// directions are wanted (the freestream angle, a face's normal).  Branches (min/max, the out-of-range
-// fallback, the farfield regimes) are taken on the values, so derivatives follow the branch the value takes.
+// directions are wanted (the freestream angle, a face's normal).  Branches (the out-of-range fallback, the
+// farfield regimes) are taken on the values, so derivatives follow the branch the value takes.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -127,19 +127,6 @@ struct Dual {
         return r;
     }
     friend __device__ __forceinline__ Dual fabs(const Dual &a) { return (a.v < 0.0) ? -a : a; }
-    friend __device__ __forceinline__ bool isnan(const Dual &a) { return ::isnan(a.v); }
-    // fmin/fmax: the operand whose value is returned (the non-NaN one when one is NaN; the
-    // first on a tie) carries its derivatives
-    friend __device__ __forceinline__ Dual fmin(const Dual &a, const Dual &b) {
-        if (::isnan(a.v)) return b;
-        if (::isnan(b.v)) return a;
-        return (b.v < a.v) ? b : a;
-    }
-    friend __device__ __forceinline__ Dual fmax(const Dual &a, const Dual &b) {
-        if (::isnan(a.v)) return b;
-        if (::isnan(b.v)) return a;
-        return (b.v > a.v) ? b : a;
-    }
     // a^b = exp(b ln a): d = b a^(b-1) da + a^b ln(a) db (the ln term only where b varies)
     friend __device__ __forceinline__ Dual pow(const Dual &a, const Dual &b) {
         Dual r;

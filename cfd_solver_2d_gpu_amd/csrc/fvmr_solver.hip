@@ -198,24 +198,22 @@ template <> __device__ __forceinline__ double fsqrt<double>(double a) {
 // The smaller / larger of two values, the other one where one is a quiet NaN: the bare instructions.
 // fmin and fmax first quiet each operand that the compiler has not seen computed (signalling NaN, which
 // no arithmetic makes): 60 more instructions per cell in the limiter.
-template <class T> __device__ __forceinline__ T vmin(T a, T b) { return fmin(a, b); }
-template <class T> __device__ __forceinline__ T vmax(T a, T b) { return fmax(a, b); }
-template <> __device__ __forceinline__ double vmin<double>(double a, double b) {
+__device__ __forceinline__ double vmin(double a, double b) {
     double r;
     asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-template <> __device__ __forceinline__ double vmax<double>(double a, double b) {
+__device__ __forceinline__ double vmax(double a, double b) {
     double r;
     asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-template <> __device__ __forceinline__ float vmin<float>(float a, float b) {
+__device__ __forceinline__ float vmin(float a, float b) {
     float r;
     asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-template <> __device__ __forceinline__ float vmax<float>(float a, float b) {
+__device__ __forceinline__ float vmax(float a, float b) {
     float r;
     asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
