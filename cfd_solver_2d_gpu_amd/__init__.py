@@ -246,6 +246,14 @@ def device_division(a, b):
     return q, r
 
 
+def device_roots(a):
+    """(sqrt(a), a / 3) as the device kernels form them in FP64 (fvmr_device_roots)."""
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    r, t = np.empty_like(a), np.empty_like(a)
+    check(lib().fvmr_device_roots(a.size, _dptr(a), _dptr(r), _dptr(t)), "fvmr_device_roots")
+    return r, t
+
+
 def field_init(mesh, params, init_type=INIT_UNIFORM, args=()):
     """FieldInitializer::setInitialAndBoundaryCondition: U (4 x num_element)."""
     U = np.zeros((4, mesh.num_element))

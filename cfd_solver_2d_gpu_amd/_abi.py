@@ -115,6 +115,7 @@ SIGNATURES = {
     "fvmr_residual": (C.c_int, [C.c_void_p, C.c_int, _dp]),
     "fvmr_permutation": (C.c_int, [C.c_void_p, _ip]),
     "fvmr_device_division": (C.c_int, [C.c_int, _dp, _dp, _dp, _dp]),
+    "fvmr_device_roots": (C.c_int, [C.c_int, _dp, _dp, _dp]),
     "fvmr_node_field": (C.c_int, [C.c_void_p, _dp * 4, _dp, _dp]),
     "fvmr_use_graphs": (C.c_int, [C.c_void_p, C.c_int]),
     "fvmr_use_resident": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),

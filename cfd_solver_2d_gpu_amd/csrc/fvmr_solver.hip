@@ -2551,6 +2551,14 @@ __global__ __launch_bounds__(kBlock) void k_division(int n, const double *__rest
     q[i] = fdiv(a[i], b[i]);
     r[i] = frcp(b[i]);
 }
+// The same for the square root and the third of a sum.
+__global__ __launch_bounds__(kBlock) void k_roots(int n, const double *__restrict__ a, double *__restrict__ root,
+                                                  double *__restrict__ third_of) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    root[i] = fsqrt(a[i]);
+    third_of[i] = third(a[i]);
+}
 
 // ---------------------------------------------------------------------------
 // Host side
@@ -3916,6 +3924,24 @@ int fvmr_device_division(int n, const double *a, const double *b, double *quotie
     if (e == hipSuccess) e = hipMemcpy(reciprocal, d + 3 * (size_t)n, bytes, hipMemcpyDeviceToHost);
     (void)hipFree(d);
     if (e != hipSuccess) return set_error(FVMR_ERR_HIP, std::string("fvmr_device_division: ") + hipGetErrorString(e));
+    return FVMR_OK;
+}
+
+int fvmr_device_roots(int n, const double *a, double *root, double *third_of) {
+    if (n < 0 || (n > 0 && (!a || !root || !third_of))) return set_error(FVMR_ERR_INVALID_ARG, "invalid argument");
+    if (n == 0) return FVMR_OK;
+    const size_t bytes = (size_t)n * sizeof(double);
+    double *d = nullptr;
+    if (hipMalloc((void **)&d, 3 * bytes) != hipSuccess) return set_error(FVMR_ERR_HIP, "hipMalloc root operands");
+    hipError_t e = hipMemcpy(d, a, bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        k_roots<<<grid_of(n), kBlock>>>(n, d, d + n, d + 2 * (size_t)n);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(root, d + n, bytes, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(third_of, d + 2 * (size_t)n, bytes, hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    if (e != hipSuccess) return set_error(FVMR_ERR_HIP, std::string("fvmr_device_roots: ") + hipGetErrorString(e));
     return FVMR_OK;
 }
 

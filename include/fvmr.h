@@ -280,6 +280,10 @@ int fvmr_permutation(fvmr_handle *h, int *perm);
  * b = 0 or b = +-inf give NaN where IEEE gives +-inf or 0 (no solver quotient has such a
  * divisor on a valid state). */
 int fvmr_device_division(int n, const double *a, const double *b, double *quotient, double *reciprocal);
+/* parity hook: the FP64 square root of a[i] (hardware estimate, one Goldschmidt step, two corrections by the
+ * residual: within 1 ulp from 1e-290 on) and a[i] / 3 (rounded as IEEE division from 1e-290 on) as the
+ * device kernels form them. */
+int fvmr_device_roots(int n, const double *a, double *root, double *third_of);
 
 /* ---------------------------------------------------------------------- */
 /* batches: many independent cases advanced together (no reference         */
