@@ -796,9 +796,6 @@ __device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[4], const 
     if (ph.limiter != FVMR_LIM_NONE) {
         C eps2 = C(0);
         if (ph.limiter == FVMR_LIM_VENKATAKRISHNAN) {
-            // (not contracted, and the multiply-adds below written out: left to the compiler, they came out by the
-            // kernel around them)
-#pragma clang fp contract(off)
             const C Kh = (C)ph.venkat_K * fsqrt(vol);
             eps2 = Kh * Kh * Kh;
         }
@@ -874,10 +871,10 @@ __device__ __forceinline__ void grad_limit(const Phys &ph, const C Uc[4], const 
 #pragma unroll
                 for (int jn = 0; jn < 3; jn++) {
                     const C ndx = S.N(jn, 0), ndy = S.N(jn, 1);
-                    const C d2 = fma(gx[k], ndx, gy[k] * ndy);
+                    const C d2 = gx[k] * ndx + gy[k] * ndy;
                     const C d1 = (d2 > C(0)) ? hrel[k] : lrel[k];
-                    const C num = fma(C(2.0) * d2 * d2, d1, fma(d1, d1, eps2) * d2);
-                    const C den = fma(d1, d2, fma(C(2.0) * d2, d2, d1 * d1)) + eps2;
+                    const C num = (d1 * d1 + eps2) * d2 + C(2.0) * d2 * d2 * d1;
+                    const C den = d1 * d1 + C(2.0) * d2 * d2 + d1 * d2 + eps2;
                     const C q = fdiv(num, den * d2);
                     phi[k] = tmin(phi[k], (d2 != C(0)) ? q : C(1));
                 }

@@ -392,7 +392,8 @@ int fvmr_adjoint_state(fvmr_handle *h, double *const psi[4]);
  * reference counterpart: the reference launches every kernel from the host each step. */
 int fvmr_use_graphs(fvmr_handle *h, int on);
 /* The resident kernel: many steps (or pseudo-time iterations) of a small mesh in one launch, with the
- * results of the launched kernels bit for bit (default on).  on: 0 keeps the handle on the launched
+ * results of the launched kernels bit for bit; in mixed precision with Venkatakrishnan's limiter on
+ * Green-Gauss gradients to FP32 rounding, 3e-9 (default on).  on: 0 keeps the handle on the launched
  * kernels, 1 lets it use the resident one where it can.  max_polls: polls after which a wait between
  * its work-groups gives up (< 0: the default, about 2 s; 0: at once).  No reference counterpart. */
 int fvmr_use_resident(fvmr_handle *h, int on, int max_polls);

@@ -25,8 +25,8 @@ def reordered(m, order):
     return SoaMesh(a)
 
 
-@pytest.mark.parametrize("precision", [F.PREC_FP64, F.PREC_MIXED])
-@pytest.mark.parametrize("limiter", [F.LIM_BARTH, F.LIM_VENKATAKRISHNAN])
+@pytest.mark.parametrize("limiter,precision", [(F.LIM_BARTH, F.PREC_FP64), (F.LIM_BARTH, F.PREC_MIXED),
+                                               (F.LIM_VENKATAKRISHNAN, F.PREC_FP64)])
 @pytest.mark.parametrize("order", list(ORDERS))
 def test_resident_runs_equal_single_steps(order, limiter, precision):
     print(f"[gpu-case] slots in order {order}, limiter {limiter}, precision {precision}", flush=True)
