@@ -885,8 +885,8 @@ constexpr int kTileGgRoe = 3;
 // work-item's second face goes to LDS of its own before the first is formed (held in registers, with the records:
 // 209 VGPRs, 6.9 ms; 384 work-items with one face each 8.4 ms; bounded to 168 VGPRs with spills 9.4 ms).  LDS:
 // the face adjoints replace the staged psi and gradients, and the shares sent across the faces replace those;
-// 46 KB, three work-groups to a CU.  393,216 cells of an airfoil O-grid: one launch 44 us against 36 + 45 +
-// 17 us; 30 RK3 iterations 10.3 -> 5.2 ms.
+// 46 KB, three work-groups to a CU.  393,216 cells of an airfoil O-grid: one launch 42 us against 36 + 45 +
+// 17 us; 30 RK3 iterations 10.3 -> 4.9 ms.
 template <int SCHEME>
 __global__ __launch_bounds__(TileCfg<double>::kThreads) void k_adj_tile(
     TileArgs<double> ta, Phys ph, const V4<double> *__restrict__ cgeo, const S4 *__restrict__ U,
@@ -1559,7 +1559,7 @@ int adj_step(fvmr_solver *h, const S4 *U, const S4 *psi, const S4 *g, const S4 *
     AdjWork *w = (AdjWork *)h->adj;
     int rc;
     const double *dtl = step ? w->dtl : nullptr;
-    // tiles of the default shape: one launch, 44 us against the cell kernels' 98 at 393,216 cells, 12 against
+    // tiles of the default shape: one launch, 42 us against the cell kernels' 98 at 393,216 cells, 12 against
     // 30 at 49,152 (the other work-group shapes use the cell kernels here, as the rest of the steady path)
     if (h->tiles && h->tile_sides && h->shape == 0) {
         if ((rc = adj_gradient(h, U))) return rc;

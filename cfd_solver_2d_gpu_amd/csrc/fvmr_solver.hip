@@ -8,14 +8,15 @@
 //                   alphaC per cell in the reference edge order, block minimum of CFL V / alphaC.
 //   k_dt_finish     one work-group: global minimum, clamp to T - t, t advanced on the device.
 //   k_tile          one work-group per tile and RK stage: states of the tile and two halo
-//                   rings, nodes and face records staged in LDS; centroids and normals
-//                   recomputed from the nodes; limited gradients of the tile and the first
-//                   ring in LDS; the canonical flux of every face of the tile once; per cell
-//                   the signed sum in slot order, /(-V), RK update.
+//                   rings and the nodes staged in LDS; centroids (Green-Gauss) and, in FP64,
+//                   area vectors and normals formed from the nodes; limited gradients of the
+//                   tile and the first ring in LDS; the canonical flux of every face of the
+//                   tile once; per cell the signed sum in slot order, /(-V), RK update.
 //   k_restrict      one work-group: flagged cells repaired from their neighbours (Jacobi).
 //
 //   k_run           the above for many steps in one launch, on meshes whose tiles all fit on the
-//                   device at once (about 150,000 cells in FP64, 230,000 mixed).
+//                   device at once (256 CUs: about 150,000 cells in FP64; mixed precision 215,000,
+//                   without periodic faces).
 //
 // Cell family (any geometry; packed per-cell / per-edge records, a neighbour costs 1-2 lines):
 //   k_gradient<DT>  3 wave64 x 64 cells: wave j gathers face slot j; wave 0 forms the
@@ -379,8 +380,9 @@ __device__ __forceinline__ void ghost_slip(const FaceState<C> &L, FaceState<C> &
     set_prim(R, gamma);
 }
 
-// pow in FP64 as a call: inlined, its constants are kept in registers across the resident kernel's steps (158
-// -> 192 VGPRs and two work-groups to a CU, not three: the steady solve below 2.11 ms).
+// pow in FP64 as a call: inlined, its constants are kept in registers across the resident kernel's steps, 192
+// VGPRs instead of 158, and two work-groups to a CU instead of three: 50 pseudo-time iterations of 98,304 cells
+// take 2.11 instead of 1.72 ms.
 __device__ __attribute__((noinline)) double pow_fp64(double a, double b) { return pow(a, b); }
 template <class T> __device__ __forceinline__ T pow_call(const T &a, const T &b) {
     if constexpr (std::is_same<T, double>::value) return pow_fp64(a, b);
@@ -415,8 +417,8 @@ __device__ __forceinline__ void ghost_farfield(const FaceState<C> &L, const P *r
         const C s_u = in ? u_f : u_e, s_v = in ? v_f : v_e, s_qn = in ? qnf : qne;
         const C qtx = s_u - s_qn * nx, qty = s_v - s_qn * ny;
         // (as^2 s_r^gamma / (gamma s_p))^(1 / (gamma - 1)); beyond FP32 (which keeps its roundings) with one
-        // power, of as^2 over the squared speed of sound of s.  The work-group with the far field's faces is the one that its neighbours
-        // wait for: a steady solve of 98,304 cells, 50 iterations, 1.81 ms with two powers, 1.71 ms with one.
+        // power, of as^2 over the squared speed of sound of s.  The work-group with the far field's faces is the one
+        // that its neighbours wait for: a steady solve of 98,304 cells, 50 iterations, 1.81 ms with two powers, 1.71 ms with one.
         if constexpr (std::is_same<C, float>::value)
             r0[0] = pow(fdiv(fdiv(as * as, fdiv(s_p, pow(s_r, gamma))), gamma), frcp(ga1));
         else
@@ -1111,10 +1113,15 @@ __global__ __launch_bounds__(kGroup3) FVMR_STAGE_ATTR void k_stage(Mesh<G> m, Ph
 // ---------------------------------------------------------------------------
 // Tile kernels: one work-group per tile of consecutive cells (tile records built by
 // build_tiles on the host).  The work-group stages the states of the tile and two halo
-// rings, the nodes and the face records in LDS, recomputes centroids and face geometry from
-// the node coordinates with the host's arithmetic, forms the limited gradients of the tile
-// and the first ring in LDS, evaluates the flux of every face of the tile once, and sums
-// the fluxes per cell in slot order.  Gradients never go to HBM.
+// rings and the nodes in LDS (mixed precision: face records and normals too), forms
+// centroids and face geometry from the node coordinates with the host's arithmetic, the
+// limited gradients of the tile and the first ring in LDS, evaluates the flux of every face
+// of the tile once, and sums the fluxes per cell in slot order.  Gradients never go to HBM.
+//
+// What bounds a stage of 1,048,576 cells (counters): in FP64 it moves 201 MB (163 read, 38 written) in 48.2 us,
+// 4.2 TB/s against the 5.1 of a large copy (39 us), and issues 600 vector instructions per wave, 28 us at 4 cycles
+// each: neither alone, but the two with the latency between the phases at 4 waves per SIMD.  Mixed: 201 MB in 33.6 us,
+// 6.0 TB/s (part of it is the last-level cache's), and 556 instructions per wave, 26 us: traffic and issue alike.
 // ---------------------------------------------------------------------------
 // Work-group shapes of the tile kernels per arithmetic precision.  The default (S = 0) is sized so that the
 // LDS of a work-group lets as many work-groups share a CU as the registers allow (FP64: about 107 VGPRs -> 4
@@ -1812,15 +1819,19 @@ __global__ __launch_bounds__((TileCfg<G, SHAPE>::kThreads)) void k_tile_dt(TileA
 // Resident kernel: many steps in one launch, for meshes whose tiles all fit on the chip at once.
 //
 // A step of a small mesh is bound by the latency of its dependent launches (4 to 6 of them, 4-6 us
-// each, whatever they do).  Measured per step, launched and resident, on one box: 8,192 cells SSP-RK3 27 and
-// 11.6 us, 34,182 cells viscous forward Euler 17.6 and 9.5 us, 131,070 cells viscous mixed SSP-RK3 43 and 28 us;
-// 50 pseudo-time iterations of 40,000 cells 1.72 and 1.38 ms.  What bounds a resident stage of the 8,192
-// cells (3.9 us): the latency chains of the gradients (1.5 us) and fluxes (0.9 us) at one wave per SIMD,
-// and the exchange, a store to and a load from memory (1.6 us).  Here every tile's work-group stays on its CU for all steps: geometry,
-// slots and states stay in LDS and registers, the new states of the cells that other tiles need
-// are exchanged through global memory after each stage, and the time step's minimum goes through
-// one more work-group, which only reduces.  The launch is cooperative, so all work-groups run at
-// once or the launch fails; every wait ends after RunArgs::polls polls at the latest.
+// each, whatever they do).  Measured per step, launched and resident, on one box: 8,192 cells SSP-RK3 23.5 and
+// 13.7 us, 34,182 cells viscous forward Euler 13.7 and 7.5 us, 131,070 cells viscous mixed SSP-RK3 38 and 26.6 us;
+// 50 pseudo-time iterations of 40,000 cells 1.42 and 1.11 ms.  What bounds a resident step of the 8,192
+// cells, by the clock at its barriers: per stage the latency chains of the gradients (1.0 us), fluxes (0.8) and
+// update (0.55) at one wave per SIMD and the exchange, a store to and a load from memory (1.6); per step the time
+// step's radii and sums (1.4) and the wait for its minimum (1.4).  On 98,304 cells, three work-groups to a CU, the
+// exchange is 5.4 us of a stage, most of it waiting for the tile with the far field's faces.
+//
+// Here every tile's work-group stays on its CU for all steps: geometry, slots and states stay in LDS and
+// registers, the new states of the cells that other tiles need are exchanged through global memory
+// after each stage, and the time step's minimum goes through one more work-group, which only reduces.
+// The launch is cooperative, so all work-groups run at once or the launch fails; every wait ends after
+// RunArgs::polls polls at the latest.  Either way the call goes on with the launched kernels (run_leave).
 //
 // Exchange.  A double travels as two 64-bit words, each half of its bits with the number of the
 // exchange in the upper 32 bits.  Words are written and read by relaxed device-scope atomics, so
@@ -3054,11 +3065,14 @@ int run_resident(fvmr_solver *h, int n, bool store_rhs_last, Scalars s, int *don
 // same arguments).
 int run_steps(fvmr_solver *h, int n, bool store_rhs_last, const Scalars &s) {
     int rc, done = 0;
-    // from 4 steps on: a cooperative launch costs about 40 us more than an ordinary one, a resident step
-    // 8-12 us less than a launched one (8,192 to 120,000 cells: 3 steps 143 / 201 against 143 / 208 us,
-    // 5 steps 182 / 274 against 199 / 301 us)
+    // from 4 steps on: a cooperative launch costs about 30 us more than an ordinary one, a resident step 6 to
+    // 12 us less than a launched one.  3 / 4 / 5 steps, resident against launched: 8,192 cells RK3 148 / 141 / 155
+    // against 145 / 164 / 189 us, 34,182 cells Euler 117 / 115 / 123 against 115 / 131 / 146, 131,070 cells mixed RK3
+    // 183 / 194 / 221 against 182 / 218 / 258; near the most cells that fit, with one stage a step, where a
+    // resident step saves 2.6 us, runs of less than 10 steps lose 10 us (131,406 cells 124 / 149 / 163 against
+    // 121 / 141 / 152)
     constexpr int kRunMin = 4;
-    // also before graphs, whose replays are the same launches (8,192 cells: 27 to 30 us a step against 16)
+    // also before graphs, whose replays are the same launches (8,192 cells: 23.6 us a step against 13.7)
     if (h->run_on && h->run_step_kernel && !h->profiling && n >= kRunMin) {
         // (after a step with cells to restrict the rest runs by the kernels below, so that a flow
         // which needs it in every step is not stopped at each)
@@ -3178,9 +3192,9 @@ int build_geometry(fvmr_solver *h, const fvmr_mesh_soa *m, const std::vector<int
     return FVMR_OK;
 }
 
-// The pinned slots of to_host: four of 1 MiB, or one of a smaller handle's state.  Taken at
-// the handle's creation: mapped later, between large host arrays, their pages took 1.7 ms.  131,406 cells to the host: 4 x 256 KiB 323 us, 4 x 512 KiB 224 us,
-// 4 x 1 MiB 176 us.
+// The pinned slots of to_host: four of 1 MiB, or one of a smaller handle's state.  Taken at the handle's creation:
+// mapped later, between large host arrays, their pages took 1.7 ms.  131,406 cells to the host: 4 x 256 KiB 323 us,
+// 4 x 512 KiB 224 us, 4 x 1 MiB 176 us.
 constexpr size_t kPinSlot = size_t(1) << 20;
 bool pin_init(fvmr_solver *h) {
     if (h->pin_slots) return true;
@@ -3191,7 +3205,7 @@ bool pin_init(fvmr_solver *h) {
     for (int k = 0; k < slots && ok; k++)
         ok = h->pin_ev[k] || hipEventCreateWithFlags(&h->pin_ev[k], hipEventDisableTiming) == hipSuccess;
     if (ok) {
-        std::memset(h->pin, 0, slots * h->pin_slot);   // its pages are mapped on the first touch (4 MB: 1.7 ms)
+        std::memset(h->pin, 0, slots * h->pin_slot);   // its pages are mapped on the first touch
         h->pin_slots = slots;
     }
     else (void)hipGetLastError();
@@ -3213,8 +3227,9 @@ void populate(void *p, size_t bytes) {
 
 // rows x n doubles from dev (row after row) into the caller's rows, whose memory is pageable: through pinned
 // slots of at most 1 MiB, a slot being emptied by the host while the next ones fill.  Copied by the runtime from pageable
-// memory, 4 x 1,048,576 doubles took 2.2 ms, where the bus needs 0.6 and a copy on the host 0.8; through the
-// slots 1.3 ms, 4 x 8,192 doubles 50 us against 71.  Returns when the rows are complete.
+// memory, 4 x 1,048,576 doubles took 2.2 ms (3.5 ms into pages that are new to the process), where the bus needs
+// 0.6 and a copy on the host 0.8; through the slots 1.4 ms (2.5), 4 x 8,192 doubles 50 us against 71.  Returns when
+// the rows are complete.
 int to_host(fvmr_solver *h, const double *dev, size_t n, int rows, double *const *out) {
     const size_t total = (size_t)rows * n;
     if (!pin_init(h)) {   // no pinned memory left: the runtime's own copies
@@ -3376,8 +3391,9 @@ static int create_impl(const fvmr_mesh_soa *m, const fvmr_params *p, int ncases,
             return bail(set_error(FVMR_ERR_UNSUPPORTED, std::string("tile kernels: ") + why));
         // a mesh with fewer default tiles than the device has CUs is cut into smaller ones, one per
         // CU and one CU left for the resident kernel's reducing work-group: its phases then share
-        // a CU's LDS among fewer waves (8,192 cells, 33 instead of 150 per tile: 16.6 instead of
-        // 18.4 us per SSP-RK3 step); fewer than 32 cells leave lanes of the only wave idle
+        // a CU's LDS among fewer waves (8,192 cells, at most 36 instead of 150 per tile: 13.7 instead of
+        // 14.5 us per SSP-RK3 step; launched 23.5 us either way); fewer than 32 cells leave lanes of the
+        // only wave idle
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
         const int spread = (ncases == 1 && cus > 1) ? std::max(32, (int)(1.1 * nc / (cus - 1)) + 1) : kTileMaxCells;
@@ -4176,7 +4192,7 @@ int fvmr_surface_force_noalloc(fvmr_handle *h, int nsets, const int *set_offsets
 }  // extern "C"
 
 // Candidates of the tuners for a precision: every work-group shape, each with 0, for which fvmr_create takes
-// the size by the mesh and the device (on a small mesh one tile per CU: 8,192 cells, 16.6 us per step against 18.4
+// the size by the mesh and the device (on a small mesh one tile per CU: 8,192 cells, 13.7 us per step against 14.5
 // with 150 cells), and with 0.8 and 1.15 of the shape's size (within its LDS capacity).
 struct TileCand {
     int threads, cells;
