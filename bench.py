@@ -159,7 +159,7 @@ def traffic_from_profiles(kernel="k_tile", precision="fp64"):
     """HBM bytes per launch of the stage kernel (k_tile, or the cell family's k_stage) measured
     with rocprofv3 --pmc (FETCH_SIZE, WRITE_SIZE), scaled by the copy-kernel calibration;
     committed in profiles/ (None when absent)."""
-    path = os.path.join(ROOT, "profiles", f"{kernel}_pmc_wedge_1M_fp64.txt")
+    path = os.path.join(ROOT, "profiles", f"{kernel}_pmc_wedge_1M_{precision}.txt")
     if not os.path.exists(path):
         return None
     for line in open(path):
@@ -586,6 +586,9 @@ def main():
     traffic = traffic_from_profiles("k_stage" if cell else "k_tile", args.precision)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                # frac counts the algorithm's bytes, of which the tile kernel keeps the gradients in LDS;
+                # traffic_frac what the counters saw
+                "traffic_frac": round(traffic / (st_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
                 "kernel": ("k_stage<double,double> (one RK stage after k_gradient: fluxes, update; cell family)" if cell
                            else "k_tile<%s,false,false,1> (one RK stage: gradients, limiter, fluxes, "
                                 "update; Green-Gauss + Barth + Roe fixed at compile time)"
